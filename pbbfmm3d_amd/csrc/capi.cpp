@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -69,6 +70,29 @@ void dfree(void *p)
     if (p) (void)hipFree(p);
 }
 
+// Device buffers freed with the scope.
+struct DeviceTemps {
+    const char *what;
+    std::vector<void *> p;
+    explicit DeviceTemps(const char *w) : what(w) {}
+    ~DeviceTemps()
+    {
+        for (void *q : p) dfree(q);
+    }
+    double *take(size_t n)
+    {
+        p.push_back(dalloc<double>(n, what));
+        return (double *)p.back();
+    }
+    template <typename T>
+    T *put(const T *v, size_t n)
+    {
+        p.push_back(dalloc<T>(n, what));
+        check(hipMemcpy(p.back(), v, n * sizeof(T), hipMemcpyHostToDevice), what);
+        return (T *)p.back();
+    }
+};
+
 int current_device()
 {
     int n = 0;
@@ -116,9 +140,26 @@ struct MixedSet {
     double tail = 0;  // discarded relative Frobenius norm (larger side)
 };
 
+// One operator set in a reflection-adapted basis (symm.cpp, kernels_sym.hip):
+// VT' (nk x n3, class p's rows from 4 kb[p], padded to 4 mk[p]), U'
+// (n3 x nf, columns in the Pf row layout of the shape) and the operator
+// blocks in the order the M2L reads them.
+struct SymSet {
+    bool ok = false;
+    dev::SymShape shape{};
+    int nk = 0, nf = 0, nj = 0, mk[8] = {0}, kb[8] = {0};
+    double *VTw = nullptr, *Uw = nullptr, *Ef = nullptr;
+};
+
+static double device_rel_diff(const double *a, const double *b, int64_t n, double *part, hipStream_t st);
+
 struct pbb_ops {
     HostOps h;
     std::mutex mu;
+    // the FP64 mode's reflection-adapted sets, made by its first matvec
+    // (sym_ready: done; a set without the symmetry keeps ok = false)
+    std::vector<SymSet> sym;
+    std::atomic<bool> sym_ready{false};
     int device = -1;
     std::unique_ptr<pbb_ops> adj;  // transposed operator set, built on demand
     double *d_Tkz = nullptr, *d_Cw = nullptr, *d_VTw = nullptr, *d_Uw = nullptr, *d_E = nullptr;
@@ -354,6 +395,189 @@ struct pbb_ops {
         d_E = dupload(h.E, "E");
         device = dev;
     }
+    // Makes the reflection-adapted sets (allocates and waits for st).
+    void ensure_sym(hipStream_t st)
+    {
+        if (sym_ready.load(std::memory_order_acquire)) return;
+        std::lock_guard<std::mutex> lk(mu);
+        if (sym_ready.load(std::memory_order_relaxed)) return;
+        sym.assign(h.nsets, SymSet{});
+        try {
+            dev::upload_sym_orbits();
+            for (int s = 0; s < h.nsets; s++)
+                // bases to 5e-15 of the operators' norm; rounding in the
+                // singular vectors can leave a spurious direction there, which
+                // the check of the rebuilt operators finds
+                for (double tau : {5e-15, 1e-14, 2e-14})
+                    if (make_sym_set(s, tau, st)) break;
+        } catch (const Error &e) {
+            for (auto &q : sym) {
+                dfree(q.VTw);
+                dfree(q.Uw);
+                dfree(q.Ef);
+                q = SymSet{};
+            }
+            // no room beside what the device holds: the sets' own factors serve
+            if (e.status != PBB_ERR_OUT_OF_MEMORY) throw;
+        }
+        sym_ready.store(true, std::memory_order_release);
+    }
+
+    // Set s: bases C_f, C_s of the columns of U and V, A = C_f^T U and
+    // B = C_s^T V; the orbits' blocks from A E_d B^T, averaged over the
+    // reflections; kept when A^T K_d B gives every E_d back to rounding.
+    bool make_sym_set(int s, double tau, hipStream_t st)
+    {
+        const int n3 = h.n3, rf = h.rf, rs = h.rs;
+        const double *E = &h.E[(size_t)s * 316 * rf * rs];
+        const double *U = &h.U[(size_t)s * n3 * rf], *VT = &h.VT[(size_t)s * rs * n3];
+        std::vector<double> wf(rf, 0.0), ws(rs, 0.0), V((size_t)n3 * rs);
+        double tot = 0;
+        {
+            std::vector<std::vector<double>> pf(316), ps(316);
+            parallel_for(316, [&](int64_t d) {
+                pf[d].assign(rf, 0.0);
+                ps[d].assign(rs, 0.0);
+                for (int j = 0; j < rs; j++)
+                    for (int i = 0; i < rf; i++) {
+                        const double v = E[((size_t)d * rs + j) * rf + i];
+                        pf[d][i] += v * v;
+                        ps[d][j] += v * v;
+                    }
+            });
+            for (int d = 0; d < 316; d++) {
+                for (int i = 0; i < rf; i++) wf[i] += pf[d][i];
+                for (int j = 0; j < rs; j++) ws[j] += ps[d][j];
+            }
+            for (double v : wf) tot += v;
+        }
+        if (!(tot > 0) || !std::isfinite(tot)) return false;
+        for (double &v : wf) v = std::sqrt(v / tot);
+        for (double &v : ws) v = std::sqrt(v / tot);
+        for (int q = 0; q < n3; q++)
+            for (int b = 0; b < rs; b++) V[q + (size_t)b * n3] = VT[b + (size_t)q * rs];
+        SymSide F, S;
+        if (!sym_side(h.n, rf, U, wf.data(), tau, rf + 8, F) || !sym_side(h.n, rs, V.data(), ws.data(), tau, rs + 8, S))
+            return false;
+        const int tf = F.rt, ts = S.rt;
+        auto transposed = [](const std::vector<double> &a, int r, int c) {  // r x c column-major
+            std::vector<double> b(a.size());
+            for (int j = 0; j < c; j++)
+                for (int i = 0; i < r; i++) b[j + (size_t)i * c] = a[i + (size_t)j * r];
+            return b;
+        };
+        SymOrbits O;
+        sym_orbits(O);
+        int ndir = 0, index[7][7][7], of[316], refl[316], dir[56 * 8];
+        for (int a = -3; a < 4; a++)
+            for (int b = -3; b < 4; b++)
+                for (int c = -3; c < 4; c++) {
+                    if (std::abs(a) < 2 && std::abs(b) < 2 && std::abs(c) < 2) continue;
+                    index[a + 3][b + 3][c + 3] = ndir;
+                    refl[ndir] = (a < 0) * 4 + (b < 0) * 2 + (c < 0);
+                    for (int w = 0; w < O.n; w++)
+                        if (O.orbit[w].d[0] == std::abs(a) && O.orbit[w].d[1] == std::abs(b) &&
+                            O.orbit[w].d[2] == std::abs(c))
+                            of[ndir] = w;
+                    ndir++;
+                }
+        for (int w = 0; w < 56; w++)
+            for (int R = 0; R < 8; R++) {
+                const int *d = O.orbit[w].d;
+                dir[w * 8 + R] = index[3 + ((R & 4) ? -d[0] : d[0])][3 + ((R & 2) ? -d[1] : d[1])]
+                                      [3 + ((R & 1) ? -d[2] : d[2])];
+            }
+        std::vector<double> K((size_t)56 * tf * ts);
+        DeviceTemps tmp("symmetric operators");
+        const int tm = std::max(std::max(tf, ts), std::max(rf, rs));
+        double *X = tmp.take((size_t)316 * tm * tm), *Y = tmp.take((size_t)316 * tm * tm);
+        double *dK = tmp.take(K.size()), *part = tmp.take(2 * 1024);
+        const int *dcf = tmp.put(F.cls.data(), tf), *dcs = tmp.put(S.cls.data(), ts);
+        const int *ddir = tmp.put(dir, 56 * 8), *dof = tmp.put(of, 316), *dre = tmp.put(refl, 316);
+        const std::vector<double> At = transposed(F.A, tf, rf), Bt = transposed(S.A, ts, rs);
+        const double *dA = tmp.put(F.A.data(), F.A.size()), *dB = tmp.put(S.A.data(), S.A.size());
+        const double *dAt = tmp.put(At.data(), At.size()), *dBt = tmp.put(Bt.data(), Bt.size());
+        const double *dE = d_E + (size_t)s * 316 * rf * rs;
+        auto gemm = [&](const double *A, int M, int Kd, const double *B, int64_t ncol, double *C) {
+            dev::GemmArgs g{};
+            g.M = M; g.K = Kd; g.ldb = Kd; g.ldc = M; g.ncol = ncol; g.alpha = 1.0; g.A = A; g.B = B; g.C = C;
+            dev::launch_gemm(g, st);
+        };
+        gemm(dA, tf, rf, dE, (int64_t)316 * rs, X);           // A E_d
+        dev::launch_transpose_blocks(X, tf, rs, 316, Y, st);
+        gemm(dB, ts, rs, Y, (int64_t)316 * tf, X);            // (A E_d B^T)^T
+        dev::launch_sym_average(X, dcf, dcs, tf, ts, ddir, dK, st);
+        check(hipMemcpyAsync(K.data(), dK, K.size() * sizeof(double), hipMemcpyDeviceToHost, st), "copy blocks");
+        check(hipStreamSynchronize(st), "hipStreamSynchronize");
+        sym_complete(F, S, rf, rs, K.data(), 56);
+        check(hipMemcpyAsync(dK, K.data(), K.size() * sizeof(double), hipMemcpyHostToDevice, st), "copy blocks");
+        dev::launch_sym_expand(dK, dcf, dcs, tf, ts, dof, dre, X, st);
+        gemm(dAt, rf, tf, X, (int64_t)316 * ts, Y);           // A^T K_d
+        dev::launch_transpose_blocks(Y, rf, ts, 316, X, st);
+        gemm(dBt, rs, ts, X, (int64_t)316 * rf, Y);           // (A^T K_d B)^T
+        dev::launch_transpose_blocks(Y, rs, rf, 316, X, st);
+        // the operators themselves hold the symmetry to a few 1e-14 of their norm
+        const double err = device_rel_diff(X, dE, (int64_t)316 * rf * rs, part, st);
+        if (!(err <= 1e-13)) return false;
+
+        SymSet q;
+        q.shape = dev::sym_shape(F.cnt);
+        q.nf = 4 * q.shape.ng * q.shape.nrow;
+        int rbase[8], cbase[8];
+        for (int p = 0, r = 0, c = 0; p < 8; p++) {
+            rbase[p] = r;
+            cbase[p] = c;
+            r += F.cnt[p];
+            c += S.cnt[p];
+            q.mk[p] = (S.cnt[p] + 3) / 4;
+            q.kb[p] = q.nj;
+            q.nj += q.mk[p];
+        }
+        q.nk = 4 * q.nj;
+        std::vector<double> VTs((size_t)q.nk * n3, 0.0), Us((size_t)n3 * q.nf, 0.0);
+        parallel_for(n3, [&](int64_t x) {
+            for (int p = 0; p < 8; p++) {
+                for (int i = 0; i < S.cnt[p]; i++) {
+                    double v = 0;
+                    for (int b = 0; b < rs; b++) v += S.A[cbase[p] + i + (size_t)b * ts] * VT[b + (size_t)x * rs];
+                    VTs[4 * q.kb[p] + i + (size_t)x * q.nk] = v * h.w.Kw[x];
+                }
+                for (int i = 0; i < F.cnt[p]; i++) {
+                    double v = 0;
+                    for (int a = 0; a < rf; a++) v += F.A[rbase[p] + i + (size_t)a * tf] * U[x + (size_t)a * n3];
+                    Us[x + (size_t)dev::sym_row(q.shape, p, i) * n3] = v * h.w.Kw[x];
+                }
+            }
+        });
+        const int ng = q.shape.ng, nrow = q.shape.nrow;
+        const size_t blk = (size_t)nrow * q.nj * ng * 16;
+        // (a step copies two k steps' worth: padded past the last odd one)
+        std::vector<double> Ef((size_t)56 * blk + ng * 16, 0.0);
+        parallel_for(56, [&](int64_t b) {
+            const double *Kw = &K[(size_t)b * tf * ts];
+            double *dst = &Ef[(size_t)b * blk];
+            for (int p = 0; p < 8; p++)
+                for (int c = 0; c < S.cnt[p]; c++) {
+                    // k steps come in pairs of 8 k, two consecutive k per lane
+                    // group; an odd last one has 4
+                    const bool pair = c / 8 * 8 + 8 <= 4 * q.mk[p];
+                    const int fk = pair ? c % 8 / 2 : c % 8, j = q.kb[p] + c / 8 * 2 + (pair ? c % 2 : 0);
+                    for (int r = 0; r < 8; r++)
+                        for (int i = 0; i < F.cnt[r]; i++) {
+                            const int row = dev::sym_row(q.shape, r, i), part_ = row / (4 * ng), g = row / 4 % ng;
+                            dst[(((size_t)part_ * q.nj + j) * ng + g) * 16 + row % 4 + 4 * fk] =
+                                Kw[rbase[r] + i + (size_t)(cbase[p] + c) * tf];
+                        }
+                }
+        });
+        q.ok = true;
+        sym[s] = q;  // (so that a failed upload is freed)
+        sym[s].VTw = dupload(VTs, "symmetric VT");
+        sym[s].Uw = dupload(Us, "symmetric U");
+        sym[s].Ef = dupload(Ef, "symmetric E");
+        return true;
+    }
+
     // The operators of the transposed FMM (P2M <-> L2P, M2M <-> L2L): U' = VT^T,
     // VT' = U^T, E'_d = E_{-d}^T with -d at index 315 - d (Ktable order is
     // symmetric under negation).  Same weights, kernel and level scales.
@@ -401,6 +625,11 @@ struct pbb_ops {
             dfree(d_Tkz); dfree(d_Cw); dfree(d_VTw); dfree(d_Uw); dfree(d_E);
             dfree(dm_E); dfree(dm_VTw); dfree(dm_Uw); dfree(dm_px);
             for (auto &x : split) dfree(x.d);
+            for (auto &x : sym) {
+                dfree(x.VTw);
+                dfree(x.Uw);
+                dfree(x.Ef);
+            }
             dfree(vt3.d); dfree(u3.d);
             if (prev >= 0) (void)hipSetDevice(prev);
         }
@@ -417,6 +646,11 @@ struct Workspace {
     double *up = nullptr;                  // partial expansions of split boxes
     double *S = nullptr;                   // expansions S / F, [box][col][n3]
     double *P = nullptr, *Pf = nullptr;    // FP64 mode
+    int ldp = 0, ldf = 0;                  // its rows per (box, column), at most
+    bool sym = false;                      // laid out for the reflection-adapted sets
+    double *part = nullptr;                // sum parts of small M2L launches
+    int64_t part_cap = 0;                  // bytes they may take (all columns of the call)
+    int all = 0;                           // columns of the whole call
     float *P32 = nullptr, *Pf32 = nullptr; // mixed modes
     unsigned *xmax = nullptr;              // per-level max |P| (FP16 scaling)
     int kpad = 0;
@@ -424,7 +658,17 @@ struct Workspace {
 };
 
 struct pbb_plan;
-static size_t layout_workspace(const pbb_plan &p, int ncols, bool mixed, char *base, Workspace &W);
+// Rows per (box, column) of P and Pf in the FP64 mode, and the doubles of
+// the M2L's sum parts.
+struct FarDims {
+    int ldp = 0, ldf = 0;
+    size_t part = 0;
+    int64_t part_cap = 0;  // bytes the sum parts may take
+    int all = 0;           // columns of the whole call
+    bool sym = false;
+};
+constexpr int64_t SYM_PART_BYTES = 32ll << 20;
+static size_t layout_workspace(const pbb_plan &p, int ncols, bool mixed, const FarDims &d, char *base, Workspace &W);
 
 struct DevLevel {
     int64_t nb = 0, off = 0;
@@ -506,9 +750,9 @@ struct pbb_plan {
 
     // The plan's own matvec buffers, grown (never shrunk) to fit ncols
     // columns in the precision class; one block, laid out by layout_workspace.
-    void ensure_workspace(int ncols, bool mixed)
+    void ensure_workspace(int ncols, bool mixed, const FarDims &d)
     {
-        const size_t need = layout_workspace(*this, ncols, mixed, nullptr, W);
+        const size_t need = layout_workspace(*this, ncols, mixed, d, nullptr, W);
         if (need > ws_bytes) {
             dfree(ws_block);
             ws_block = nullptr;
@@ -516,14 +760,104 @@ struct pbb_plan {
             ws_block = dalloc<char>(need, "matvec workspace");
             ws_bytes = need;
         }
-        layout_workspace(*this, ncols, mixed, ws_block, W);
+        layout_workspace(*this, ncols, mixed, d, ws_block, W);
     }
 };
+
+// ---- the FP64 M2L in the reflection-adapted bases ---------------------------
+// The set of level l's M2L, or nullptr where the level keeps the set's own
+// factors (no bases of pure parity within the bounds of make_sym_set).  Where
+// they exist they were faster down to the smallest plan measured (1M points,
+// 8 columns 293 -> 78 ms; 5k points, 1 column 1.77 -> 0.42 ms per matvec).
+static const SymSet *sym_level(const pbb_plan &p, const pbb_ops *o, int l)
+{
+    if (!o->sym_ready.load(std::memory_order_acquire) || o->fp64_reduced) return nullptr;
+    const SymSet &q = o->sym[o->h.ops_set(l)];
+    return q.ok ? &q : nullptr;
+}
+
+// Tile and sum parts of a level's M2L for ncols of the call's `all` columns.
+// The sum parts decide the order of the sums, so they follow from the whole
+// call: a call that runs in column chunks gives the same bits.
+struct SymTile {
+    int cpt = 0, TB = 0, nchunks = 0, npz = 1, noz = 1;
+    int tiles = 0, class_tiles[8] = {0};
+};
+static SymTile sym_tile(const pbb_plan &p, const SymSet &q, int l, int ncols, int all, int64_t part_cap)
+{
+    if (ncols != all) {
+        const SymTile whole = sym_tile(p, q, l, all, all, part_cap);
+        SymTile t = sym_tile(p, q, l, ncols, ncols, 0);
+        t.npz = whole.npz;
+        t.noz = whole.noz;
+        return t;
+    }
+    const DevLevel &D = p.lv[l];
+    SymTile best;
+    int64_t best_cost = -1;
+    // the column chunk that leaves fewest of the tiles' columns idle
+    const int W = dev::sym_width(q.shape);
+    for (int nch = (ncols + W - 1) / W, k = 0; k < 3 && nch + k <= ncols; k++) {
+        SymTile t;
+        t.cpt = (ncols + nch + k - 1) / (nch + k);
+        t.nchunks = (ncols + t.cpt - 1) / t.cpt;
+        t.TB = std::max(1, std::min(dev::SYM_TB, W / t.cpt));
+        for (int c = 0; c < 8; c++) {
+            t.class_tiles[c] = (int)((D.class_count[c] + t.TB - 1) / t.TB);
+            t.tiles += t.class_tiles[c];
+        }
+        const int64_t cost = (int64_t)t.tiles * t.nchunks;
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = t;
+        }
+    }
+    // sum parts until the launch fills the GPU, within part_cap bytes of partial sums
+    const int64_t wgs = (int64_t)best.tiles * best.nchunks * q.shape.nrow;
+    const int64_t bytes = D.nb * ncols * (int64_t)q.nf * 8;
+    while (wgs * best.npz * best.noz < 768 && best.npz * best.noz < 64 &&
+           2 * best.npz * best.noz * bytes <= part_cap) {
+        if (best.npz < 8) best.npz *= 2;
+        else best.noz *= 2;
+    }
+    return best;
+}
+
+static FarDims far_dims(const pbb_plan &p, const pbb_ops *o, int ncols, int all, bool sym,
+                        int64_t part_cap = SYM_PART_BYTES)
+{
+    FarDims d;
+    d.part_cap = part_cap;
+    d.all = all;
+    const int rmax = std::max(o->h.rf, o->h.rs);
+    d.ldp = d.ldf = rmax;
+    for (int l = 2; sym && l <= p.Lv; l++) {
+        const SymSet *q = sym_level(p, o, l);
+        if (!q) continue;
+        d.sym = true;
+        d.ldp = std::max(d.ldp, q->nk);
+        d.ldf = std::max(d.ldf, q->nf);
+        const SymTile t = sym_tile(p, *q, l, ncols, all, part_cap);
+        if (t.npz * t.noz > 1) d.part = std::max(d.part, (size_t)t.npz * t.noz * p.lv[l].nb * ncols * q->nf);
+    }
+    return d;
+}
+static FarDims merge(const FarDims &a, const FarDims &b)
+{
+    FarDims d;
+    d.ldp = std::max(a.ldp, b.ldp);
+    d.ldf = std::max(a.ldf, b.ldf);
+    d.part = std::max(a.part, b.part);
+    d.part_cap = a.part_cap;
+    d.all = a.all;
+    d.sym = a.sym || b.sym;
+    return d;
+}
 
 // Lays out the buffers of one matvec of p with ncols columns from base
 // (nullptr: sizes only, pointers left null) and returns the bytes used; every
 // buffer starts on a 256-byte boundary.
-static size_t layout_workspace(const pbb_plan &p, int ncols, bool mixed, char *base, Workspace &W)
+static size_t layout_workspace(const pbb_plan &p, int ncols, bool mixed, const FarDims &d, char *base, Workspace &W)
 {
     const HostOps &h = p.ops->h;
     size_t off = 0;
@@ -548,8 +882,15 @@ static size_t layout_workspace(const pbb_plan &p, int ncols, bool mixed, char *b
             W.Pf32 = (float *)take(Bc * rmax * sizeof(float));
             W.xmax = (unsigned *)take((size_t)(p.Lv + 1) * sizeof(unsigned));
         } else {
-            W.P = (double *)take(Bc * rmax * sizeof(double));
-            W.Pf = (double *)take(Bc * rmax * sizeof(double));
+            W.ldp = d.ldp;
+            W.ldf = d.ldf;
+            W.sym = d.sym;
+            // (with the reflection-adapted sets each level's region starts with a box of zeros)
+            W.P = (double *)take((Bc + (d.sym ? (size_t)(p.Lv - 1) * ncols : 0)) * d.ldp * sizeof(double));
+            W.Pf = (double *)take(Bc * d.ldf * sizeof(double));
+            W.part_cap = d.part_cap;
+            W.all = d.all;
+            if (d.part) W.part = (double *)take(d.part * sizeof(double));
         }
     }
     if (p.n_up_slots > 0) W.up = (double *)take((size_t)p.n_up_slots * ncols * h.n3 * sizeof(double));
@@ -1465,9 +1806,21 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
     const bool mixed = prec != PBB_PREC_FP64;
     const PointIo io = point_io(p, o);
     int chunk = ncols;
+    bool sym = false;
+    if (!mixed && p->Lv >= 2 && !o->fp64_reduced) {
+        sym = o->sym_ready.load(std::memory_order_acquire);
+        if (!sym) {  // nothing is prepared inside a caller's stream capture
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            check(hipStreamIsCapturing(st, &cs), "hipStreamIsCapturing");
+            if (cs == hipStreamCaptureStatusNone) {
+                o->ensure_sym(st);
+                sym = true;
+            }
+        }
+    }
     if (out) {
         Workspace tmp;
-        size_t need = layout_workspace(*p, chunk, mixed, nullptr, tmp);
+        size_t need = layout_workspace(*p, chunk, mixed, far_dims(*p, o, chunk, ncols, sym), nullptr, tmp);
         if (need > p->ws_bytes || (p->ws_limit && need > p->ws_limit)) {
             size_t free_b = 0, total_b = 0;
             check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
@@ -1479,13 +1832,13 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
             if (p->ws_limit) room = std::min(room, p->ws_limit);
             while (chunk > 1 && need > room) {
                 chunk = (chunk + 1) / 2;
-                need = layout_workspace(*p, chunk, mixed, nullptr, tmp);
+                need = layout_workspace(*p, chunk, mixed, far_dims(*p, o, chunk, ncols, sym), nullptr, tmp);
             }
         }
     }
     for (int c0 = 0; c0 < ncols; c0 += chunk) {
         const int cn = std::min(chunk, ncols - c0);
-        p->ensure_workspace(cn, mixed);
+        p->ensure_workspace(cn, mixed, far_dims(*p, o, cn, ncols, sym));
         matvec_run(p, o, p->W, w + (size_t)c0 * io.in_n, cn, out ? out + (size_t)c0 * io.out_n : nullptr, st, prec,
                    true);
     }
@@ -1728,6 +2081,7 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
     const bool split_acc = split_acc_on(p, prec);
     const pbb_plan::M2LTile &tmx = p->m2l_tile[1];
     const int ldP = mixed ? W.kpad : h.rs;
+    auto sym_of = [&](int l) -> const SymSet * { return !mixed && W.sym ? sym_level(*p, o, l) : nullptr; };
     if (mixed && h.rs > W.kpad) fail(PBB_ERR_INTERNAL, "proxy padding too small");
     mark(0);
     // orders 4..8 run the direct passes: P2M at every level instead of
@@ -1837,6 +2191,19 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
         ldp = k16(l) ? 16 : dev::PX_K;
         return W.P32 + (size_t)p->lv[l].off * ncols * (ldP - ldp);
     };
+    // FP64: level l's region of P, led by a box of zeros where the level's M2L
+    // runs the reflection-adapted set
+    auto P64 = [&](int l) { return W.P + (size_t)(p->lv[l].off + (W.sym ? l - 2 : 0)) * ncols * W.ldp; };
+    if (!mixed && W.sym) {
+        dev::ZeroBoxes zb{};
+        int nz = 0;
+        for (int l = 2; l <= Lv; l++)
+            if (const SymSet *q = sym_of(l)) {
+                zb.p[nz] = P64(l);
+                zb.n[nz++] = ncols * q->nk;
+            }
+        dev::launch_zero_boxes(zb, nz, st);
+    }
     for (int l = 2; l <= Lv; l++) {
         const DevLevel &D = p->lv[l];
         const int sl = h.ops_set(l);
@@ -1854,7 +2221,13 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
             g.c_f32 = 1;
             g.C = W.P32 + (size_t)D.off * ncols * ldP;
         } else {
-            g.C = W.P + (size_t)D.off * ncols * h.rs;
+            g.C = P64(l);
+        }
+        if (const SymSet *q = sym_of(l)) {
+            g.M = g.ldc = q->nk;
+            g.A = q->VTw;
+            g.C = P64(l) + (size_t)ncols * q->nk;
+            g.pairs = ncols;
         }
         if (l >= Lp) {  // proxies straight from the points (rows past ks are zero)
             dev::ProxyArgs x{};
@@ -1957,6 +2330,33 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
     for (int l = 2; l <= Lv && !mixed; l++) {
         lev_mark(l);
         const DevLevel &D = p->lv[l];
+        if (const SymSet *q = sym_of(l)) {
+            const SymTile t = sym_tile(*p, *q, l, ncols, W.all, W.part_cap);
+            const int parts = t.npz * t.noz;
+            dev::SymArgs a{};
+            a.ncols = ncols; a.TB = t.TB; a.cpt = t.cpt; a.side = 1 << l;
+            a.ldp = q->nk; a.ldf = q->nf; a.nrow = q->shape.nrow; a.npz = t.npz; a.noz = t.noz; a.nj = q->nj;
+            std::copy(std::begin(q->mk), std::end(q->mk), a.mk);
+            std::copy(std::begin(q->kb), std::end(q->kb), a.kb);
+            a.out_off = D.off;
+            std::copy(std::begin(t.class_tiles), std::end(t.class_tiles), a.class_tiles);
+            for (int c = 0; c < 8; c++) a.class_start[c + 1] = a.class_start[c] + D.class_count[c];
+            a.order = D.order; a.coord = D.coord; a.map = D.map; a.Ef = q->Ef;
+            a.P = P64(l);
+            // (a level's rows lie at the start of its region of Pf)
+            double *pf = W.Pf + (size_t)D.off * ncols * (W.ldf - q->nf);
+            a.out = pf;
+            if (parts > 1) {
+                a.out = W.part;
+                a.out_off = 0;
+                a.part_stride = D.nb * ncols * (int64_t)q->nf;
+            }
+            dev::launch_m2l_sym(a, q->shape, t.nchunks, st);
+            if (parts > 1)
+                dev::launch_m2l_sym_reduce(W.part, parts, a.part_stride, a.part_stride,
+                                           pf + (size_t)D.off * ncols * q->nf, st);
+            continue;
+        }
         const pbb_plan::M2LTile &t64 = p->m2l_level[0][l].width ? p->m2l_level[0][l] : p->m2l_tile[0];
         const int cpt = t64.width ? std::min(ncols, t64.cpt) : std::min(ncols, 64);
         const int width = t64.width ? t64.width : ncols >= 32 || ncols <= 16 ? 128 : 64;
@@ -1979,7 +2379,8 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
             a.rs = mset(l).ks;
             a.E = o->dm_E + mset(l).e_off;
         }
-        a.P = W.P; a.Pf = W.Pf;
+        a.P = P64(l) - (size_t)D.off * ncols * h.rs;
+        a.Pf = W.Pf + (size_t)D.off * ncols * (W.ldf - h.rf);
         dev::launch_m2l(a, a.tile_prefix[8], nchunks, st);
     }
     if (Lv >= 2) lev_mark(Lv + 1);
@@ -2001,7 +2402,11 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
             g.b_f32 = 1;
             g.B = W.Pf32 + (size_t)D.off * ncols * h.rf;
         } else {
-            g.B = W.Pf + (size_t)D.off * ncols * h.rf;
+            g.B = W.Pf + (size_t)D.off * ncols * W.ldf;
+        }
+        if (const SymSet *q = sym_of(l)) {
+            g.K = g.ldb = q->nf;
+            g.A = q->Uw;
         }
         g.c_f32 = s32 ? 1 : 0;
         g.C = s32 ? (void *)((float *)W.S + (size_t)D.off * ncols * n3) : (void *)(W.S + (size_t)D.off * ncols * n3);
@@ -2138,14 +2543,21 @@ PBB_API pbb_status pbb_plan_matvec_noalloc(pbb_plan *plan, const double *w_dev, 
             fail(PBB_ERR_INVALID_ARG, "unknown precision mode");
         const bool mixed = precision != PBB_PREC_FP64;
         Workspace W;
-        const size_t need = layout_workspace(*plan, ncols, mixed, nullptr, W);
+        // the reflection-adapted sets where an earlier matvec made them and the
+        // workspace with them fits, else the sets' own factors
+        FarDims fd = far_dims(*plan, plan->ops, ncols, ncols, !mixed);
+        size_t need = layout_workspace(*plan, ncols, mixed, fd, nullptr, W);
+        for (int k = 0; k < 2 && need > (size_t)PBB_NOALLOC_SCRATCH_BYTES && fd.sym; k++) {
+            fd = far_dims(*plan, plan->ops, ncols, ncols, k == 0, 0);  // without sum parts, then without the sets
+            need = layout_workspace(*plan, ncols, mixed, fd, nullptr, W);
+        }
         if (need > (size_t)PBB_NOALLOC_SCRATCH_BYTES)
             fail(PBB_ERR_INVALID_ARG, "this matvec needs " + std::to_string(need) +
                                           " bytes of workspace; the allocation-free matvec has " +
                                           std::to_string((size_t)PBB_NOALLOC_SCRATCH_BYTES));
         DeviceGuard g(plan->device);
         char *base = scratch_ptr(plan->device);
-        layout_workspace(*plan, ncols, mixed, base, W);
+        layout_workspace(*plan, ncols, mixed, fd, base, W);
         // build = false: the split operators of a mixed mode must exist already
         matvec_run(plan, plan->ops, W, w_dev, ncols, out_dev, (hipStream_t)stream, precision, false);
     });
@@ -2290,6 +2702,7 @@ static void batch_create(const pbb_batch_entry *E, int nplans, int ncols, int pr
     // the transposed operator sets of a plan fit one workspace layout.
     std::vector<pbb_ops *> ops(nplans);
     std::vector<Workspace> wsp(nplans);
+    std::vector<FarDims> dims(nplans);  // of a plan's first entry: what all its entries need
     for (int i = 0; i < nplans; i++) {
         pbb_plan *p = plans[i];
         ops[i] = (E[i].flags & PBB_BATCH_TRANSPOSE) ? p->ops->adjoint() : p->ops;
@@ -2297,6 +2710,16 @@ static void batch_create(const pbb_batch_entry *E, int nplans, int ncols, int pr
         const SplitE *se = nullptr;
         const pbb_ops::SplitA *sa = nullptr;
         split_ops(p, ops[i], precision, true, b->stream, se, sa);
+        if (!mixed && p->Lv >= 2 && !ops[i]->fp64_reduced) ops[i]->ensure_sym(b->stream);
+        dims[i] = far_dims(*p, ops[i], ncols, ncols, !mixed);
+        for (int k = 0; k < i; k++)
+            if (plans[k] == p) {
+                dims[k] = merge(dims[k], dims[i]);
+                break;
+            }
+    }
+    for (int i = 0; i < nplans; i++) {
+        pbb_plan *p = plans[i];
         int first = i;
         for (int k = 0; k < i; k++)
             if (plans[k] == p) {
@@ -2308,9 +2731,9 @@ static void batch_create(const pbb_batch_entry *E, int nplans, int ncols, int pr
             continue;
         }
         Workspace tmp;
-        const size_t need = layout_workspace(*p, ncols, mixed, nullptr, tmp);
+        const size_t need = layout_workspace(*p, ncols, mixed, dims[i], nullptr, tmp);
         b->blocks.push_back(dalloc<char>(need, "batch workspace"));
-        layout_workspace(*p, ncols, mixed, b->blocks.back(), wsp[i]);
+        layout_workspace(*p, ncols, mixed, dims[i], b->blocks.back(), wsp[i]);
     }
     check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
     // independent entries run as concurrent graph branches.  Entries

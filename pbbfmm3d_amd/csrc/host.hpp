@@ -104,6 +104,37 @@ struct ReducedSet {
 };
 void reduce_set(const HostOps &ops, int set, const double *VTw, const double *Uw, double tau, ReducedSet &out);
 
+// ---- reflection symmetry of an operator set (symm.cpp) ----------------------
+// One side's basis of pure parity: rt columns ordered by class (bits x 4, y 2,
+// z 1; set = odd), cnt of each class, A = C^T U (rt x r, column-major).
+struct SymSide {
+    int rt = 0;
+    int cnt[8] = {0};
+    std::vector<int> cls;   // class of every column
+    std::vector<double> A;
+};
+// Finds the basis of the columns of U (n3 x r), each weighted with w, to
+// within tau of the weighted Frobenius norm; false when more than max_rt
+// columns would be needed.
+bool sym_side(int n, int r, const double *U, const double *w, double tau, int max_rt, SymSide &out);
+// M: nblocks operators (rt_f x rt_s, column-major) averaged over the
+// reflections; undoes the projection on the columns that a cluster cut by
+// the rank added to the bases.
+void sym_complete(const SymSide &f, const SymSide &s, int rf, int rs, double *M, int nblocks);
+
+// Orbits of the 316 far directions under the axis reflections.  pm, zm: the
+// axes whose component is 1 or 2 (both signs occur), and 0; slot: the first
+// of the orbit's directions among the 189 of a class.
+struct SymOrbit {
+    int d[3], pm, zm, slot;
+};
+struct SymOrbits {
+    int n, nslots;
+    SymOrbit orbit[56];
+    int slot_orbit[189], slot_sign[189];  // sign bits within pm
+};
+void sym_orbits(SymOrbits &o);
+
 // Kernel blocks of one operator set (H2_3D_Tree.cpp:277-374):
 // Kcell[d*n6 + i + j*n3] = K(t_i, s_j^(d)) / (Kw_i Kw_j).
 void kernel_blocks(const HostOps &ops, const HostEval &eval, double boxLen,

@@ -337,65 +337,12 @@ __global__ __launch_bounds__(256) void l2l_fp64(M2MArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// C[:, j] = alpha * A B[:, j] for j < ncol: A (M x K, lda M, FP64), B
-// (K x ncol, ldb >= K), C (ldc >= M rows per column; rows M..ldc-1 are
-// written as zeros), column-major.  64 x 64 output tiles, K in chunks of 16
-// through LDS, 4 x 4 outputs per thread, FP64 arithmetic; B and C may be
-// FP32.  Serves the proxy projection P = VTw S (compute.hpp:376-395) and
-// the local expansion F = scale Uw Pf (compute.hpp:497-508).
-template <typename TB, typename TC>
-__global__ __launch_bounds__(256) void gemm_small_a(GemmArgs g)
-{
-    __shared__ double As[16][64 + 1];
-    __shared__ double Bs[16][64 + 1];
-    const TB *B = (const TB *)g.B;
-    TC *C = (TC *)g.C;
-    const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
-    const int64_t n0 = (int64_t)blockIdx.x * 64;
-    const int m0 = blockIdx.y * 64;
-    double acc[4][4] = {};
-    for (int k0 = 0; k0 < g.K; k0 += 16) {
-        for (int q = tid; q < 16 * 64; q += 256) {
-            int row = q % 64, k = q / 64;
-            int gr = m0 + row, gk = k0 + k;
-            As[k][row] = (gr < g.M && gk < g.K) ? g.A[gr + (int64_t)gk * g.M] : 0.0;
-        }
-        for (int q = tid; q < 16 * 64; q += 256) {
-            int k = q % 16, col = q / 16;
-            int gk = k0 + k;
-            int64_t gc = n0 + col;
-            Bs[k][col] = (gk < g.K && gc < g.ncol) ? (double)B[gk + gc * g.ldb] : 0.0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < 16; k++) {
-            double av[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) av[i] = As[k][tx + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; j++) bv[j] = Bs[k][ty + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] += av[i] * bv[j];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        int64_t gc = n0 + ty + 16 * j;
-        if (gc >= g.ncol) continue;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            int gr = m0 + tx + 16 * i;
-            if (gr < g.M) C[gr + gc * g.ldc] = (TC)(g.alpha * acc[i][j]);
-            else if (gr < g.ldc) C[gr + gc * g.ldc] = (TC)0;
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// The same GEMM on the FP64 matrix cores: a workgroup of 4 waves computes all
+// C[:, j] = alpha * A B[:, j] for j < ncol: A (M x K, stride lda, FP64), B
+// (K x ncol, ldb >= K), C (ldc >= M; rows M..zrows-1 are written as zeros),
+// column-major; B and C may be FP32.  Serves the proxy projection P = VTw S
+// (compute.hpp:376-395) and the local expansion F = scale Uw Pf
+// (compute.hpp:497-508).
+// On the FP64 matrix cores: a workgroup of 4 waves computes all
 // RB 16-row blocks of M x 64 columns (one 16-column block per wave), K in
 // chunks of 16.  A (small, shared by every workgroup) goes through a
 // double-buffered LDS tile; each lane loads its own B fragment straight from
@@ -424,7 +371,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         for (int r = 0; r < AR; r++) {
             const int q = tid + r * NT, row = q % R, gk = k0 + q / R;
             const bool ok = q < KC * R && row < g.M && gk < g.K;
-            const double v = g.A[ok ? row + (int64_t)gk * g.M : 0];
+            const double v = g.A[ok ? row + (int64_t)gk * g.lda : 0];
             ra[r] = ok ? v : 0.0;
         }
     };
@@ -470,16 +417,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
         run_step(step, bA, bB);
         if (step + 1 < nsteps) run_step(step + 1, bB, bA);
     }
-    if (gc < g.ncol) {
+    if (gc < g.ncol && g.pairs > 0) {
+        const int64_t box = gc / g.pairs;
+        TC *c = C + box * g.pairs * g.ldc + 2 * (gc - box * g.pairs);
+#pragma unroll
+        for (int rb_ = 0; rb_ < RB; rb_++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int row = rb_ * 16 + fk + 4 * v;
+                if (row < g.M) c[(int64_t)((row + g.row0) / 2) * 2 * g.pairs + (row & 1)] = (TC)(g.alpha * acc[rb_][v]);
+            }
+    } else if (gc < g.ncol) {
 #pragma unroll
         for (int rb_ = 0; rb_ < RB; rb_++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = rb_ * 16 + fk + 4 * v;
                 if (row < g.M) C[row + gc * g.ldc] = (TC)(g.alpha * acc[rb_][v]);
-                else if (row < g.ldc) C[row + gc * g.ldc] = (TC)0;
+                else if (row < g.zrows) C[row + gc * g.ldc] = (TC)0;
             }
-        for (int row = R; row < g.ldc; row++)  // padding rows beyond the MFMA tile
+        for (int row = R; row < g.zrows; row++)  // padding rows beyond the MFMA tile
             if (fk == 0) C[row + gc * g.ldc] = (TC)0;
     }
 }
@@ -1718,13 +1675,26 @@ void launch_l2l(const M2MArgs &a, int nparent, hipStream_t st)
     check(hipGetLastError(), "l2l_fp64");
 }
 
-void launch_gemm(const GemmArgs &g, hipStream_t st)
+void launch_gemm(const GemmArgs &args, hipStream_t st)
 {
+    GemmArgs g = args;
     if (g.ncol <= 0) return;
     if (g.ldb < g.K || g.ldc < g.M) fail(PBB_ERR_INTERNAL, "gemm: leading dimension too small");
-    const int rb = (g.M + 15) / 16;
-    if (rb <= 16) {
-        dim3 grid((unsigned)((g.ncol + 63) / 64));
+    if (g.lda == 0) g.lda = g.M;
+    if (g.zrows == 0) g.zrows = g.ldc;
+    // at most 16 row blocks (256 rows) per launch: larger products run as row
+    // ranges of about equal size
+    const int rball = (g.M + 15) / 16, nparts = (rball + 15) / 16, rb = (rball + nparts - 1) / nparts;
+    dim3 grid((unsigned)((g.ncol + 63) / 64));
+    const int M = g.M, zrows = g.zrows;
+    for (int part = 0; part < nparts; part++) {
+        const int r0 = part * rb * 16;
+        g.M = std::min(M - r0, rb * 16);
+        g.zrows = part + 1 < nparts ? g.M : zrows - r0;
+        g.A = args.A + r0;
+        g.row0 = g.pairs > 0 ? r0 : 0;
+        const int c0 = g.pairs > 0 ? 0 : r0;
+        g.C = g.c_f32 ? (void *)((float *)args.C + c0) : (void *)((double *)args.C + c0);
 #define PBB_G(R)                                                                                   \
     case R:                                                                                        \
         if (!g.b_f32 && !g.c_f32) gemm_mfma_f64<double, double, R><<<grid, 256, 0, st>>>(g);       \
@@ -1738,14 +1708,7 @@ void launch_gemm(const GemmArgs &g, hipStream_t st)
         }
 #undef PBB_G
         check(hipGetLastError(), "gemm_mfma_f64");
-        return;
     }
-    dim3 grid((unsigned)((g.ncol + 63) / 64), (unsigned)((std::max(g.M, g.ldc) + 63) / 64));
-    if (!g.b_f32 && !g.c_f32) gemm_small_a<double, double><<<grid, 256, 0, st>>>(g);
-    else if (!g.b_f32 && g.c_f32) gemm_small_a<double, float><<<grid, 256, 0, st>>>(g);
-    else if (g.b_f32 && !g.c_f32) gemm_small_a<float, double><<<grid, 256, 0, st>>>(g);
-    else gemm_small_a<float, float><<<grid, 256, 0, st>>>(g);
-    check(hipGetLastError(), "gemm_small_a");
 }
 
 void launch_m2l(const M2LArgs &a, int ntiles, int ncolchunks, hipStream_t st)

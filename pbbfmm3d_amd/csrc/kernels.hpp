@@ -126,6 +126,9 @@ struct ProxyArgs {
 
 struct GemmArgs {
     int M, K, ldb, ldc;
+    int lda = 0, zrows = 0;    // A's stride (0: M); rows M..zrows-1 of C are zeroed (0: to ldc)
+    // > 0: C's columns come in boxes of `pairs`, stored [box][row / 2][column][2] (FP64, ldc = M even)
+    int pairs = 0, row0 = 0;   // (row0: the launcher's, the first row of a row range)
     int b_f32, c_f32;          // B / C element type: 0 FP64, 1 FP32
     int64_t ncol;
     double alpha;
@@ -144,6 +147,51 @@ struct M2LArgs {
     const double *E, *P;
     double *Pf;
 };
+
+// The FP64 M2L in a reflection-adapted basis (kernels_sym.hip).
+constexpr int SYM_TB = 64;    // boxes of a tile
+constexpr int SYM_CONFS = 9;  // row configurations
+constexpr int SYM_NG2 = 32;   // row groups up to which a wave holds 32 columns (else 16)
+constexpr int SYM_NB = 2;     // orbits to a barrier
+
+// Row layout of a set: the configuration's groups of 4 rows (ng in each of
+// nrow slices, where a class has more than the configuration holds)
+struct SymShape {
+    int conf, ng, nrow;
+};
+
+struct SymArgs {
+    int ncols, TB, cpt, side;
+    int ldp, ldf;              // P and Pf strides per (box, column)
+    int nrow;                  // row slices (SymShape)
+    int npz, noz;              // sum parts: classes p = zp mod npz, orbits = zo mod noz
+    int nj;                    // k steps (of 4) of all classes
+    int mk[8], kb[8];          // k steps of a class, the first one
+    int64_t out_off;           // global box offset of the level in out
+    int64_t part_stride;       // doubles between the sum parts at out
+    int class_tiles[8];        // tiles of an octant class
+    int64_t class_start[9];
+    const int32_t *order, *coord, *map;
+    const double *Ef;          // operators [orbit][row slice][k step][group][4 rows + 4 * (4 k)]
+    const double *P;           // the level's proxies: a box of zeros, then its boxes, [k / 2][column][2] each
+    double *out;
+};
+struct ZeroBoxes {
+    double *p[MAX_FAR_LEVELS];
+    int n[MAX_FAR_LEVELS];
+};
+void launch_zero_boxes(const ZeroBoxes &z, int nlevels, hipStream_t st);
+SymShape sym_shape(const int cnt[8]);
+int sym_width(const SymShape &s);  // columns of a tile
+int sym_row(const SymShape &s, int q, int i);  // Pf row of row i of class q
+void upload_sym_orbits();
+void launch_m2l_sym(const SymArgs &a, const SymShape &s, int ncolchunks, hipStream_t st);
+void launch_m2l_sym_reduce(const double *part, int nparts, int64_t stride, int64_t n, double *out, hipStream_t st);
+void launch_transpose_blocks(const double *src, int r, int c, int64_t nd, double *dst, hipStream_t st);
+void launch_sym_average(const double *Z, const int *cf, const int *cs, int rf, int rs, const int *dir, double *M,
+                        hipStream_t st);
+void launch_sym_expand(const double *K, const int *cf, const int *cs, int rf, int rs, const int *of, const int *refl,
+                       double *E, hipStream_t st);
 
 constexpr int NEAR_CLASSES = 6;
 
