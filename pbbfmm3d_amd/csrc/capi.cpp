@@ -2848,9 +2848,12 @@ PBB_API pbb_status pbb_direct_sum(const pbb_kernel_desc *kernel, const double *t
         hipStream_t st = (hipStream_t)stream;
         dev::DirectArgs a{};
         a.T = ntargets; a.Ns = nsources; a.ncols = ncols;
-        int64_t tblocks = (ntargets + 63) / 64;
-        a.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(256, (4096 + tblocks - 1) / std::max<int64_t>(1, tblocks)));
-        a.nsplit = (int)std::min<int64_t>(a.nsplit, std::max<int64_t>(1, nsources / 256));
+        // workgroups of 64 targets and one slice of the sources: 4096 and more
+        // keep the last round of the 256 CUs (two workgroups each) short;
+        // slices of fewer than 512 sources leave a wave less than its reduction
+        const int64_t tblocks = (ntargets + 63) / 64;
+        a.nsplit = (int)std::min<int64_t>(256, std::max<int64_t>(1, 4096 / std::max<int64_t>(1, tblocks)));
+        a.nsplit = (int)std::min<int64_t>(a.nsplit, std::max<int64_t>(1, nsources / 512));
         std::memcpy(a.kp.p, kernel->param, sizeof(a.kp.p));
         a.tgt = tgt_dev; a.src = src_dev; a.w = w_dev; a.out = out_dev;
         if (ntargets == 0) return;
@@ -2858,7 +2861,7 @@ PBB_API pbb_status pbb_direct_sum(const pbb_kernel_desc *kernel, const double *t
             check(hipMemsetAsync(out_dev, 0, sizeof(double) * ntargets * ncols, st), "clear output");
             return;
         }
-        a.part = dalloc<double>((size_t)a.nsplit * ncols * ntargets, "direct-sum partials");
+        if (a.nsplit > 1) a.part = dalloc<double>((size_t)a.nsplit * ncols * ntargets, "direct-sum partials");
         try {
             dev::launch_direct(a, kernel->id, st);
             check(hipStreamSynchronize(st), "hipStreamSynchronize");

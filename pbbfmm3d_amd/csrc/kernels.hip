@@ -28,15 +28,39 @@ typedef double dbl4 __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 // device kernel functors (formulas of pbb_kernel_id); r2 = |s - t|^2 with
 // the differences taken as source - target (kernel_Types.cpp:21-23)
+//
+// 1 / sqrt(x) for x other than 0 and infinity (there a NaN): the hardware's
+// estimate (2^-23) and one third-order step, 7 operations in place of a square
+// root and a division (about 35), and as close (an error of at most about one
+// unit in the last place either way)
+__device__ __forceinline__ double rsqrt_inner(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = __builtin_fma(-(x * y), y, 1.0);
+    return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double rsqrt_step(double x)
+{
+    const double z = rsqrt_inner(x);
+    return __builtin_amdgcn_class(x, 0x264) ? __builtin_amdgcn_rsq(x) : z;  // (+-0, +-infinity)
+}
+// a / b for a b that many values share (1 / b is formed once outside the
+// loop): the quotient's residual corrects it to the division's rounding
+__device__ __forceinline__ double div_shared(double a, double b)
+{
+    const double inv = 1.0 / b, q = a * inv;
+    const double z = __builtin_fma(__builtin_fma(-q, b, a), inv, q);
+    return z == z ? z : q;  // (an infinite a)
+}
 template <int KID>
 __device__ __forceinline__ double keval(double dx, double dy, double dz, const KParams &p)
 {
     double r2 = dx * dx + dy * dy + dz * dz;
-    if constexpr (KID == PBB_KERNEL_LAPLACIAN) return 1.0 / sqrt(r2);
-    else if constexpr (KID == PBB_KERNEL_ONEOVERR2) { double ri = 1.0 / sqrt(r2); return ri * ri; }
-    else if constexpr (KID == PBB_KERNEL_GAUSSIAN) return exp(-r2 / (p.p[0] * p.p[0]));
-    else if constexpr (KID == PBB_KERNEL_EXPONENTIAL) return p.p[1] * exp(-sqrt(r2) / p.p[0]);
-    else if constexpr (KID == PBB_KERNEL_SOFT_LAPLACIAN) return 1.0 / sqrt(r2 + p.p[0]);
+    if constexpr (KID == PBB_KERNEL_LAPLACIAN) return rsqrt_step(r2);
+    else if constexpr (KID == PBB_KERNEL_ONEOVERR2) { double ri = rsqrt_step(r2); return ri * ri; }
+    else if constexpr (KID == PBB_KERNEL_GAUSSIAN) return exp(-div_shared(r2, p.p[0] * p.p[0]));
+    else if constexpr (KID == PBB_KERNEL_EXPONENTIAL) return p.p[1] * exp(-div_shared(sqrt(r2), p.p[0]));
+    else if constexpr (KID == PBB_KERNEL_SOFT_LAPLACIAN) return rsqrt_step(r2 + p.p[0]);
     else if constexpr (KID == PBB_KERNEL_QUADRIC) return 1.0 + r2;
     else if constexpr (KID == PBB_KERNEL_INV_QUADRIC) return 1.0 / (1.0 + r2);
     else if constexpr (KID == PBB_KERNEL_LOGARITHM) return r2 == 0 ? 0.0 : 0.5 * log(r2);
@@ -46,6 +70,39 @@ __device__ __forceinline__ double keval(double dx, double dy, double dz, const K
     else if constexpr (KID == PBB_KERNEL_EXP_ANISO)
         return p.p[0] * exp(-sqrt(p.p[1] * dx * dx + p.p[2] * dy * dy + p.p[3] * dz * dz));
     else return 0.0;
+}
+
+// The values of the near field and the direct sum, 0 in place of an infinity
+// (coincident points).  An inverse root needs one select for that: it is 0 at
+// an infinite argument as well; a Gaussian is never infinite.
+template <int KID>
+__device__ __forceinline__ double keval0(double dx, double dy, double dz, const KParams &p)
+{
+    if constexpr (KID == PBB_KERNEL_LAPLACIAN || KID == PBB_KERNEL_SOFT_LAPLACIAN) {
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        const double x = KID == PBB_KERNEL_LAPLACIAN ? r2 : r2 + p.p[0];
+        const double z = rsqrt_inner(x);
+        return __builtin_amdgcn_class(x, 0x264) ? 0.0 : z;  // (+-0, +-infinity)
+    } else {
+        const double kv = keval<KID>(dx, dy, dz, p);
+        return KID != PBB_KERNEL_GAUSSIAN && isinf(kv) ? 0.0 : kv;
+    }
+}
+
+// The values the operators are made from.  They keep the library's square
+// root and division: within a degenerate cluster the singular vectors (and
+// with them the subspace a cut through the cluster keeps) turn with the last
+// bit of the kernel blocks.
+template <int KID>
+__device__ __forceinline__ double keval_blocks(double dx, double dy, double dz, const KParams &p)
+{
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    if constexpr (KID == PBB_KERNEL_LAPLACIAN) return 1.0 / sqrt(r2);
+    else if constexpr (KID == PBB_KERNEL_ONEOVERR2) { double ri = 1.0 / sqrt(r2); return ri * ri; }
+    else if constexpr (KID == PBB_KERNEL_GAUSSIAN) return exp(-r2 / (p.p[0] * p.p[0]));
+    else if constexpr (KID == PBB_KERNEL_EXPONENTIAL) return p.p[1] * exp(-sqrt(r2) / p.p[0]);
+    else if constexpr (KID == PBB_KERNEL_SOFT_LAPLACIAN) return 1.0 / sqrt(r2 + p.p[0]);
+    else return keval<KID>(dx, dy, dz, p);
 }
 
 // The same functors with the transcendental part in FP32 (the mixed modes'
@@ -1541,60 +1598,55 @@ __global__ __launch_bounds__(64) void near_grad_fp64(NearGradArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Direct sum (DirectCalc3D, test.hpp:18-34, isinf -> 0): partial sums of
-// one slice of the sources per workgroup row, reduced by a second kernel.
-//   part[(split*ncols + c)*T + i] = sum_{j in slice} K(t_i, s_j) w[c*Ns + j]
-constexpr int DS_TGT = 64, DS_SRC = 64, DS_CPT = 8;
+// Direct sum (DirectCalc3D, test.hpp:18-34, isinf -> 0): a workgroup holds 64
+// targets, one per lane, its 16 waves a sixteenth of one slice of the sources
+// each.  A wave's source is the same for all its lanes, so positions and
+// weights come through the scalar cache and cost no LDS; the VALU evaluates
+// each kernel value once for NC columns.  With one slice (enough targets to
+// fill the GPU) the sums go straight to out, else to part[(split*ncols + c)*T
+// + i], reduced by a second kernel.
+// Bound: the VALU, some 16 FP64 operations a pair.  50k x 50k points, 1/r, 1
+// column: 14.3 ms with sources in LDS, a slice per wave and the library's root
+// and division, 1.43 ms here (1.75e12 pairs/s; its operations alone 1.1 ms).
+constexpr int DS_TGT = 64, DS_WAVES = 16;
 
-template <int KID>
-__global__ __launch_bounds__(256) void direct_partial(DirectArgs a)
+template <int KID, int NC>
+__global__ __launch_bounds__(64 * DS_WAVES) void direct_partial(DirectArgs a, int c0)
 {
-    __shared__ double sx[DS_SRC], sy[DS_SRC], sz[DS_SRC];
-    __shared__ double sw[4 * DS_CPT][DS_SRC];
-    const int tid = threadIdx.x, slot = tid / 4, g = tid % 4;
-    const int64_t i = (int64_t)blockIdx.x * DS_TGT + slot;
+    __shared__ double sh[DS_WAVES][DS_TGT];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t i = (int64_t)blockIdx.x * DS_TGT + lane;
     const int split = blockIdx.y;
     const int64_t per = (a.Ns + a.nsplit - 1) / a.nsplit;
-    const int64_t j0s = split * per, j1s = min(a.Ns, j0s + per);
+    const int64_t s0 = split * per, s1 = min(a.Ns, s0 + per);
+    const int64_t pw = s1 > s0 ? (s1 - s0 + DS_WAVES - 1) / DS_WAVES : 0;
+    const int64_t j0 = s0 + wave * pw, j1 = min(s1, j0 + pw);
     const bool active = i < a.T;
-    double xi = 0, yi = 0, zi = 0;
-    if (active) { xi = a.tgt[3 * i]; yi = a.tgt[3 * i + 1]; zi = a.tgt[3 * i + 2]; }
-    for (int c0 = 0; c0 < a.ncols; c0 += 4 * DS_CPT) {
-        const int cn = min(4 * DS_CPT, a.ncols - c0);
-        double acc[DS_CPT];
+    const int64_t it = active ? i : 0;
+    const double xi = a.tgt[3 * it], yi = a.tgt[3 * it + 1], zi = a.tgt[3 * it + 2];
+    const int cn = min(NC, a.ncols - c0);
+    const double *__restrict__ src = a.src;
+    const double *__restrict__ w = a.w + (int64_t)c0 * a.Ns;
+    double acc[NC];
 #pragma unroll
-        for (int k = 0; k < DS_CPT; k++) acc[k] = 0;
-        for (int64_t j0 = j0s; j0 < j1s; j0 += DS_SRC) {
-            const int jn = (int)min((int64_t)DS_SRC, j1s - j0);
-            __syncthreads();
-            if (tid < jn) {
-                sx[tid] = a.src[3 * (j0 + tid)];
-                sy[tid] = a.src[3 * (j0 + tid) + 1];
-                sz[tid] = a.src[3 * (j0 + tid) + 2];
-            }
-            for (int q = tid; q < cn * DS_SRC; q += 256) {
-                int c = q / DS_SRC, p = q % DS_SRC;
-                sw[c][p] = p < jn ? a.w[(int64_t)(c0 + c) * a.Ns + j0 + p] : 0.0;
-            }
-            __syncthreads();
-            if (active) {
-                for (int p = 0; p < jn; p++) {
-                    double kv = keval<KID>(sx[p] - xi, sy[p] - yi, sz[p] - zi, a.kp);
-                    if (isinf(kv)) kv = 0.0;
+    for (int k = 0; k < NC; k++) acc[k] = 0;
+#pragma unroll 4
+    for (int64_t j = j0; j < j1; j++) {
+        const double kv = keval0<KID>(src[3 * j] - xi, src[3 * j + 1] - yi, src[3 * j + 2] - zi, a.kp);
 #pragma unroll
-                    for (int k = 0; k < DS_CPT; k++) {
-                        int cl = g + 4 * k;
-                        if (cl < cn) acc[k] += kv * sw[cl][p];
-                    }
-                }
-            }
-        }
-        if (active) {
+        for (int k = 0; k < NC; k++) acc[k] += kv * w[(int64_t)min(k, cn - 1) * a.Ns + j];
+    }
 #pragma unroll
-            for (int k = 0; k < DS_CPT; k++) {
-                int cl = g + 4 * k;
-                if (cl < cn) a.part[((int64_t)split * a.ncols + c0 + cl) * a.T + i] = acc[k];
-            }
+    for (int k = 0; k < NC; k++) {
+        if (k >= cn) break;
+        __syncthreads();
+        sh[wave][lane] = acc[k];
+        __syncthreads();
+        if (wave == 0 && active) {
+            double s = 0;
+            for (int v = 0; v < DS_WAVES; v++) s += sh[v][lane];
+            double *dst = a.nsplit > 1 ? a.part + (int64_t)split * a.ncols * a.T : a.out;
+            dst[(int64_t)(c0 + k) * a.T + i] = s;
         }
     }
 }
@@ -1848,21 +1900,27 @@ void launch_direct(const DirectArgs &a, int kid, hipStream_t st)
 {
     if (a.T <= 0) return;
     dim3 grid((unsigned)((a.T + DS_TGT - 1) / DS_TGT), (unsigned)a.nsplit);
-#define PBB_DIRECT_CASE(K)                                \
-    case K:                                               \
-        direct_partial<K><<<grid, 256, 0, st>>>(a);       \
+    for (int c0 = 0; c0 < a.ncols; c0 += 16) {
+        const int cn = a.ncols - c0;
+#define PBB_DIRECT_CASE(K)                                                                   \
+    case K:                                                                                  \
+        if (cn <= 1) direct_partial<K, 1><<<grid, 64 * DS_WAVES, 0, st>>>(a, c0);            \
+        else if (cn <= 4) direct_partial<K, 4><<<grid, 64 * DS_WAVES, 0, st>>>(a, c0);       \
+        else direct_partial<K, 16><<<grid, 64 * DS_WAVES, 0, st>>>(a, c0);                   \
         break;
-    switch (kid) {
-        PBB_DIRECT_CASE(PBB_KERNEL_LAPLACIAN) PBB_DIRECT_CASE(PBB_KERNEL_ONEOVERR2)
-        PBB_DIRECT_CASE(PBB_KERNEL_GAUSSIAN) PBB_DIRECT_CASE(PBB_KERNEL_EXPONENTIAL)
-        PBB_DIRECT_CASE(PBB_KERNEL_SOFT_LAPLACIAN) PBB_DIRECT_CASE(PBB_KERNEL_QUADRIC)
-        PBB_DIRECT_CASE(PBB_KERNEL_INV_QUADRIC) PBB_DIRECT_CASE(PBB_KERNEL_LOGARITHM)
-        PBB_DIRECT_CASE(PBB_KERNEL_THIN_PLATE) PBB_DIRECT_CASE(PBB_KERNEL_R2)
-        PBB_DIRECT_CASE(PBB_KERNEL_CONSTANT) PBB_DIRECT_CASE(PBB_KERNEL_EXP_ANISO)
-    default: fail(PBB_ERR_UNSUPPORTED, "no device functor for this kernel id");
-    }
+        switch (kid) {
+            PBB_DIRECT_CASE(PBB_KERNEL_LAPLACIAN) PBB_DIRECT_CASE(PBB_KERNEL_ONEOVERR2)
+            PBB_DIRECT_CASE(PBB_KERNEL_GAUSSIAN) PBB_DIRECT_CASE(PBB_KERNEL_EXPONENTIAL)
+            PBB_DIRECT_CASE(PBB_KERNEL_SOFT_LAPLACIAN) PBB_DIRECT_CASE(PBB_KERNEL_QUADRIC)
+            PBB_DIRECT_CASE(PBB_KERNEL_INV_QUADRIC) PBB_DIRECT_CASE(PBB_KERNEL_LOGARITHM)
+            PBB_DIRECT_CASE(PBB_KERNEL_THIN_PLATE) PBB_DIRECT_CASE(PBB_KERNEL_R2)
+            PBB_DIRECT_CASE(PBB_KERNEL_CONSTANT) PBB_DIRECT_CASE(PBB_KERNEL_EXP_ANISO)
+        default: fail(PBB_ERR_UNSUPPORTED, "no device functor for this kernel id");
+        }
 #undef PBB_DIRECT_CASE
-    check(hipGetLastError(), "direct_partial");
+        check(hipGetLastError(), "direct_partial");
+    }
+    if (a.nsplit <= 1) return;
     int64_t total = a.T * a.ncols;
     int blocks = (int)std::min<int64_t>((total + 255) / 256, 65536);
     direct_reduce<<<blocks, 256, 0, st>>>(a.part, a.nsplit, total, a.out);
@@ -1911,7 +1969,7 @@ __global__ __launch_bounds__(256) void kernel_blocks_dev(KernelBlockArgs a)
         const double s0 = (a.dirs[3 * d] + 0.5 * a.nodes[j1]) * a.box_len,
                      s1 = (a.dirs[3 * d + 1] + 0.5 * a.nodes[j2]) * a.box_len,
                      s2 = (a.dirs[3 * d + 2] + 0.5 * a.nodes[j3]) * a.box_len;
-        a.Kcell[q] = keval<KID>(s0 - t0, s1 - t1, s2 - t2, a.kp) / (a.Kw[i] * a.Kw[j]);
+        a.Kcell[q] = keval_blocks<KID>(s0 - t0, s1 - t1, s2 - t2, a.kp) / (a.Kw[i] * a.Kw[j]);
     }
 }
 
