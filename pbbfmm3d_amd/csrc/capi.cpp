@@ -870,6 +870,7 @@ static size_t layout_workspace(const pbb_plan &p, int ncols, bool mixed, const F
     const int rmax = std::max(h.rf, h.rs);
     W = Workspace{};
     W.ncols = ncols;
+    W.all = d.all;
     W.mixed = mixed ? 1 : 0;
     W.kpad = 32 * ((rmax + 31) / 32);
     W.ws = (double *)take(Nc * sizeof(double));
@@ -889,7 +890,6 @@ static size_t layout_workspace(const pbb_plan &p, int ncols, bool mixed, const F
             W.P = (double *)take((Bc + (d.sym ? (size_t)(p.Lv - 1) * ncols : 0)) * d.ldp * sizeof(double));
             W.Pf = (double *)take(Bc * d.ldf * sizeof(double));
             W.part_cap = d.part_cap;
-            W.all = d.all;
             if (d.part) W.part = (double *)take(d.part * sizeof(double));
         }
     }
@@ -2477,6 +2477,8 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
         a.leaf_class = p->leaf_class;
         std::copy(std::begin(p->leaf_class_off), std::end(p->leaf_class_off), a.leaf_class_off);
         a.kf32 = mixed ? 1 : 0;
+        a.max_leaf = (int)p->info.max_leaf_points;
+        a.all = W.all;
         if (!(direct && dev::launch_near_split(a, h.kernel.id, (int)LL.nb, st)))
             dev::launch_near(a, h.kernel.id, (int)LL.nb, st);
     }

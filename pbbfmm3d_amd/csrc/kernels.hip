@@ -853,13 +853,7 @@ __global__ __launch_bounds__(64) void near_fp64(NearArgs a)
 //             with coalesced loads; lanes (target, column, part) split the
 //             n^3 sum and reduce across the parts, so that leaves of one or
 //             two points keep every lane busy.
-//   p2p_fp64  P2P (compute.hpp:650-737) + scatter (:739-749) on top of lp.
-//             One wave per leaf; lane (i, g) holds columns g, g+G, ... of
-//             target i (G = 64 / targets per pass) in registers.  Source
-//             chunks of 32 points (positions, point-major weights) are staged
-//             in LDS while the next chunk is loaded.  Passes of up to 16
-//             targets evaluate each K(t, s) once into LDS; wider passes
-//             evaluate it per lane (at most 2 lanes per target).
+//   p2p_*     P2P + scatter on top of lp (below)
 
 constexpr int L2P_CC = 8;    // columns of F staged per step
 constexpr int L2P_TGT = 32;  // targets per pass
@@ -1129,35 +1123,148 @@ __global__ void p2m_reduce(UpReduce r)
     }
 }
 
-constexpr int P2P_SC = 32;  // source points per LDS chunk
-constexpr int P2P_NC = 32;  // columns per pass
-constexpr int P2P_SK = 16;  // passes of at most this many targets share K through LDS
-
-struct P2PShared {
-    double sw[P2P_SC][P2P_NC + 1];
-    double sx[P2P_SC], sy[P2P_SC], sz[P2P_SC];
-    double sK[P2P_SK][P2P_SC + 1];
-    double tx[P2P_SK], ty[P2P_SK], tz[P2P_SK];
-    int s_start[27], s_pre[28];
+// P2P (compute.hpp:650-737) + scatter (:739-749) on top of the L2P sums lp:
+// one wave per leaf (or per pass over a large leaf's targets), the largest
+// first.  The neighbours' points form one index
+// space, staged in LDS chunk by chunk.  Three ways to share the work, by
+// columns and leaf size:
+//   p2p_few    up to 8 columns: lane (i, g) takes every G-th source for target
+//              i and all columns, so a kernel value is evaluated once and used
+//              from a register; the G lanes of a target add up at the end.
+//   p2p_small  more columns, leaves of up to 16 targets: each value goes
+//              through LDS to the lanes that hold the target's columns.
+//   p2p_dense  more columns, larger leaves: the matrix cores sum.
+// A launch per leaf class, the passes of a large leaf one after another in one
+// workgroup, left a tail of a few waves: 5k points, 1 column 200 us -> 16 us;
+// 1M uniform points, 1/r, 8 columns (1e8 pairs) 1.82 -> 0.95 ms (bound by the
+// VALU: 24 FP64 operations a pair and the staging of 4 points a leaf); 1M
+// clustered points, Gaussian in FP32, 32 columns (1.7e9 pairs) 12.3 -> 6.8 ms
+// (bound by kernel values and products, which share the SIMD's issue slots).
+struct P2PRange {
+    int start[27], pre[28];
 };
 
-template <int KID, int TT>
-__device__ __forceinline__ void p2p_pass(const NearArgs &a, P2PShared &sh, int t0, int i0, int tn, int c0,
-                                         int cn, int ns)
+// The leaf's neighbours: first points and, added up, their counts (wave scan)
+__device__ __forceinline__ void p2p_range(const NearArgs &a, int b, P2PRange &r)
 {
-    constexpr int G = 64 / TT, CPL = P2P_NC / G, WR = P2P_SC * P2P_NC / 64;
-    constexpr bool SHARED_K = TT <= P2P_SK;
-    const int lane = threadIdx.x, i = lane / G, g = lane % G;
-    const bool active = i < tn;
-    const int64_t ti = t0 + i0 + (active ? i : 0);
-    const double tx = a.x[ti], ty = a.y[ti], tz = a.z[ti];
-    if constexpr (SHARED_K) {
-        __syncthreads();
-        if (lane < tn) {
-            sh.tx[lane] = a.x[t0 + i0 + lane];
-            sh.ty[lane] = a.y[t0 + i0 + lane];
-            sh.tz[lane] = a.z[t0 + i0 + lane];
+    const int lane = threadIdx.x;
+    const uint32_t cc = (uint32_t)a.coord[b];
+    const int ix = cc & 1023, iy = (cc >> 10) & 1023, iz = (cc >> 20) & 1023;
+    const int S = a.side;
+    int start = 0, cnt = 0;
+    if (lane < 27) {
+        const int x = ix + lane / 9 - 1, y = iy + (lane / 3) % 3 - 1, z = iz + lane % 3 - 1;
+        const int sb = (x >= 0 && y >= 0 && z >= 0 && x < S && y < S && z < S) ? a.map[((int64_t)x * S + y) * S + z] : -1;
+        if (sb >= 0) {
+            start = a.leaf_start[sb];
+            cnt = a.leaf_start[sb + 1] - start;
         }
+        r.start[lane] = start;
+    }
+    int sum = cnt;
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) {
+        const int v = __shfl_up(sum, o);
+        if (lane >= o) sum += v;
+    }
+    if (lane < 27) r.pre[lane + 1] = sum;
+    if (lane == 0) r.pre[0] = 0;
+    __syncthreads();
+}
+
+// Point q of the neighbours' index space; m: the neighbour found for a
+// smaller q before (0 at the start)
+__device__ __forceinline__ int p2p_point(const P2PRange &r, int q, int &m)
+{
+    while (r.pre[m + 1] <= q) m++;
+    return r.start[m] + q - r.pre[m];
+}
+
+template <int KID, int NC>
+__device__ __forceinline__ void p2p_few(const NearArgs &a, const P2PRange &r, double *lds, int t0, int nt, int i0, int lg,
+                                        bool f32)
+{
+    // lds: positions x, y, z and NC weights of 64 sources
+    double *sx = lds, *sy = lds + 64, *sz = lds + 128, *sw = lds + 192;
+    const int lane = threadIdx.x, G = 64 >> lg, i = lane >> (6 - lg), g = lane & (G - 1);
+    const bool active = i0 + i < nt;
+    const int64_t ti = t0 + (active ? i0 + i : 0);
+    const double tx = a.x[ti], ty = a.y[ti], tz = a.z[ti];
+    const int ns = r.pre[27], cn = a.ncols;
+    double acc[NC], px = 0, py = 0, pz = 0, pw[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) acc[c] = pw[c] = 0;
+    int m = 0;
+    auto load = [&](int j0) {
+        if (j0 + lane < ns) {
+            const int64_t gi = p2p_point(r, j0 + lane, m);
+            px = a.x[gi];
+            py = a.y[gi];
+            pz = a.z[gi];
+#pragma unroll
+            for (int c = 0; c < NC; c++) pw[c] = c < cn ? a.wsT[gi * cn + c] : 0.0;
+        }
+    };
+    load(0);
+    for (int j0 = 0; j0 < ns; j0 += 64) {
+        const int jn = min(64, ns - j0);
+        __syncthreads();  // the previous chunk is consumed
+        sx[lane] = px;
+        sy[lane] = py;
+        sz[lane] = pz;
+#pragma unroll
+        for (int c = 0; c < NC; c++) sw[lane * NC + c] = pw[c];
+        __syncthreads();
+        load(j0 + 64);  // in flight during the sums
+        if (f32) {
+            for (int j = g; j < jn; j += G) {
+                double kv = keval_f32<KID>(sx[j] - tx, sy[j] - ty, sz[j] - tz, a.kp);
+                if (isinf(kv)) kv = 0.0;
+#pragma unroll
+                for (int c = 0; c < NC; c++) acc[c] += kv * sw[j * NC + c];
+            }
+        } else {
+#pragma unroll 2
+            for (int j = g; j < jn; j += G) {
+                const double kv = keval0<KID>(sx[j] - tx, sy[j] - ty, sz[j] - tz, a.kp);
+#pragma unroll
+                for (int c = 0; c < NC; c++) acc[c] += kv * sw[j * NC + c];
+            }
+        }
+    }
+    for (int o = 1; o < G; o <<= 1) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) acc[c] += __shfl_xor(acc[c], o);
+    }
+    const int64_t oi = active && g == 0 ? a.perm[ti] - a.out_lo : -1;
+    if ((uint64_t)oi < (uint64_t)a.out_n) {
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+            if (c < cn) a.out[(int64_t)c * a.out_n + oi] += a.lp ? acc[c] + a.lp[ti * cn + c] : acc[c];
+    }
+}
+
+constexpr int P2P_DENSE = 4;  // first leaf class (17 targets and more) of the matrix cores
+constexpr int P2P_SC = 32;  // source points per LDS chunk
+constexpr int P2P_NC = 32;  // columns per pass
+constexpr int P2P_WS = P2P_NC + 1;
+
+// lds: weights [P2P_SC][P2P_WS], then x, y, z of the sources, then the kernel
+// values [16][P2P_SC + 1] and the targets' x, y, z
+template <int KID, int TT>
+__device__ __forceinline__ void p2p_small(const NearArgs &a, const P2PRange &r, double *lds, int t0, int tn, int c0)
+{
+    constexpr int G = 64 / TT, CPL = P2P_NC / G, WR = P2P_SC * P2P_NC / 64, KS = P2P_SC + 1;
+    double *sw = lds, *sx = lds + P2P_SC * P2P_WS, *sy = sx + P2P_SC, *sz = sy + P2P_SC, *sK = sz + P2P_SC,
+           *stx = sK + 16 * KS, *sty = stx + 16, *stz = sty + 16;
+    const int lane = threadIdx.x, i = lane / G, g = lane % G;
+    const int cn = min(P2P_NC, a.ncols - c0), ns = r.pre[27];
+    const bool active = i < tn;
+    const int64_t ti = t0 + (active ? i : 0);
+    if (lane < tn) {
+        stx[lane] = a.x[t0 + lane];
+        sty[lane] = a.y[t0 + lane];
+        stz[lane] = a.z[t0 + lane];
     }
     double acc[CPL];
 #pragma unroll
@@ -1166,23 +1273,22 @@ __device__ __forceinline__ void p2p_pass(const NearArgs &a, P2PShared &sh, int t
         acc[k] = (a.lp && active && cl < cn) ? a.lp[ti * a.ncols + c0 + cl] : 0.0;
     }
     double pw[WR], px = 0, py = 0, pz = 0;
+    int m = 0;
     auto load = [&](int j0) {
         const int jn = min(P2P_SC, ns - j0);
         int gi = 0;
         if (lane < jn) {
-            const int q = j0 + lane;
-            int m = 0;
-            while (sh.s_pre[m + 1] <= q) m++;
-            gi = sh.s_start[m] + q - sh.s_pre[m];
+            gi = p2p_point(r, j0 + lane, m);
             px = a.x[gi];
             py = a.y[gi];
             pz = a.z[gi];
         }
 #pragma unroll
-        for (int r = 0; r < WR; r++) {
-            const int u = lane + 64 * r, j = u / P2P_NC, c = u % P2P_NC;
+        for (int k = 0; k < WR; k++) {
+            const int u = lane + 64 * k, j = u / P2P_NC, c = u % P2P_NC;
             const int gj = __shfl(gi, j);
-            pw[r] = (j < jn && c < cn) ? a.wsT[(int64_t)gj * a.ncols + c0 + c] : 0.0;
+            const double v = a.wsT[(int64_t)gj * a.ncols + c0 + min(c, cn - 1)];
+            pw[k] = (j < jn && c < cn) ? v : 0.0;
         }
     };
     if (ns > 0) load(0);
@@ -1190,43 +1296,30 @@ __device__ __forceinline__ void p2p_pass(const NearArgs &a, P2PShared &sh, int t
         const int jn = min(P2P_SC, ns - j0);
         __syncthreads();  // the previous chunk is consumed
 #pragma unroll
-        for (int r = 0; r < WR; r++) {
-            const int u = lane + 64 * r;
-            sh.sw[u / P2P_NC][u % P2P_NC] = pw[r];
+        for (int k = 0; k < WR; k++) {
+            const int u = lane + 64 * k;
+            sw[(u / P2P_NC) * P2P_WS + u % P2P_NC] = pw[k];
         }
         if (lane < P2P_SC) {
-            sh.sx[lane] = px;
-            sh.sy[lane] = py;
-            sh.sz[lane] = pz;
+            sx[lane] = px;
+            sy[lane] = py;
+            sz[lane] = pz;
         }
         __syncthreads();
         if (j0 + P2P_SC < ns) load(j0 + P2P_SC);  // in flight during the sums
-        if constexpr (SHARED_K) {
-            for (int q = lane; q < TT * P2P_SC; q += 64) {
-                const int ii = q / P2P_SC, jj = q % P2P_SC;
-                double kv = 0.0;
-                if (ii < tn && jj < jn) {
-                    kv = keval<KID>(sh.sx[jj] - sh.tx[ii], sh.sy[jj] - sh.ty[ii], sh.sz[jj] - sh.tz[ii], a.kp);
-                    if (isinf(kv)) kv = 0.0;
-                }
-                sh.sK[ii][jj] = kv;
-            }
-            __syncthreads();
-            if (active)
-                for (int jj = 0; jj < jn; jj++) {
-                    const double kv = sh.sK[i][jj];
-#pragma unroll
-                    for (int k = 0; k < CPL; k++) acc[k] += kv * sh.sw[jj][g + G * k];
-                }
-        } else {
-            if (active)
-                for (int jj = 0; jj < jn; jj++) {
-                    double kv = keval<KID>(sh.sx[jj] - tx, sh.sy[jj] - ty, sh.sz[jj] - tz, a.kp);
-                    if (isinf(kv)) kv = 0.0;
-#pragma unroll
-                    for (int k = 0; k < CPL; k++) acc[k] += kv * sh.sw[jj][g + G * k];
-                }
+        for (int q = lane; q < TT * P2P_SC; q += 64) {
+            const int ii = q / P2P_SC, jj = q % P2P_SC;
+            double kv = 0.0;
+            if (ii < tn && jj < jn) kv = keval0<KID>(sx[jj] - stx[ii], sy[jj] - sty[ii], sz[jj] - stz[ii], a.kp);
+            sK[ii * KS + jj] = kv;
         }
+        __syncthreads();
+        if (active)
+            for (int jj = 0; jj < jn; jj++) {
+                const double kv = sK[i * KS + jj];
+#pragma unroll
+                for (int k = 0; k < CPL; k++) acc[k] += kv * sw[jj * P2P_WS + g + G * k];
+            }
     }
     const int64_t oi = active ? a.perm[ti] - a.out_lo : -1;
     if ((uint64_t)oi < (uint64_t)a.out_n) {
@@ -1238,148 +1331,169 @@ __device__ __forceinline__ void p2p_pass(const NearArgs &a, P2PShared &sh, int t
     }
 }
 
-// one workgroup per leaf of a list whose leaves hold at most TT targets (or
-// more, in passes of TT, for the widest class)
-template <int KID, int TT>
-__global__ __launch_bounds__(64) void p2p_fp64(NearArgs a, const int32_t *__restrict__ leaves)
+// K (targets x sources) times W (sources x columns) is a product of 16 x 4
+// blocks of K with 4 x 16 blocks of W: the A fragment of
+// v_mfma_f64_16x16x4f64 holds one value per lane, so each lane evaluates the
+// kernel for its (target, source) entry of every block and the matrix cores
+// accumulate 16*TB targets x 16*CB columns in FP64.  FP64 matrix
+// instructions keep the VALU of their SIMD busy, so the two add up: 64 pairs
+// x 32 columns cost 128 cycles of products and the 64 kernel values.  KF32
+// (mixed modes): the kernel values in FP32 (keval_f32), the sums still FP64.
+// lds: weights [P2P_SC][P2P_WS], then x, y, z of the sources.
+template <int KID, int TB, int CB, bool KF32>
+__device__ __forceinline__ void p2p_dense(const NearArgs &a, const P2PRange &r, double *lds, int t0, int nt, int i0, int c0)
 {
-    __shared__ P2PShared sh;
-    const int b = leaves[blockIdx.x], lane = threadIdx.x;
+    double *sw = lds, *sx = lds + P2P_SC * P2P_WS, *sy = sx + P2P_SC, *sz = sy + P2P_SC;
+    const int lane = threadIdx.x, fr = lane & 15, fk = lane >> 4;
+    const int cn = min(16 * CB, a.ncols - c0), ns = r.pre[27];
+    // this lane's target row fr of each 16-target block (rows past the leaf
+    // repeat its last target; their sums are not stored)
+    double tx[TB], ty[TB], tz[TB];
+#pragma unroll
+    for (int tb = 0; tb < TB; tb++) {
+        const int64_t ti = t0 + min(i0 + tb * 16 + fr, nt - 1);
+        tx[tb] = a.x[ti];
+        ty[tb] = a.y[ti];
+        tz[tb] = a.z[ti];
+    }
+    // accumulators: D[fk + 4v][fr] of block (tb, cb), with the L2P sums
+    dbl4 acc[TB][CB];
+#pragma unroll
+    for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+        for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int ti = i0 + tb * 16 + fk + 4 * v, col = cb * 16 + fr;
+                acc[tb][cb][v] = (a.lp && ti < nt && col < cn) ? a.lp[(int64_t)(t0 + ti) * a.ncols + c0 + col] : 0.0;
+            }
+    int m = 0;
+    for (int j0 = 0; j0 < ns; j0 += P2P_SC) {
+        const int jn = min(P2P_SC, ns - j0);
+        __syncthreads();  // the previous chunk is consumed
+        int gi = 0;
+        if (lane < jn) {
+            gi = p2p_point(r, j0 + lane, m);
+            sx[lane] = a.x[gi];
+            sy[lane] = a.y[gi];
+            sz[lane] = a.z[gi];
+        }
+        constexpr int NC = 16 * CB;
+#pragma unroll
+        for (int k = 0; k < P2P_SC * NC / 64; k++) {
+            const int u = lane + 64 * k, j = u / NC, c = u % NC;
+            const int gj = __shfl(gi, j);
+            const double v = a.wsT[(int64_t)gj * a.ncols + c0 + min(c, cn - 1)];
+            sw[j * P2P_WS + c] = (j < jn && c < cn) ? v : 0.0;
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int k0 = 0; k0 < jn; k0 += 4) {
+            const int jj = k0 + fk;  // this lane's source of the 4-block (padding sources carry zero weights)
+            const int js = min(jj, jn - 1);
+            const double px = sx[js], py = sy[js], pz = sz[js];
+            double b[CB];
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++) b[cb] = sw[jj * P2P_WS + cb * 16 + fr];
+#pragma unroll
+            for (int tb = 0; tb < TB; tb++) {
+                double kv = KF32 ? keval_f32<KID>(px - tx[tb], py - ty[tb], pz - tz[tb], a.kp)
+                                 : keval0<KID>(px - tx[tb], py - ty[tb], pz - tz[tb], a.kp);
+                if ((KF32 && isinf(kv)) || jj >= jn) kv = 0.0;  // (padding sources add nothing)
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++)
+                    acc[tb][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv, b[cb], acc[tb][cb], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int ti = i0 + tb * 16 + fk + 4 * v;
+            if (ti >= nt) continue;
+            const int64_t oi = a.perm[t0 + ti] - a.out_lo;
+            if ((uint64_t)oi >= (uint64_t)a.out_n) continue;
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++) {
+                const int col = cb * 16 + fr;
+                if (col < cn) a.out[(int64_t)(c0 + col) * a.out_n + oi] += acc[tb][cb][v];
+            }
+        }
+}
+
+// Workgroup w of a launch over the classes lo..hi: its leaf class (the largest
+// leaves first, then class by class), leaf and pass of 64 targets (the last
+// class only)
+__device__ __forceinline__ int p2p_leaf(const NearArgs &a, int lo, int hi, int w, int &c, int &pass)
+{
+    c = hi;
+    pass = 0;
+    if (c == NEAR_CLASSES - 1) {
+        const int big = a.leaf_class_off[c + 1] - a.leaf_class_off[c];
+        if (w < big * a.passes) {
+            pass = w / big;
+            return a.leaf_class[a.leaf_class_off[c] + w - pass * big];
+        }
+        w -= big * a.passes;
+        c--;
+    }
+    for (; c > lo; c--) {
+        const int n = a.leaf_class_off[c + 1] - a.leaf_class_off[c];
+        if (w < n) break;
+        w -= n;
+    }
+    return a.leaf_class[a.leaf_class_off[c] + w];
+}
+
+template <int KID, int NC>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void p2p_few_columns(NearArgs a)
+{
+    __shared__ double lds[64 * (3 + NC)];
+    __shared__ P2PRange r;
+    int c, pass;
+    const int b = p2p_leaf(a, 0, NEAR_CLASSES - 1, blockIdx.x, c, pass);
     const int t0 = a.leaf_start[b], nt = a.leaf_start[b + 1] - t0;
-    const uint32_t cc = (uint32_t)a.coord[b];
-    const int ix = cc & 1023, iy = (cc >> 10) & 1023, iz = (cc >> 20) & 1023;
-    const int S = a.side;
-    if (lane < 27) {
-        const int x = ix + lane / 9 - 1, y = iy + (lane / 3) % 3 - 1, z = iz + lane % 3 - 1;
-        const int sb = (x >= 0 && y >= 0 && z >= 0 && x < S && y < S && z < S) ? a.map[((int64_t)x * S + y) * S + z] : -1;
-        sh.s_start[lane] = sb >= 0 ? a.leaf_start[sb] : 0;
-        sh.s_pre[lane + 1] = sb >= 0 ? a.leaf_start[sb + 1] - a.leaf_start[sb] : 0;
-    }
-    __syncthreads();
-    if (lane == 0) {
-        sh.s_pre[0] = 0;
-        for (int m = 0; m < 27; m++) sh.s_pre[m + 1] += sh.s_pre[m];
-    }
-    __syncthreads();
-    const int ns = sh.s_pre[27];
-    for (int c0 = 0; c0 < a.ncols; c0 += P2P_NC) {
-        const int cn = min(P2P_NC, a.ncols - c0);
-        for (int i0 = 0; i0 < nt; i0 += TT) p2p_pass<KID, TT>(a, sh, t0, i0, min(TT, nt - i0), c0, cn, ns);
+    if (pass * 64 >= nt) return;
+    p2p_range(a, b, r);
+    p2p_few<KID, NC>(a, r, lds, t0, nt, pass * 64, c + 1, a.kf32 && c >= P2P_DENSE);
+}
+
+template <int KID>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void p2p_small_leaves(NearArgs a)
+{
+    __shared__ double lds[P2P_SC * (P2P_WS + 3) + 16 * (P2P_SC + 1) + 48];
+    __shared__ P2PRange r;
+    int c, pass;
+    const int b = p2p_leaf(a, 0, P2P_DENSE - 1, blockIdx.x, c, pass);
+    const int t0 = a.leaf_start[b], nt = a.leaf_start[b + 1] - t0, c0 = blockIdx.y * P2P_NC;
+    p2p_range(a, b, r);
+    switch (c) {
+    case 0: p2p_small<KID, 2>(a, r, lds, t0, nt, c0); break;
+    case 1: p2p_small<KID, 4>(a, r, lds, t0, nt, c0); break;
+    case 2: p2p_small<KID, 8>(a, r, lds, t0, nt, c0); break;
+    default: p2p_small<KID, 16>(a, r, lds, t0, nt, c0);
     }
 }
 
-// Near field of the dense leaves on the FP64 matrix cores (leaves of 16 or
-// more targets).  K (targets x sources) times W (sources x columns) is a
-// product of 16 x 4 blocks of K with 4 x 16 blocks of W: the A fragment of
-// v_mfma_f64_16x16x4f64 holds one value per lane, so each lane evaluates
-// the kernel for its (target, source) entry of every block and the matrix
-// cores accumulate 16*TB targets x 32 columns in FP64; the VALU only
-// evaluates kernels.  Sources are staged 32 at a time in LDS as in
-// p2p_fp64; the result (with the leaf's L2P sums) is added to the output
-// through perm, in FP64 as there.  KF32 (mixed modes): the kernel values in
-// FP32 (keval_f32), the sums still FP64.
-constexpr int PM_SC = 32;
-
-template <int KID, int TB, bool KF32>
-__global__ __launch_bounds__(64) void p2p_mfma(NearArgs a, const int32_t *__restrict__ leaves)
+template <int KID, bool KF32>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void p2p_dense_leaves(NearArgs a)
 {
-    __shared__ double sw[PM_SC][33];
-    __shared__ double sx[PM_SC], sy[PM_SC], sz[PM_SC];
-    __shared__ int s_start[27], s_pre[28];
-    const int lane = threadIdx.x, fr = lane & 15, fk = lane >> 4;
-    const int b = leaves[blockIdx.x];
-    const int t0 = a.leaf_start[b], nt = a.leaf_start[b + 1] - t0;
-    const uint32_t cc = (uint32_t)a.coord[b];
-    const int ix = cc & 1023, iy = (cc >> 10) & 1023, iz = (cc >> 20) & 1023;
-    const int S = a.side;
-    if (lane < 27) {
-        const int x = ix + lane / 9 - 1, y = iy + (lane / 3) % 3 - 1, z = iz + lane % 3 - 1;
-        const int sb = (x >= 0 && y >= 0 && z >= 0 && x < S && y < S && z < S) ? a.map[((int64_t)x * S + y) * S + z] : -1;
-        s_start[lane] = sb >= 0 ? a.leaf_start[sb] : 0;
-        s_pre[lane + 1] = sb >= 0 ? a.leaf_start[sb + 1] - a.leaf_start[sb] : 0;
-    }
-    __syncthreads();
-    if (lane == 0) {
-        s_pre[0] = 0;
-        for (int m = 0; m < 27; m++) s_pre[m + 1] += s_pre[m];
-    }
-    __syncthreads();
-    const int ns = s_pre[27];
-    for (int c0 = 0; c0 < a.ncols; c0 += 32) {
-        const int cn = min(32, a.ncols - c0);
-        for (int i0 = 0; i0 < nt; i0 += 16 * TB) {
-            // this lane's target row fr of each 16-target block (rows past
-            // the leaf repeat its last target; their sums are not stored)
-            double tx[TB], ty[TB], tz[TB];
-#pragma unroll
-            for (int tb = 0; tb < TB; tb++) {
-                const int64_t ti = t0 + min(i0 + tb * 16 + fr, nt - 1);
-                tx[tb] = a.x[ti];
-                ty[tb] = a.y[ti];
-                tz[tb] = a.z[ti];
-            }
-            // accumulators: D[fk + 4v][fr] of block (tb, cb), with the L2P sums
-            dbl4 acc[TB][2];
-#pragma unroll
-            for (int tb = 0; tb < TB; tb++)
-#pragma unroll
-                for (int cb = 0; cb < 2; cb++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        const int ti = i0 + tb * 16 + fk + 4 * v, col = cb * 16 + fr;
-                        acc[tb][cb][v] = (a.lp && ti < nt && col < cn) ? a.lp[(int64_t)(t0 + ti) * a.ncols + c0 + col] : 0.0;
-                    }
-            for (int j0 = 0; j0 < ns; j0 += PM_SC) {
-                const int jn = min(PM_SC, ns - j0);
-                __syncthreads();  // the previous chunk is consumed
-                int gi = 0;
-                if (lane < jn) {
-                    const int q = j0 + lane;
-                    int m = 0;
-                    while (s_pre[m + 1] <= q) m++;
-                    gi = s_start[m] + q - s_pre[m];
-                    sx[lane] = a.x[gi];
-                    sy[lane] = a.y[gi];
-                    sz[lane] = a.z[gi];
-                }
-#pragma unroll
-                for (int r = 0; r < PM_SC * 32 / 64; r++) {
-                    const int u = lane + 64 * r, j = u / 32, c = u % 32;
-                    const int gj = __shfl(gi, j);
-                    sw[j][c] = (j < jn && c < cn) ? a.wsT[(int64_t)gj * a.ncols + c0 + c] : 0.0;
-                }
-                __syncthreads();
-                for (int k0 = 0; k0 < jn; k0 += 4) {
-                    const int jj = k0 + fk;  // this lane's source of the 4-block (rows past jn carry zero weights)
-                    const int js = min(jj, jn - 1);
-                    const double px = sx[js], py = sy[js], pz = sz[js];
-                    const double w0 = sw[jj & (PM_SC - 1)][fr], w1 = sw[jj & (PM_SC - 1)][16 + fr];
-                    const double b0 = jj < jn ? w0 : 0.0, b1 = jj < jn ? w1 : 0.0;
-#pragma unroll
-                    for (int tb = 0; tb < TB; tb++) {
-                        double kv = KF32 ? keval_f32<KID>(px - tx[tb], py - ty[tb], pz - tz[tb], a.kp)
-                                         : keval<KID>(px - tx[tb], py - ty[tb], pz - tz[tb], a.kp);
-                        if (isinf(kv) || jj >= jn) kv = 0.0;  // (padding sources add nothing)
-                        acc[tb][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv, b0, acc[tb][0], 0, 0, 0);
-                        acc[tb][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(kv, b1, acc[tb][1], 0, 0, 0);
-                    }
-                }
-            }
-#pragma unroll
-            for (int tb = 0; tb < TB; tb++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int ti = i0 + tb * 16 + fk + 4 * v;
-                    if (ti >= nt) continue;
-                    const int64_t oi = a.perm[t0 + ti] - a.out_lo;
-                    if ((uint64_t)oi >= (uint64_t)a.out_n) continue;
-#pragma unroll
-                    for (int cb = 0; cb < 2; cb++) {
-                        const int col = cb * 16 + fr;
-                        if (col < cn) a.out[(int64_t)(c0 + col) * a.out_n + oi] += acc[tb][cb][v];
-                    }
-                }
-        }
+    __shared__ double lds[P2P_SC * (P2P_WS + 3)];
+    __shared__ P2PRange r;
+    int c, pass;
+    const int b = p2p_leaf(a, P2P_DENSE, NEAR_CLASSES - 1, blockIdx.x, c, pass);
+    const int t0 = a.leaf_start[b], nt = a.leaf_start[b + 1] - t0, c0 = blockIdx.y * P2P_NC;
+    if (pass * 64 >= nt) return;
+    p2p_range(a, b, r);
+    // 32 targets where no more are left, 16 columns where no more are
+    const bool half = a.ncols - c0 <= 16;
+    if (nt - pass * 64 <= 32) {
+        if (half) p2p_dense<KID, 2, 1, KF32>(a, r, lds, t0, nt, pass * 64, c0);
+        else p2p_dense<KID, 2, 2, KF32>(a, r, lds, t0, nt, pass * 64, c0);
+    } else {
+        if (half) p2p_dense<KID, 4, 1, KF32>(a, r, lds, t0, nt, pass * 64, c0);
+        else p2p_dense<KID, 4, 2, KF32>(a, r, lds, t0, nt, pass * 64, c0);
     }
 }
 
@@ -1404,11 +1518,11 @@ __device__ __forceinline__ void kgrad(double dx, double dy, double dz, const KPa
         gx = gy = gz = 0.0;
         return;
     }
-    if constexpr (KID == PBB_KERNEL_LAPLACIAN) { double ri = 1.0 / sqrt(r2); s = ri * ri * ri; }
+    if constexpr (KID == PBB_KERNEL_LAPLACIAN) { double ri = rsqrt_step(r2); s = ri * ri * ri; }
     else if constexpr (KID == PBB_KERNEL_ONEOVERR2) { s = 2.0 / (r2 * r2); }
     else if constexpr (KID == PBB_KERNEL_GAUSSIAN) { double a2 = p.p[0] * p.p[0]; s = 2.0 / a2 * exp(-r2 / a2); }
     else if constexpr (KID == PBB_KERNEL_EXPONENTIAL) { double r = sqrt(r2); s = p.p[1] * exp(-r / p.p[0]) / (p.p[0] * r); }
-    else if constexpr (KID == PBB_KERNEL_SOFT_LAPLACIAN) { double q = 1.0 / sqrt(r2 + p.p[0]); s = q * q * q; }
+    else if constexpr (KID == PBB_KERNEL_SOFT_LAPLACIAN) { double q = rsqrt_step(r2 + p.p[0]); s = q * q * q; }
     else if constexpr (KID == PBB_KERNEL_QUADRIC || KID == PBB_KERNEL_R2) { s = -2.0; }
     else if constexpr (KID == PBB_KERNEL_INV_QUADRIC) { double q = 1.0 / (1.0 + r2); s = 2.0 * q * q; }
     else if constexpr (KID == PBB_KERNEL_LOGARITHM) { s = -1.0 / r2; }
@@ -1807,41 +1921,41 @@ void launch_near(const NearArgs &a, int kid, int nleaf, hipStream_t st)
     check(hipGetLastError(), "near_fp64");
 }
 
-bool launch_near_split(const NearArgs &a, int kid, int nleaf, hipStream_t st)
+bool launch_near_split(const NearArgs &args, int kid, int nleaf, hipStream_t st)
 {
+    NearArgs a = args;
     if (a.n < 4 || a.n > 8) return false;
     if (nleaf <= 0) return true;
-    const NearArgs &b = a;
-    for (int c = 0; c < NEAR_CLASSES; c++) {
-        const int cnt = a.leaf_class_off[c + 1] - a.leaf_class_off[c];
-        if (cnt <= 0) continue;
-        const int32_t *lst = a.leaf_class + a.leaf_class_off[c];
-#define PBB_P2P_TT(K, T)                                                    \
-    case T:                                                                 \
-        if constexpr (T >= 32) {                                            \
-            if (a.kf32) p2p_mfma<K, T / 16, true><<<cnt, 64, 0, st>>>(b, lst);  \
-            else p2p_mfma<K, T / 16, false><<<cnt, 64, 0, st>>>(b, lst);        \
-        } else {                                                            \
-            p2p_fp64<K, T><<<cnt, 64, 0, st>>>(b, lst);                     \
-        }                                                                   \
+    const int last = NEAR_CLASSES - 1, big = a.leaf_class_off[last + 1] - a.leaf_class_off[last];
+    a.passes = big > 0 ? (a.max_leaf + 63) / 64 : 0;
+    const int few = a.leaf_class_off[P2P_DENSE];
+    const int64_t dense = (int64_t)big * a.passes + a.leaf_class_off[last] - few;
+    if (dense + few > INT32_MAX) fail(PBB_ERR_UNSUPPORTED, "too many near-field passes");
+    const unsigned cols = (unsigned)((a.ncols + P2P_NC - 1) / P2P_NC);
+    // (the whole call's columns choose, so that a chunk of them sums in the same order)
+    const dim3 all((unsigned)(dense + few)), gs((unsigned)few, cols), gd((unsigned)dense, cols);
+#define PBB_P2P_CASE(K)                                                        \
+    case K:                                                                    \
+        if (a.all <= 8 && a.ncols <= 1) p2p_few_columns<K, 1><<<all, 64, 0, st>>>(a); \
+        else if (a.all <= 8 && a.ncols <= 2) p2p_few_columns<K, 2><<<all, 64, 0, st>>>(a); \
+        else if (a.all <= 8 && a.ncols <= 4) p2p_few_columns<K, 4><<<all, 64, 0, st>>>(a); \
+        else if (a.all <= 8) p2p_few_columns<K, 8><<<all, 64, 0, st>>>(a);     \
+        else {                                                                 \
+            if (dense && a.kf32) p2p_dense_leaves<K, true><<<gd, 64, 0, st>>>(a); \
+            else if (dense) p2p_dense_leaves<K, false><<<gd, 64, 0, st>>>(a);  \
+            if (few) p2p_small_leaves<K><<<gs, 64, 0, st>>>(a);                \
+        }                                                                      \
         break;
-#define PBB_P2P_CASE(K)                                                     \
-    case K:                                                                 \
-        switch (2 << c) { PBB_P2P_TT(K, 2) PBB_P2P_TT(K, 4) PBB_P2P_TT(K, 8) \
-                          PBB_P2P_TT(K, 16) PBB_P2P_TT(K, 32) PBB_P2P_TT(K, 64) } \
-        break;
-        switch (kid) {
-            PBB_P2P_CASE(PBB_KERNEL_LAPLACIAN) PBB_P2P_CASE(PBB_KERNEL_ONEOVERR2) PBB_P2P_CASE(PBB_KERNEL_GAUSSIAN)
-            PBB_P2P_CASE(PBB_KERNEL_EXPONENTIAL) PBB_P2P_CASE(PBB_KERNEL_SOFT_LAPLACIAN)
-            PBB_P2P_CASE(PBB_KERNEL_QUADRIC) PBB_P2P_CASE(PBB_KERNEL_INV_QUADRIC)
-            PBB_P2P_CASE(PBB_KERNEL_LOGARITHM) PBB_P2P_CASE(PBB_KERNEL_THIN_PLATE) PBB_P2P_CASE(PBB_KERNEL_R2)
-            PBB_P2P_CASE(PBB_KERNEL_CONSTANT) PBB_P2P_CASE(PBB_KERNEL_EXP_ANISO)
-        default: fail(PBB_ERR_UNSUPPORTED, "no device functor for this kernel id");
-        }
-#undef PBB_P2P_CASE
-#undef PBB_P2P_TT
+    switch (kid) {
+        PBB_P2P_CASE(PBB_KERNEL_LAPLACIAN) PBB_P2P_CASE(PBB_KERNEL_ONEOVERR2) PBB_P2P_CASE(PBB_KERNEL_GAUSSIAN)
+        PBB_P2P_CASE(PBB_KERNEL_EXPONENTIAL) PBB_P2P_CASE(PBB_KERNEL_SOFT_LAPLACIAN)
+        PBB_P2P_CASE(PBB_KERNEL_QUADRIC) PBB_P2P_CASE(PBB_KERNEL_INV_QUADRIC)
+        PBB_P2P_CASE(PBB_KERNEL_LOGARITHM) PBB_P2P_CASE(PBB_KERNEL_THIN_PLATE) PBB_P2P_CASE(PBB_KERNEL_R2)
+        PBB_P2P_CASE(PBB_KERNEL_CONSTANT) PBB_P2P_CASE(PBB_KERNEL_EXP_ANISO)
+    default: fail(PBB_ERR_UNSUPPORTED, "no device functor for this kernel id");
     }
-    check(hipGetLastError(), "p2p_fp64");
+#undef PBB_P2P_CASE
+    check(hipGetLastError(), "p2p");
     return true;
 }
 

@@ -250,6 +250,8 @@ struct NearArgs {
     const int32_t *leaf_class;
     int leaf_class_off[NEAR_CLASSES + 1];
     int kf32;                   // dense leaves: kernel values in FP32 (mixed modes)
+    int all;                    // columns of the whole call (of which ncols run now)
+    int max_leaf, passes;       // points of the largest leaf; passes over the last class (the launcher's)
 };
 
 struct DirectArgs {

@@ -33,7 +33,7 @@ def _want(f, t, s, w):
 @pytest.mark.parametrize("name", list(KERNELS))
 @pytest.mark.parametrize("nt,ns,ncols", [(1, 1, 1), (63, 15, 2), (64, 16, 4), (65, 17, 5), (3, 1023, 16),
                                          (130, 1024, 17), (200, 1537, 33), (700, 5000, 3)])
-def test_against_numpy(name, nt, ns, ncols):
+def test_against_numpy(gpu, name, nt, ns, ncols):
     kernel, f = KERNELS[name]
     rng = np.random.default_rng(nt + ns)
     t, s, w = rng.random((nt, 3)), rng.random((ns, 3)), rng.standard_normal((ncols, ns))
@@ -45,7 +45,7 @@ def test_against_numpy(name, nt, ns, ncols):
 
 @pytest.mark.parametrize("r", [0.0, 1e-158, 1e-150, 1e-100, 1e-20, 1.0, 1e20, 1e100, 1e150, 1e160, np.inf, np.nan])
 @pytest.mark.parametrize("name", ["lap", "soft"])
-def test_range_of_the_inverse_root(name, r):
+def test_range_of_the_inverse_root(gpu, name, r):
     """One pair on an axis over the range of FP64, down to squares below the
     normal numbers (4 units in the last place)."""
     kernel, f = KERNELS[name]
