@@ -2616,21 +2616,26 @@ PBB_API pbb_status pbb_plan_grad_positions(pbb_plan *plan, const double *sigma_d
         if (Lv >= 2)
             check(hipMemcpyAsync(p->gF, W.S + (size_t)LL.off * ncols * n3, leafF * sizeof(double),
                                  hipMemcpyDeviceToDevice, st), "save leaf expansions");
-        check(hipMemcpyAsync(p->gU, W.ws, (size_t)p->N * ncols * sizeof(double), hipMemcpyDeviceToDevice, st),
-              "save sorted weights");
+        const PointIo io = point_io(p, p->ops);
+        dev::launch_gather_weights_t(sigma_dev, p->perm, p->N, ncols, p->gU, io.in_lo, io.in_n, st);
         // transposed FMM with psi: its leaf expansions and sorted psi
         matvec_own(p, adj, psi_dev, ncols, nullptr, st, precision);
+        dev::launch_gather_weights_t(psi_dev, p->perm, p->N, ncols, W.wsT, io.in_lo, io.in_n, st);
         dev::NearGradArgs a{};
         a.n = h.n; a.ncols = ncols; a.side = 1 << Lv; a.N = p->N; a.len = LL.len;
         std::memcpy(a.kp.p, h.kernel.param, sizeof(a.kp.p));
         a.leaf_start = p->leaf_start; a.coord = LL.coord; a.map = LL.map; a.perm = p->perm;
         a.ctab = LL.ctab; a.Tkz = p->ops->d_Tkz; a.x = p->x; a.y = p->y; a.z = p->z;
+        a.leaf_class = p->leaf_class;
+        std::copy(std::begin(p->leaf_class_off), std::end(p->leaf_class_off), a.leaf_class_off);
+        a.max_leaf = (int)p->info.max_leaf_points;
         a.grad = grad_dev;
-        // target side: d/dx_i of (A sigma)_i weighted by psi_i
-        a.v = W.ws; a.u = p->gU; a.F = Lv >= 2 ? p->gF : nullptr;
-        dev::launch_near_grad(a, h.kernel.id, (int)LL.nb, st);
-        // source side: d/dx_j of (A^T psi)_j weighted by sigma_j
-        a.v = p->gU; a.u = W.ws; a.F = Lv >= 2 ? W.S + (size_t)LL.off * ncols * n3 : nullptr;
+        a.sig = p->gU;
+        a.psi = W.wsT;
+        if (Lv >= 2) {
+            a.Fs = p->gF;
+            a.Fp = W.S + (size_t)LL.off * ncols * n3;
+        }
         dev::launch_near_grad(a, h.kernel.id, (int)LL.nb, st);
     });
 }

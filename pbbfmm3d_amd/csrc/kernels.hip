@@ -1145,7 +1145,8 @@ struct P2PRange {
 };
 
 // The leaf's neighbours: first points and, added up, their counts (wave scan)
-__device__ __forceinline__ void p2p_range(const NearArgs &a, int b, P2PRange &r)
+template <class Args>
+__device__ __forceinline__ void p2p_range(const Args &a, int b, P2PRange &r)
 {
     const int lane = threadIdx.x;
     const uint32_t cc = (uint32_t)a.coord[b];
@@ -1425,7 +1426,8 @@ __device__ __forceinline__ void p2p_dense(const NearArgs &a, const P2PRange &r, 
 // Workgroup w of a launch over the classes lo..hi: its leaf class (the largest
 // leaves first, then class by class), leaf and pass of 64 targets (the last
 // class only)
-__device__ __forceinline__ int p2p_leaf(const NearArgs &a, int lo, int hi, int w, int &c, int &pass)
+template <class Args>
+__device__ __forceinline__ int p2p_leaf(const Args &a, int lo, int hi, int w, int &c, int &pass)
 {
     c = hi;
     pass = 0;
@@ -1503,212 +1505,295 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void p2
 //   g_i += sum_c v_ic [ sum_l F_c[l] grad S_l(x_i) + sum_{j near} grad_1 K(x_i, x_j) u_jc ]
 // where grad S_l is the derivative of the tensor-product Chebyshev
 // interpolant (S_m'(u) = (2/n) sum_k T_k(x_m) k U_{k-1}(u), times 2/len) and
-// grad_1 K the kernel's gradient in its first (target) argument.  Called
-// with (v, F, u) = (dL/dout, forward leaf expansions, weights) for the
-// target side and (weights, transposed-FMM leaf expansions, dL/dout) for the
-// source side (symmetric kernels: d/dy K(x, y) = grad_1 K(y, x)).
+// grad_1 K the kernel's gradient in its first (target) argument, summed over
+// (v, F, u) = (psi, forward leaf expansions Fs, sigma), the target side, and
+// (sigma, transposed-FMM leaf expansions Fp, psi), the source side (symmetric
+// kernels: d/dy K(x, y) = grad_1 K(y, x)); sigma the weights, psi dL/dout.
+// d = source - target: the gradient with respect to the target position is
+// kgrad * d (on the axes scaled by kgrad_axis)
 template <int KID>
-__device__ __forceinline__ void kgrad(double dx, double dy, double dz, const KParams &p, double &gx, double &gy,
-                                      double &gz)
+__device__ __forceinline__ double kgrad(double dx, double dy, double dz, const KParams &p)
 {
-    // d = source - target; returns grad wrt the target position
     const double r2 = dx * dx + dy * dy + dz * dz;
-    double s = 0.0;  // grad = s * d
-    if (r2 == 0.0) {
-        gx = gy = gz = 0.0;
-        return;
+    double s = 0.0;
+    if constexpr (KID == PBB_KERNEL_LAPLACIAN) {
+        const double ri = rsqrt_inner(r2);
+        return __builtin_amdgcn_class(r2, 0x264) ? 0.0 : ri * ri * ri;  // (0, infinity)
     }
-    if constexpr (KID == PBB_KERNEL_LAPLACIAN) { double ri = rsqrt_step(r2); s = ri * ri * ri; }
     else if constexpr (KID == PBB_KERNEL_ONEOVERR2) { s = 2.0 / (r2 * r2); }
-    else if constexpr (KID == PBB_KERNEL_GAUSSIAN) { double a2 = p.p[0] * p.p[0]; s = 2.0 / a2 * exp(-r2 / a2); }
-    else if constexpr (KID == PBB_KERNEL_EXPONENTIAL) { double r = sqrt(r2); s = p.p[1] * exp(-r / p.p[0]) / (p.p[0] * r); }
-    else if constexpr (KID == PBB_KERNEL_SOFT_LAPLACIAN) { double q = rsqrt_step(r2 + p.p[0]); s = q * q * q; }
+    else if constexpr (KID == PBB_KERNEL_GAUSSIAN) { const double a2 = p.p[0] * p.p[0]; s = 2.0 / a2 * exp(-div_shared(r2, a2)); }
+    else if constexpr (KID == PBB_KERNEL_EXPONENTIAL) {
+        const double r = sqrt(r2);
+        s = p.p[1] * exp(-div_shared(r, p.p[0])) / (p.p[0] * r);
+    }
+    else if constexpr (KID == PBB_KERNEL_SOFT_LAPLACIAN) { const double q = rsqrt_step(r2 + p.p[0]); s = q * q * q; }
     else if constexpr (KID == PBB_KERNEL_QUADRIC || KID == PBB_KERNEL_R2) { s = -2.0; }
-    else if constexpr (KID == PBB_KERNEL_INV_QUADRIC) { double q = 1.0 / (1.0 + r2); s = 2.0 * q * q; }
+    else if constexpr (KID == PBB_KERNEL_INV_QUADRIC) { const double q = 1.0 / (1.0 + r2); s = 2.0 * q * q; }
     else if constexpr (KID == PBB_KERNEL_LOGARITHM) { s = -1.0 / r2; }
     else if constexpr (KID == PBB_KERNEL_THIN_PLATE) { s = -(log(r2) + 1.0); }
     else if constexpr (KID == PBB_KERNEL_EXP_ANISO) {
         const double rho = sqrt(p.p[1] * dx * dx + p.p[2] * dy * dy + p.p[3] * dz * dz);
-        const double f = rho > 0 ? p.p[0] * exp(-rho) / rho : 0.0;
-        gx = f * p.p[1] * dx; gy = f * p.p[2] * dy; gz = f * p.p[3] * dz;
-        return;
+        s = rho > 0 ? p.p[0] * exp(-rho) / rho : 0.0;
     }
-    gx = s * dx; gy = s * dy; gz = s * dz;
+    return r2 == 0.0 ? 0.0 : s;
 }
-
-// S_m(u) and S_m'(u), m < n
-__device__ __forceinline__ void sn_eval_d(int n, const double *__restrict__ Tkz, double u, double *S, double *dS)
-{
-    double T[16], dT[16];
-    T[0] = 1.0; dT[0] = 0.0;
-    if (n > 1) { T[1] = u; dT[1] = 1.0; }
-    double Um2 = 1.0, Um1 = 2.0 * u;  // U_0, U_1
-    for (int k = 2; k < n; k++) {
-        T[k] = 2.0 * u * T[k - 1] - T[k - 2];
-        dT[k] = k * Um1;  // T_k' = k U_{k-1}
-        const double Uk = 2.0 * u * Um1 - Um2;
-        Um2 = Um1;
-        Um1 = Uk;
-    }
-    const double pfac = 2.0 / n;
-    for (int m = 0; m < n; m++) {
-        const double *Tk = Tkz + m * n;
-        double s = 0.5 * Tk[0], d = 0.0;
-        for (int k = 1; k < n; k++) {
-            s += Tk[k] * T[k];
-            d += Tk[k] * dT[k];
-        }
-        S[m] = pfac * s;
-        dS[m] = pfac * d;
-    }
-}
-
 template <int KID>
-__global__ __launch_bounds__(64) void near_grad_fp64(NearGradArgs a)
+__device__ __forceinline__ double kgrad_axis(int axis, const KParams &p)
 {
-    __shared__ double sG[3][NV_TGT][NV_SRC + 1];
-    __shared__ double su[NV_COL][NV_SRC + 1];
-    __shared__ double sx[NV_SRC], sy[NV_SRC], sz[NV_SRC];
-    __shared__ double tx[NV_TGT], ty[NV_TGT], tz[NV_TGT];
-    __shared__ double red[3][64];
-    __shared__ double sS[6][16][NV_TGT];  // S_m and S_m' of each target coordinate
-    __shared__ int s_start[27], s_pre[28];
-    const int b = blockIdx.x, lane = threadIdx.x;
-    const int n = a.n, n2 = n * n, n3 = n2 * n;
+    return KID == PBB_KERNEL_EXP_ANISO ? p.p[1 + axis] : 1.0;
+}
+
+// The far part: one wave per leaf (or per pass over 64 targets of a large
+// one), the leaf's expansion coefficients l over the lanes.  The columns of
+// both sides are summed per coefficient first, t_l = sum_c psi_ic Fs_c[l] +
+// sigma_ic Fp_c[l], so the derivative terms run once per (target, l) instead
+// of once per column; rows of psi and sigma are the same for all lanes and
+// come through the scalar cache.  Bound by the reads of Fs and Fp, once per
+// block of FG_TGT targets.  Far and near part of both sides, before (one kernel
+// per side, every derivative term per column) and now: 500k uniform points,
+// soft 1/r, order 5, 4 columns 21.7 -> 1.43 ms (1.11 far: the leaves hold two
+// points each, so F is read once per two targets; 0.31 near); 60k clustered
+// points, Gaussian, order 6, 16 columns 16.8 -> 1.1 ms.
+constexpr int FG_TGT = 4;
+__global__ __launch_bounds__(64) void far_grad(NearGradArgs a)
+{
+    __shared__ double sS[2][3][16][FG_TGT];  // S_m, S_m' of each target coordinate
+    const int lane = threadIdx.x, n = a.n, n3 = n * n * n, C = a.ncols;
+    int c, pass;
+    const int b = p2p_leaf(a, 0, NEAR_CLASSES - 1, blockIdx.x, c, pass);
     const int t0 = a.leaf_start[b], nt = a.leaf_start[b + 1] - t0;
     const uint32_t cc = (uint32_t)a.coord[b];
-    const int ix = cc & 1023, iy = (cc >> 10) & 1023, iz = (cc >> 20) & 1023;
-    const int S = a.side;
-    const double cen[3] = {a.ctab[ix], a.ctab[iy], a.ctab[iz]};
+    const double cen[3] = {a.ctab[cc & 1023], a.ctab[(cc >> 10) & 1023], a.ctab[(cc >> 20) & 1023]};
     const double ihalfL = 2.0 / a.len;
-    if (lane < 27) {
-        int x = ix + lane / 9 - 1, y = iy + (lane / 3) % 3 - 1, z = iz + lane % 3 - 1;
-        int sb = (x >= 0 && y >= 0 && z >= 0 && x < S && y < S && z < S) ? a.map[((int64_t)x * S + y) * S + z] : -1;
-        s_start[lane] = sb >= 0 ? a.leaf_start[sb] : 0;
-        s_pre[lane + 1] = sb >= 0 ? a.leaf_start[sb + 1] - a.leaf_start[sb] : 0;
+    const double *__restrict__ Fs = a.Fs + (size_t)b * C * n3, *__restrict__ Fp = a.Fp + (size_t)b * C * n3;
+    const int end = min(nt, pass * 64 + 64);
+    for (int i0 = pass * 64; i0 < end; i0 += FG_TGT) {
+        const int tn = min(FG_TGT, end - i0);
+        __syncthreads();
+        for (int q = lane; q < tn * 3 * n; q += 64) {
+            const int m = q % n, ax = q / n % 3, ti = q / (3 * n);
+            const double *pos = ax == 0 ? a.x : ax == 1 ? a.y : a.z;
+            const double u = ihalfL * (pos[t0 + i0 + ti] - (ax == 0 ? cen[0] : ax == 1 ? cen[1] : cen[2]));
+            const double *Tk = a.Tkz + m * n;
+            // T_k, U_{k-1} by their recurrences; T_k' = k U_{k-1}
+            double tp = 1.0, tc = u, up = 0.0, uc = 1.0, s = 0.5 * Tk[0], d = 0.0;
+            for (int k = 1; k < n; k++) {
+                s += Tk[k] * tc;
+                d += Tk[k] * (k * uc);
+                const double tn2 = 2.0 * u * tc - tp, un = 2.0 * u * uc - up;
+                tp = tc; tc = tn2;
+                up = uc; uc = un;
+            }
+            sS[0][ax][m][ti] = 2.0 / n * s;
+            sS[1][ax][m][ti] = 2.0 / n * d;
+        }
+        __syncthreads();
+        double g[FG_TGT][3];
+#pragma unroll
+        for (int k = 0; k < FG_TGT; k++) g[k][0] = g[k][1] = g[k][2] = 0;
+        // (scalar rows; targets past the leaf repeat its last one and are not stored)
+        const double *__restrict__ ps[FG_TGT], *__restrict__ sg[FG_TGT];
+#pragma unroll
+        for (int k = 0; k < FG_TGT; k++) {
+            const int64_t r = (int64_t)(t0 + i0 + min(k, tn - 1)) * C;
+            ps[k] = a.psi + r;
+            sg[k] = a.sig + r;
+        }
+        for (int l0 = 0; l0 < n3; l0 += 64) {
+            const int l = min(l0 + lane, n3 - 1);
+            double t[FG_TGT];
+#pragma unroll
+            for (int k = 0; k < FG_TGT; k++) t[k] = 0;
+#pragma unroll 4
+            for (int q = 0; q < C; q++) {
+                const double fs = Fs[(size_t)q * n3 + l], fp = Fp[(size_t)q * n3 + l];
+#pragma unroll
+                for (int k = 0; k < FG_TGT; k++) t[k] += ps[k][q] * fs + sg[k][q] * fp;
+            }
+            const int l1 = l / (n * n), l2 = l / n % n, l3 = l % n;
+#pragma unroll
+            for (int k = 0; k < FG_TGT; k++) {
+                const double tk = l0 + lane < n3 ? t[k] : 0.0;
+                const double sx = sS[0][0][l1][k], sy = sS[0][1][l2][k], sz = sS[0][2][l3][k];
+                g[k][0] += tk * sS[1][0][l1][k] * (sy * sz);
+                g[k][1] += tk * sS[1][1][l2][k] * (sx * sz);
+                g[k][2] += tk * sS[1][2][l3][k] * (sx * sy);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < FG_TGT; k++)
+#pragma unroll
+            for (int ax = 0; ax < 3; ax++)
+                for (int o = 1; o < 64; o <<= 1) g[k][ax] += __shfl_xor(g[k][ax], o);
+        double mine = 0;
+#pragma unroll
+        for (int k = 0; k < FG_TGT; k++)
+#pragma unroll
+            for (int ax = 0; ax < 3; ax++) mine = lane == 3 * k + ax ? g[k][ax] : mine;
+        if (lane < 3 * tn) a.grad[3 * (int64_t)a.perm[t0 + i0 + lane / 3] + lane % 3] += mine * ihalfL;
     }
-    __syncthreads();
-    if (lane == 0) {
-        s_pre[0] = 0;
-        for (int m = 0; m < 27; m++) s_pre[m + 1] += s_pre[m];
-    }
-    __syncthreads();
-    const int ns = s_pre[27];
-    for (int i0 = 0; i0 < nt; i0 += NV_TGT) {
-        const int tn = min(NV_TGT, nt - i0);
-        const int TT = tn <= 1 ? 1 : tn <= 2 ? 2 : tn <= 4 ? 4 : tn <= 8 ? 8 : 16;
-        const int G = 64 / TT;
-        const int i = lane / G, g = lane % G;
-        const bool active = i < tn;
-        __syncthreads();
-        if (lane < tn) {
-            tx[lane] = a.x[t0 + i0 + lane];
-            ty[lane] = a.y[t0 + i0 + lane];
-            tz[lane] = a.z[t0 + i0 + lane];
-        }
-        __syncthreads();
-        if (a.F != nullptr && lane < 3 * tn) {
-            const int ti = lane / 3, ax = lane % 3;
-            const double xv = ax == 0 ? tx[ti] : ax == 1 ? ty[ti] : tz[ti];
-            double Sv[16], dSv[16];
-            sn_eval_d(n, a.Tkz, ihalfL * (xv - cen[ax]), Sv, dSv);
-            for (int m = 0; m < n; m++) {
-                sS[ax][m][ti] = Sv[m];
-                sS[3 + ax][m][ti] = dSv[m];
-            }
-        }
-        __syncthreads();
-        double gx = 0, gy = 0, gz = 0;
-        for (int c0 = 0; c0 < a.ncols; c0 += NV_COL) {
-            const int cn = min(NV_COL, a.ncols - c0);
-            double vv[NV_COL / 4];
+}
+
+// The near part.  A pair's gradient carries the factor
+//   s_ij = sum_c psi_ic sigma_jc + sigma_ic psi_jc
+// of both sides, so one evaluation of the kernel's derivative serves them.
+// Small leaves (up to 16 targets): lane (i, g) takes every G-th source for
+// target i; the target's rows stay in registers, the sources' in LDS.
+template <int KID, int NC>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void near_grad_small(NearGradArgs a)
+{
+    constexpr int ST = 2 * NC + 1;  // (odd: the lanes' rows start in different banks)
+    __shared__ double sx[64], sy[64], sz[64], sw[64 * ST];
+    __shared__ P2PRange r;
+    const int lane = threadIdx.x, C = a.ncols;
+    int c, pass;
+    const int b = p2p_leaf(a, 0, P2P_DENSE - 1, blockIdx.x, c, pass);
+    const int t0 = a.leaf_start[b], nt = a.leaf_start[b + 1] - t0;
+    p2p_range(a, b, r);
+    const int lg = c + 1, G = 64 >> lg, i = lane >> (6 - lg), g = lane & (G - 1), ns = r.pre[27];
+    const bool active = i < nt;
+    const int64_t ti = t0 + (active ? i : 0);
+    const double tx = a.x[ti], ty = a.y[ti], tz = a.z[ti];
+    double gx = 0, gy = 0, gz = 0;
+    for (int c0 = 0; c0 < C; c0 += NC) {
+        double vp[NC], vs[NC];
 #pragma unroll
-            for (int k = 0; k < NV_COL / 4; k++) {
-                const int cl = g + G * k;
-                vv[k] = (active && cl < cn) ? a.v[(int64_t)(c0 + cl) * a.N + t0 + i0 + i] : 0.0;
-            }
-            if (a.F != nullptr && active) {
-                const double *Sx = &sS[0][0][i], *Sy = &sS[1][0][i], *Sz = &sS[2][0][i];
-                const double *dSx = &sS[3][0][i], *dSy = &sS[4][0][i], *dSz = &sS[5][0][i];
-                const double *Fb = a.F + ((size_t)b * a.ncols + c0) * n3;
-#pragma unroll
-                for (int k = 0; k < NV_COL / 4; k++) {
-                    const int cl = g + G * k;
-                    if (cl >= cn) break;
-                    const double *F = Fb + (size_t)cl * n3;
-                    double ax = 0, ay = 0, az = 0;
-                    int l = 0;
-                    for (int l1 = 0; l1 < n; l1++)
-                        for (int l2 = 0; l2 < n; l2++)
-                            for (int l3 = 0; l3 < n; l3++) {
-                                const double f = F[l++];
-                                const int o1 = l1 * NV_TGT, o2 = l2 * NV_TGT, o3 = l3 * NV_TGT;
-                                ax += f * dSx[o1] * Sy[o2] * Sz[o3];
-                                ay += f * Sx[o1] * dSy[o2] * Sz[o3];
-                                az += f * Sx[o1] * Sy[o2] * dSz[o3];
-                            }
-                    gx += vv[k] * ax * ihalfL;
-                    gy += vv[k] * ay * ihalfL;
-                    gz += vv[k] * az * ihalfL;
-                }
-            }
-            for (int j0 = 0; j0 < ns; j0 += NV_SRC) {
-                const int jn = min(NV_SRC, ns - j0);
-                __syncthreads();
-                if (lane < jn) {
-                    const int q = j0 + lane;
-                    int m = 0;
-                    while (s_pre[m + 1] <= q) m++;
-                    const int gi = s_start[m] + q - s_pre[m];
-                    sx[lane] = a.x[gi];
-                    sy[lane] = a.y[gi];
-                    sz[lane] = a.z[gi];
-                    for (int c = 0; c < cn; c++) su[c][lane] = a.u[(int64_t)(c0 + c) * a.N + gi];
-                }
-                __syncthreads();
-                for (int q = lane; q < TT * NV_SRC; q += 64) {
-                    const int ii = q / NV_SRC, jj = q % NV_SRC;
-                    double kx = 0, ky = 0, kz = 0;
-                    if (ii < tn && jj < jn) kgrad<KID>(sx[jj] - tx[ii], sy[jj] - ty[ii], sz[jj] - tz[ii], a.kp, kx, ky, kz);
-                    sG[0][ii][jj] = kx;
-                    sG[1][ii][jj] = ky;
-                    sG[2][ii][jj] = kz;
-                }
-                __syncthreads();
-                if (active) {
-                    for (int jj = 0; jj < jn; jj++) {
-                        double w = 0;
-#pragma unroll
-                        for (int k = 0; k < NV_COL / 4; k++) {
-                            const int cl = g + G * k;
-                            if (cl < cn) w += vv[k] * su[cl][jj];
-                        }
-                        gx += w * sG[0][i][jj];
-                        gy += w * sG[1][i][jj];
-                        gz += w * sG[2][i][jj];
-                    }
-                }
-            }
+        for (int k = 0; k < NC; k++) {
+            vp[k] = c0 + k < C ? a.psi[ti * C + c0 + k] : 0.0;
+            vs[k] = c0 + k < C ? a.sig[ti * C + c0 + k] : 0.0;
         }
-        // reduce the G lanes of each target
-        __syncthreads();
-        red[0][lane] = gx;
-        red[1][lane] = gy;
-        red[2][lane] = gz;
-        __syncthreads();
-        if (lane < tn) {
-            double sxg = 0, syg = 0, szg = 0;
-            for (int q = 0; q < G; q++) {
-                sxg += red[0][lane * G + q];
-                syg += red[1][lane * G + q];
-                szg += red[2][lane * G + q];
+        int m = 0;
+        for (int j0 = 0; j0 < ns; j0 += 64) {
+            const int jn = min(64, ns - j0);
+            __syncthreads();  // the previous chunk is consumed
+            if (lane < jn) {
+                const int64_t gi = p2p_point(r, j0 + lane, m);
+                sx[lane] = a.x[gi];
+                sy[lane] = a.y[gi];
+                sz[lane] = a.z[gi];
+#pragma unroll
+                for (int k = 0; k < NC; k++) {
+                    sw[lane * ST + k] = c0 + k < C ? a.sig[gi * C + c0 + k] : 0.0;
+                    sw[lane * ST + NC + k] = c0 + k < C ? a.psi[gi * C + c0 + k] : 0.0;
+                }
             }
-            const int64_t oi = a.perm[t0 + i0 + lane];
-            a.grad[3 * oi] += sxg;
-            a.grad[3 * oi + 1] += syg;
-            a.grad[3 * oi + 2] += szg;
+            __syncthreads();
+            for (int j = g; j < jn; j += G) {
+                double s = 0;
+#pragma unroll
+                for (int k = 0; k < NC; k++) s += vp[k] * sw[j * ST + k] + vs[k] * sw[j * ST + NC + k];
+                const double dx = sx[j] - tx, dy = sy[j] - ty, dz = sz[j] - tz;
+                s *= kgrad<KID>(dx, dy, dz, a.kp);
+                gx += s * dx;
+                gy += s * dy;
+                gz += s * dz;
+            }
         }
     }
+    for (int o = 1; o < G; o <<= 1) {
+        gx += __shfl_xor(gx, o);
+        gy += __shfl_xor(gy, o);
+        gz += __shfl_xor(gz, o);
+    }
+    if (active && g == 0) {
+        const int64_t oi = a.perm[ti];
+        a.grad[3 * oi] += gx * kgrad_axis<KID>(0, a.kp);
+        a.grad[3 * oi + 1] += gy * kgrad_axis<KID>(1, a.kp);
+        a.grad[3 * oi + 2] += gz * kgrad_axis<KID>(2, a.kp);
+    }
+}
+
+// Larger leaves: s is the product of the targets' rows (psi, sigma) with the
+// sources' (sigma, psi), 2 NC long, which v_mfma_f64_16x16x4f64 forms for 16
+// targets x 16 sources at a time; a lane then evaluates the derivative for
+// its 4 pairs of a block and keeps 4 targets' sums.  The k of a fragment are
+// assigned so that a lane reads NC / 2 values of one row in a piece.
+template <int KID, int NC, int TB>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void near_grad_dense(NearGradArgs a)
+{
+    constexpr int KF = NC / 2;  // k per lane = fragments
+    __shared__ P2PRange r;
+    const int lane = threadIdx.x, fr = lane & 15, fk = lane >> 4, C = a.ncols;
+    int c, pass;
+    const int b = p2p_leaf(a, P2P_DENSE, NEAR_CLASSES - 1, blockIdx.x, c, pass);
+    const int t0 = a.leaf_start[b], nt = a.leaf_start[b + 1] - t0, i0 = pass * 64 + blockIdx.y * 16 * TB;
+    if (i0 >= nt) return;
+    p2p_range(a, b, r);
+    const int ns = r.pre[27];
+    const double *__restrict__ va = fk < 2 ? a.psi : a.sig, *__restrict__ vb = fk < 2 ? a.sig : a.psi;
+    const int ck = (fk & 1) * KF;  // this lane's first column of the chunk
+    double tx[TB][4], ty[TB][4], tz[TB][4], gx[TB][4], gy[TB][4], gz[TB][4];
+#pragma unroll
+    for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int64_t ti = t0 + min(i0 + tb * 16 + fk + 4 * v, nt - 1);
+            tx[tb][v] = a.x[ti];
+            ty[tb][v] = a.y[ti];
+            tz[tb][v] = a.z[ti];
+            gx[tb][v] = gy[tb][v] = gz[tb][v] = 0;
+        }
+    for (int c0 = 0; c0 < C; c0 += NC) {
+        double A[TB][KF];
+#pragma unroll
+        for (int tb = 0; tb < TB; tb++) {
+            const int64_t row = (int64_t)(t0 + min(i0 + tb * 16 + fr, nt - 1)) * C;
+#pragma unroll
+            for (int f = 0; f < KF; f++) A[tb][f] = c0 + ck + f < C ? va[row + c0 + ck + f] : 0.0;
+        }
+        int m = 0;
+        double px, py, pz, B[KF];
+        auto load = [&](int j0) {
+            const int j = min(j0 + fr, ns - 1);
+            const int64_t gi = p2p_point(r, j, m);
+            px = a.x[gi];
+            py = a.y[gi];
+            pz = a.z[gi];
+            const double *row = vb + gi * C + c0 + ck;
+#pragma unroll
+            for (int f = 0; f < KF; f++) B[f] = j0 + fr < ns && c0 + ck + f < C ? row[f] : 0.0;
+        };
+        load(0);
+#pragma unroll 1
+        for (int j0 = 0; j0 < ns; j0 += 16) {
+            const double qx = px, qy = py, qz = pz;
+            dbl4 s[TB];
+#pragma unroll
+            for (int tb = 0; tb < TB; tb++) {
+                s[tb] = dbl4{0, 0, 0, 0};
+#pragma unroll
+                for (int f = 0; f < KF; f++) s[tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[tb][f], B[f], s[tb], 0, 0, 0);
+            }
+            load(j0 + 16);  // in flight during the derivatives
+#pragma unroll
+            for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const double dx = qx - tx[tb][v], dy = qy - ty[tb][v], dz = qz - tz[tb][v];
+                    const double w = s[tb][v] * kgrad<KID>(dx, dy, dz, a.kp);
+                    gx[tb][v] += w * dx;
+                    gy[tb][v] += w * dy;
+                    gz[tb][v] += w * dz;
+                }
+        }
+    }
+#pragma unroll
+    for (int tb = 0; tb < TB; tb++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            for (int o = 1; o < 16; o <<= 1) {
+                gx[tb][v] += __shfl_xor(gx[tb][v], o);
+                gy[tb][v] += __shfl_xor(gy[tb][v], o);
+                gz[tb][v] += __shfl_xor(gz[tb][v], o);
+            }
+            const int ti = i0 + tb * 16 + fk + 4 * v;
+            if (fr == 0 && ti < nt) {
+                const int64_t oi = a.perm[t0 + ti];
+                a.grad[3 * oi] += gx[tb][v] * kgrad_axis<KID>(0, a.kp);
+                a.grad[3 * oi + 1] += gy[tb][v] * kgrad_axis<KID>(1, a.kp);
+                a.grad[3 * oi + 2] += gz[tb][v] * kgrad_axis<KID>(2, a.kp);
+            }
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -2041,12 +2126,28 @@ void launch_direct(const DirectArgs &a, int kid, hipStream_t st)
     check(hipGetLastError(), "direct_reduce");
 }
 
-void launch_near_grad(const NearGradArgs &a, int kid, int nleaf, hipStream_t st)
+void launch_near_grad(const NearGradArgs &args, int kid, int nleaf, hipStream_t st)
 {
     if (nleaf <= 0) return;
-#define PBB_GRAD_CASE(K)                                  \
-    case K:                                               \
-        near_grad_fp64<K><<<nleaf, 64, 0, st>>>(a);       \
+    NearGradArgs a = args;
+    const int last = NEAR_CLASSES - 1, big = a.leaf_class_off[last + 1] - a.leaf_class_off[last];
+    a.passes = big > 0 ? (a.max_leaf + 63) / 64 : 0;
+    const int few = a.leaf_class_off[P2P_DENSE];
+    const int64_t dense = (int64_t)big * a.passes + a.leaf_class_off[last] - few;
+    if (dense + few > INT32_MAX) fail(PBB_ERR_UNSUPPORTED, "too many near-field passes");
+    const bool wide = a.ncols > 4;
+    if (a.Fs && dense + few) {
+        far_grad<<<(unsigned)(dense + few), 64, 0, st>>>(a);
+        check(hipGetLastError(), "far_grad");
+    }
+    // 16 x 2 targets at a time: the 64 targets of a pass in two workgroups
+    const dim3 gd((unsigned)dense, 2);
+#define PBB_GRAD_CASE(K)                                                          \
+    case K:                                                                       \
+        if (dense && wide) near_grad_dense<K, 16, 2><<<gd, 64, 0, st>>>(a);       \
+        else if (dense) near_grad_dense<K, 4, 2><<<gd, 64, 0, st>>>(a);           \
+        if (few && wide) near_grad_small<K, 16><<<few, 64, 0, st>>>(a);           \
+        else if (few) near_grad_small<K, 4><<<few, 64, 0, st>>>(a);               \
         break;
     switch (kid) {
         PBB_GRAD_CASE(PBB_KERNEL_LAPLACIAN) PBB_GRAD_CASE(PBB_KERNEL_ONEOVERR2) PBB_GRAD_CASE(PBB_KERNEL_GAUSSIAN)
@@ -2057,7 +2158,7 @@ void launch_near_grad(const NearGradArgs &a, int kid, int nleaf, hipStream_t st)
     default: fail(PBB_ERR_UNSUPPORTED, "no device functor for this kernel id");
     }
 #undef PBB_GRAD_CASE
-    check(hipGetLastError(), "near_grad_fp64");
+    check(hipGetLastError(), "near_grad");
 }
 
 // out[0..n) = 0, as a kernel so that it can sit in a captured graph

@@ -290,8 +290,11 @@ struct NearGradArgs {
     const int32_t *leaf_start, *coord, *map, *perm;
     const double *ctab, *Tkz;
     const double *x, *y, *z;
-    const double *u, *v;        // sorted source weights / target coefficients (column-major N)
-    const double *F;            // leaf expansions [leaf][col][n3] (nullptr: none)
+    const double *sig, *psi;    // the weights and dL/dout, sorted, point-major [N][ncols]
+    const double *Fs, *Fp;      // leaf expansions [leaf][col][n3] of sig (forward) and psi (transposed), or nullptr
+    const int32_t *leaf_class;  // as in NearArgs
+    int leaf_class_off[NEAR_CLASSES + 1];
+    int max_leaf, passes;
     double *grad;               // AoS N x 3, caller's order, accumulated
 };
 
