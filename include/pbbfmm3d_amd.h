@@ -352,6 +352,26 @@ PBB_API pbb_status pbb_plan_grad_positions(pbb_plan *plan, const double *sigma_d
                                            double *grad_dev, int32_t precision,
                                            void *stream);
 
+/* Both gradients of a training step from one transposed FMM pass: grad as
+ * pbb_plan_grad_positions, and wgrad += A~^T psi (nullptr: not wanted; else
+ * as pbb_plan_matvec_transpose).  kept_dev: what pbb_plan_matvec_keep of the
+ * same sigma, points and precision wrote, or NULL (the forward FMM is run
+ * again).  pbb_plan_matvec_keep is pbb_plan_matvec that also writes the leaf
+ * expansions, pbb_plan_kept_size doubles; that size is 0 where a forward had
+ * better not keep them (fewer than two levels, the mixed modes, plans without
+ * position gradients or with a workspace cap, not enough free device memory).
+ * No reference counterpart; used by the autograd function.                 */
+PBB_API pbb_status pbb_plan_kept_size(pbb_plan *plan, int32_t ncols, int32_t precision,
+                                      int64_t *count);
+PBB_API pbb_status pbb_plan_matvec_keep(pbb_plan *plan, const double *w_dev,
+                                        int32_t ncols, double *out_dev,
+                                        double *kept_dev, int32_t precision,
+                                        void *stream);
+PBB_API pbb_status pbb_plan_gradients(pbb_plan *plan, const double *sigma_dev,
+                                      const double *kept_dev, const double *psi_dev,
+                                      int32_t ncols, double *wgrad_dev, double *grad_dev,
+                                      int32_t precision, void *stream);
+
 /* Caps the plan's matvec workspace at `bytes` (0: what the device holds).
  * A matvec whose workspace for all its columns does not fit runs as
  * chunks of columns, each a complete FMM pass with the same sums (phase

@@ -125,6 +125,9 @@ _SIGNATURES = {
     "pbb_plan_matvec_noalloc": (C.c_int, [_vp, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     "pbb_plan_matvec_transpose": (C.c_int, [_vp, _vp, C.c_int32, _vp, C.c_int32, _vp]),
     "pbb_plan_grad_positions": (C.c_int, [_vp, _vp, _vp, C.c_int32, _vp, C.c_int32, _vp]),
+    "pbb_plan_kept_size": (C.c_int, [_vp, C.c_int32, C.c_int32, C.POINTER(C.c_int64)]),
+    "pbb_plan_matvec_keep": (C.c_int, [_vp, _vp, C.c_int32, _vp, _vp, C.c_int32, _vp]),
+    "pbb_plan_gradients": (C.c_int, [_vp, _vp, _vp, _vp, C.c_int32, _vp, _vp, C.c_int32, _vp]),
     "pbb_batch_create": (C.c_int, [C.POINTER(_vp), C.c_int32, C.POINTER(_vp), C.POINTER(_vp), C.c_int32,
                                    C.c_int32, C.c_int32, C.POINTER(_vp)]),
     "pbb_batch_create_entries": (C.c_int, [C.POINTER(BatchEntry), C.c_int32, C.c_int32, C.c_int32,

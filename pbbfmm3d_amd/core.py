@@ -403,6 +403,43 @@ class Plan:
             C.c_void_p(grad.data_ptr()), int(precision), C.c_void_p(stream)))
         return grad
 
+    def _matvec_keep(self, w, precision: int):
+        """(matvec(w), leaf expansions for _gradients), or (matvec(w), None)
+        where the gradient recomputes them (see pbb_plan_kept_size)."""
+        import torch
+        w, out, ncols = self._io(w, None)
+        count = C.c_int64()
+        capi.check(capi.lib().pbb_plan_kept_size(self._h, int(ncols), int(precision), C.byref(count)))
+        if not count.value:
+            return self.matvec(w, out, precision), None
+        kept = torch.empty(count.value, dtype=torch.float64, device=w.device)
+        stream = torch.cuda.current_stream(w.device).cuda_stream
+        capi.check(capi.lib().pbb_plan_matvec_keep(
+            self._h, C.c_void_p(w.data_ptr()), int(ncols), C.c_void_p(out.data_ptr()), C.c_void_p(kept.data_ptr()),
+            int(precision), C.c_void_p(stream)))
+        return out, kept
+
+    def _gradients(self, sigma, kept, psi, precision: int, weights: bool):
+        """(A~^T psi or None, dL/dx) for out = A~(x) sigma, psi = dL/dout and
+        the expansions kept by _matvec_keep(sigma) (None: recomputed)."""
+        import torch
+        sigma, wgrad, ncols = self._io(sigma, None)
+        psi = _f64_cuda(psi.contiguous(), "psi", shape=sigma.shape)
+        if psi.device != sigma.device:
+            raise ValueError("psi must be on sigma's device")
+        if kept is not None:
+            count = self.info()["boxes"][-1] * ncols * self.ops.order ** 3
+            _f64_cuda(kept, "kept", shape=(count,))
+            if kept.device != sigma.device:
+                raise ValueError("kept must be on sigma's device")
+        grad = torch.zeros((self.npoints, 3), dtype=torch.float64, device=sigma.device)
+        stream = torch.cuda.current_stream(sigma.device).cuda_stream
+        capi.check(capi.lib().pbb_plan_gradients(
+            self._h, C.c_void_p(sigma.data_ptr()), C.c_void_p(kept.data_ptr() if kept is not None else None),
+            C.c_void_p(psi.data_ptr()), int(ncols), C.c_void_p(wgrad.data_ptr() if weights else None),
+            C.c_void_p(grad.data_ptr()), int(precision), C.c_void_p(stream)))
+        return (wgrad if weights else None), grad
+
     def set_workspace_limit(self, nbytes: int):
         """Caps the matvec workspace (0: device memory); larger matvecs run
         in chunks of columns."""

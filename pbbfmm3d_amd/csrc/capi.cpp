@@ -713,7 +713,8 @@ struct pbb_plan {
     std::vector<uint32_t> h_leaf;
     std::vector<Level> h_geom;
     int32_t *pt_leaf = nullptr;  // device: leaf coordinates of every sorted point
-    int g_ncols = 0;
+    int g_ncols = 0;              // columns of gU
+    size_t gF_len = 0;            // doubles of gF
     bool timing = false;
     struct M2LTile {
         int width = 0, cpt = 0, flags = 0;  // width 0 = built-in choice
@@ -1793,15 +1794,16 @@ static PointIo point_io(const pbb_plan *p, const pbb_ops *o)
 }
 
 static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double *w, int ncols, double *out,
-                       hipStream_t st, int prec, bool build);
+                       hipStream_t st, int prec, bool build, bool keep = false);
 
 // One matvec of the plan's operator set o in its own workspace.
 // Columns are independent: when the workspace of all ncols columns does not
 // fit beside what the device already holds, the matvec runs over chunks of
 // columns, each a complete FMM pass (the same sums, so the same results).
-// A pass that keeps its expansions for the caller (out == nullptr) is not
-// split.
-static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, double *out, hipStream_t st, int prec)
+// A pass that keeps its expansions for the caller (keep: the complete leaf
+// expansions in W.S; out may be nullptr) is not split.
+static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, double *out, hipStream_t st, int prec,
+                       bool keep = false)
 {
     const bool mixed = prec != PBB_PREC_FP64;
     const PointIo io = point_io(p, o);
@@ -1818,7 +1820,7 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
             }
         }
     }
-    if (out) {
+    if (!keep) {
         Workspace tmp;
         size_t need = layout_workspace(*p, chunk, mixed, far_dims(*p, o, chunk, ncols, sym), nullptr, tmp);
         if (need > p->ws_bytes || (p->ws_limit && need > p->ws_limit)) {
@@ -1840,7 +1842,7 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
         const int cn = std::min(chunk, ncols - c0);
         p->ensure_workspace(cn, mixed, far_dims(*p, o, cn, ncols, sym));
         matvec_run(p, o, p->W, w + (size_t)c0 * io.in_n, cn, out ? out + (size_t)c0 * io.out_n : nullptr, st, prec,
-                   true);
+                   true, keep);
     }
 }
 
@@ -2066,7 +2068,7 @@ static void split_ops(const pbb_plan *p, pbb_ops *o, int prec, bool build, hipSt
 }
 
 static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double *w, int ncols, double *out,
-                       hipStream_t st, int prec, bool build)
+                       hipStream_t st, int prec, bool build, bool keep)
 {
     const bool mixed = prec != PBB_PREC_FP64;
     const HostOps &h = o->h;
@@ -2088,7 +2090,7 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
     // P2M + M2M, and (with a near field to add into) L2P at every level
     // instead of L2L + L2P; both are exact rewritings (see p2m_levels)
     const bool direct = n >= 4 && n <= 8;
-    const bool direct_down = direct && out != nullptr && Lv >= 2;
+    const bool direct_down = direct && out != nullptr && Lv >= 2 && !keep;
     // the mixed modes keep S / F in FP32 when the direct passes read them
     // (not with the FP64 VT / U of the cross-product-sum tile)
     const bool s32 = mixed && direct_down && !split_acc;
@@ -2121,13 +2123,11 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
     const bool hyb = direct_down && Lp <= Lv;
     const int Le = hyb ? Lp - 1 : Lv;
     const PointIo io = point_io(p, o);
-    // the direct passes and the split near field read only the point-major
-    // sorted weights wsT; W.ws (column-major sorted) serves the other paths
-    // and, on the direct path, holds the transposed input on the way to wsT
-    const bool ws_needed = !direct_down;  // (the split near field covers the direct orders 4..8)
-    if (ws_needed) dev::launch_gather_weights(w, p->perm, p->N, ncols, W.ws, io.in_lo, io.in_n, st);
-    if (direct && ws_needed) dev::launch_gather_weights_t(w, p->perm, p->N, ncols, W.wsT, io.in_lo, io.in_n, st);
-    else if (direct) dev::launch_gather_rows_t(w, p->perm, p->N, ncols, W.ws, W.wsT, io.in_lo, io.in_n, st);
+    // the direct upward pass and the split near field (orders 4..8) read only
+    // the point-major sorted weights wsT; W.ws (column-major sorted) serves the
+    // other orders and, on the way to wsT, holds the transposed input
+    if (!direct) dev::launch_gather_weights(w, p->perm, p->N, ncols, W.ws, io.in_lo, io.in_n, st);
+    else dev::launch_gather_rows_t(w, p->perm, p->N, ncols, W.ws, W.wsT, io.in_lo, io.in_n, st);
     const int cc_p2m = std::max(1, std::min({ncols, 64, 4096 / n3}));
     const int cc_m2m = std::max(1, std::min(ncols, 2048 / n3));
     if (Lv >= 2 && direct) {
@@ -2460,6 +2460,14 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
         a.child = p->lv[l - 1].child; a.Cw = o->d_Cw; a.Sparent = W.S; a.Schild = W.S;
         dev::launch_l2l(a, (int)p->lv[l - 1].nb, st);
     }
+    if (out && direct && keep && Lv >= 2) {  // the complete leaf expansions, once at every point
+        const DevLevel &D = p->lv[Lv];
+        dev::DownArgs a{};
+        a.n = n; a.ncols = ncols; a.off = D.off; a.len = D.len;
+        a.seg_box = D.seg_box; a.seg_p0 = D.seg_p0; a.pstart = D.pstart; a.coord = D.coord; a.ctab = D.ctab;
+        a.Tkz = o->d_Tkz; a.x = p->x; a.y = p->y; a.z = p->z; a.F = W.S; a.lp = W.lp;
+        dev::launch_l2p_level(a, D.nseg, st);
+    }
     mark(6);
     if (out) {
         const DevLevel &LL = p->lv[Lv];
@@ -2473,7 +2481,7 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
         a.out_lo = io.out_lo;
         a.out_n = io.out_n;
         a.wsT = W.wsT;
-        a.lp = direct_down ? W.lp : nullptr;
+        a.lp = direct && Lv >= 2 ? W.lp : nullptr;
         a.leaf_class = p->leaf_class;
         std::copy(std::begin(p->leaf_class_off), std::end(p->leaf_class_off), a.leaf_class_off);
         a.kf32 = mixed ? 1 : 0;
@@ -2582,61 +2590,141 @@ PBB_API pbb_status pbb_plan_matvec_transpose(pbb_plan *plan, const double *w_dev
     });
 }
 
+// Doubles of the leaf expansions of ncols columns that a forward keeps for
+// its gradient, or 0 where the gradient recomputes them: no far field, a plan
+// without position gradients, a mixed mode (its plain forward holds the
+// expansions in FP32 and takes the proxy passes, which a kept pass does not),
+// or device memory that would not leave the same room beside them.
+static int64_t kept_doubles(pbb_plan *p, int ncols, int prec)
+{
+    const HostOps &h = p->ops->h;
+    if (prec != PBB_PREC_FP64 || p->Lv < 2 || p->sep || h.kernel.symmetry != 1 || p->ws_limit) return 0;
+    const int64_t n = p->lv[p->Lv].nb * ncols * (int64_t)h.n3;
+    const bool sym = !p->ops->fp64_reduced;
+    if (sym) p->ops->ensure_sym((hipStream_t)0);
+    Workspace tmp;
+    const size_t need = layout_workspace(*p, ncols, false, far_dims(*p, p->ops, ncols, ncols, sym), nullptr, tmp);
+    size_t free_b = 0, total_b = 0;
+    check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    const size_t margin = std::max((size_t)(1ull << 30), total_b / 16);
+    const size_t grow = need > p->ws_bytes ? need - p->ws_bytes : 0;
+    return grow + (size_t)n * sizeof(double) + margin <= free_b ? n : 0;
+}
+
+PBB_API pbb_status pbb_plan_kept_size(pbb_plan *plan, int32_t ncols, int32_t precision, int64_t *count)
+{
+    return guarded([&] {
+        if (!plan || !count) fail(PBB_ERR_INVALID_ARG, "NULL argument");
+        if (ncols < 1) fail(PBB_ERR_INVALID_ARG, "ncols must be >= 1");
+        if (precision < PBB_PREC_FP64 || precision > PBB_PREC_MIXED_BF16X2)
+            fail(PBB_ERR_INVALID_ARG, "unknown precision mode");
+        DeviceGuard g(plan->device);
+        *count = kept_doubles(plan, ncols, precision);
+    });
+}
+
+PBB_API pbb_status pbb_plan_matvec_keep(pbb_plan *plan, const double *w_dev, int32_t ncols, double *out_dev,
+                                        double *kept_dev, int32_t precision, void *stream)
+{
+    return guarded([&] {
+        if (!plan || !w_dev || !out_dev || !kept_dev) fail(PBB_ERR_INVALID_ARG, "NULL argument");
+        if (ncols < 1) fail(PBB_ERR_INVALID_ARG, "ncols must be >= 1");
+        if (precision < PBB_PREC_FP64 || precision > PBB_PREC_MIXED_BF16X2)
+            fail(PBB_ERR_INVALID_ARG, "unknown precision mode");
+        if (plan->Lv < 2) fail(PBB_ERR_INVALID_ARG, "a plan of fewer than two levels has no leaf expansions");
+        DeviceGuard g(plan->device);
+        matvec_own(plan, plan->ops, w_dev, ncols, out_dev, (hipStream_t)stream, precision, true);
+        const DevLevel &LL = plan->lv[plan->Lv];
+        const size_t per = (size_t)ncols * plan->ops->h.n3;
+        check(hipMemcpyAsync(kept_dev, plan->W.S + (size_t)LL.off * per, LL.nb * per * sizeof(double),
+                             hipMemcpyDeviceToDevice, (hipStream_t)stream), "keep leaf expansions");
+    });
+}
+
+// Position gradients (grad_dev) from one transposed FMM pass on psi, which
+// also gives the weights' gradient (wgrad_dev, nullptr: not wanted), and the
+// forward pass's leaf expansions kept_dev (nullptr: that pass is run again).
+// A training step of FP64 matvecs so runs two far fields in place of four,
+// one of a mixed mode three: 500k points, 4 columns 157 -> 85 ms; 60k clustered points, 16 columns,
+// f16x2 27.5 -> 23.0 ms.
+static void gradients(pbb_plan *p, const double *sigma_dev, const double *kept_dev, const double *psi_dev, int ncols,
+                      double *wgrad_dev, double *grad_dev, int prec, hipStream_t st)
+{
+    if (ncols < 1) fail(PBB_ERR_INVALID_ARG, "ncols must be >= 1");
+    if (prec < PBB_PREC_FP64 || prec > PBB_PREC_MIXED_BF16X2) fail(PBB_ERR_INVALID_ARG, "unknown precision mode");
+    if (p->ops->h.kernel.symmetry != 1) fail(PBB_ERR_UNSUPPORTED, "position gradients need a symmetric kernel");
+    if (p->sep) fail(PBB_ERR_UNSUPPORTED, "position gradients need a plan whose sources are its targets");
+    pbb_ops *adj = p->ops->adjoint();
+    DeviceGuard g(p->device);
+    adj->upload(p->device);
+    const HostOps &h = p->ops->h;
+    const int Lv = p->Lv, n3 = h.n3;
+    const DevLevel &LL = p->lv[Lv];
+    const size_t leafF = (size_t)LL.nb * ncols * n3;
+    if (ncols > p->g_ncols) {
+        dfree(p->gU);
+        p->gU = nullptr;
+        p->g_ncols = 0;
+        p->gU = dalloc<double>((size_t)p->N * ncols, "sorted weights (gradient)");
+        p->g_ncols = ncols;
+    }
+    const double *Fs = kept_dev;
+    if (!Fs) {
+        if (Lv >= 2 && leafF > p->gF_len) {
+            dfree(p->gF);
+            p->gF = nullptr;
+            p->gF_len = 0;
+            p->gF = dalloc<double>(leafF, "saved leaf expansions");
+            p->gF_len = leafF;
+        }
+        // forward FMM with sigma: leaf expansions F
+        matvec_own(p, p->ops, sigma_dev, ncols, nullptr, st, prec, true);
+        if (Lv >= 2)
+            check(hipMemcpyAsync(p->gF, p->W.S + (size_t)LL.off * ncols * n3, leafF * sizeof(double),
+                                 hipMemcpyDeviceToDevice, st), "save leaf expansions");
+        Fs = p->gF;
+    }
+    const PointIo io = point_io(p, p->ops);
+    dev::launch_gather_weights_t(sigma_dev, p->perm, p->N, ncols, p->gU, io.in_lo, io.in_n, st);
+    // transposed FMM with psi: its leaf expansions and sorted psi
+    matvec_own(p, adj, psi_dev, ncols, wgrad_dev, st, prec, true);
+    const Workspace &W = p->W;
+    if (h.n < 4 || h.n > 8)  // (the direct orders' pass has sorted psi already)
+        dev::launch_gather_weights_t(psi_dev, p->perm, p->N, ncols, W.wsT, io.in_lo, io.in_n, st);
+    dev::NearGradArgs a{};
+    a.n = h.n; a.ncols = ncols; a.side = 1 << Lv; a.N = p->N; a.len = LL.len;
+    std::memcpy(a.kp.p, h.kernel.param, sizeof(a.kp.p));
+    a.leaf_start = p->leaf_start; a.coord = LL.coord; a.map = LL.map; a.perm = p->perm;
+    a.ctab = LL.ctab; a.Tkz = p->ops->d_Tkz; a.x = p->x; a.y = p->y; a.z = p->z;
+    a.leaf_class = p->leaf_class;
+    std::copy(std::begin(p->leaf_class_off), std::end(p->leaf_class_off), a.leaf_class_off);
+    a.max_leaf = (int)p->info.max_leaf_points;
+    a.grad = grad_dev;
+    a.sig = p->gU;
+    a.psi = W.wsT;
+    if (Lv >= 2) {
+        a.Fs = Fs;
+        a.Fp = W.S + (size_t)LL.off * ncols * n3;
+    }
+    dev::launch_near_grad(a, h.kernel.id, (int)LL.nb, st);
+}
+
 PBB_API pbb_status pbb_plan_grad_positions(pbb_plan *plan, const double *sigma_dev, const double *psi_dev,
                                            int32_t ncols, double *grad_dev, int32_t precision, void *stream)
 {
     return guarded([&] {
         if (!plan || !sigma_dev || !psi_dev || !grad_dev) fail(PBB_ERR_INVALID_ARG, "NULL argument");
-        if (ncols < 1) fail(PBB_ERR_INVALID_ARG, "ncols must be >= 1");
-        if (precision < PBB_PREC_FP64 || precision > PBB_PREC_MIXED_BF16X2)
-            fail(PBB_ERR_INVALID_ARG, "unknown precision mode");
-        if (plan->ops->h.kernel.symmetry != 1)
-            fail(PBB_ERR_UNSUPPORTED, "position gradients need a symmetric kernel");
-        if (plan->sep) fail(PBB_ERR_UNSUPPORTED, "position gradients need a plan whose sources are its targets");
-        pbb_ops *adj = plan->ops->adjoint();
-        DeviceGuard g(plan->device);
-        adj->upload(plan->device);
-        hipStream_t st = (hipStream_t)stream;
-        pbb_plan *p = plan;
-        const HostOps &h = p->ops->h;
-        const int Lv = p->Lv, n3 = h.n3;
-        const DevLevel &LL = p->lv[Lv];
-        if (ncols > p->g_ncols) {
-            dfree(p->gF); dfree(p->gU);
-            p->gF = p->gU = nullptr;
-            p->g_ncols = 0;
-            if (Lv >= 2) p->gF = dalloc<double>((size_t)LL.nb * ncols * n3, "saved leaf expansions");
-            p->gU = dalloc<double>((size_t)p->N * ncols, "sorted weights (gradient)");
-            p->g_ncols = ncols;
-        }
-        const size_t leafF = (size_t)LL.nb * ncols * n3;
-        // forward FMM with sigma: leaf expansions F and sorted sigma
-        matvec_own(p, p->ops, sigma_dev, ncols, nullptr, st, precision);
-        const Workspace &W = p->W;
-        if (Lv >= 2)
-            check(hipMemcpyAsync(p->gF, W.S + (size_t)LL.off * ncols * n3, leafF * sizeof(double),
-                                 hipMemcpyDeviceToDevice, st), "save leaf expansions");
-        const PointIo io = point_io(p, p->ops);
-        dev::launch_gather_weights_t(sigma_dev, p->perm, p->N, ncols, p->gU, io.in_lo, io.in_n, st);
-        // transposed FMM with psi: its leaf expansions and sorted psi
-        matvec_own(p, adj, psi_dev, ncols, nullptr, st, precision);
-        dev::launch_gather_weights_t(psi_dev, p->perm, p->N, ncols, W.wsT, io.in_lo, io.in_n, st);
-        dev::NearGradArgs a{};
-        a.n = h.n; a.ncols = ncols; a.side = 1 << Lv; a.N = p->N; a.len = LL.len;
-        std::memcpy(a.kp.p, h.kernel.param, sizeof(a.kp.p));
-        a.leaf_start = p->leaf_start; a.coord = LL.coord; a.map = LL.map; a.perm = p->perm;
-        a.ctab = LL.ctab; a.Tkz = p->ops->d_Tkz; a.x = p->x; a.y = p->y; a.z = p->z;
-        a.leaf_class = p->leaf_class;
-        std::copy(std::begin(p->leaf_class_off), std::end(p->leaf_class_off), a.leaf_class_off);
-        a.max_leaf = (int)p->info.max_leaf_points;
-        a.grad = grad_dev;
-        a.sig = p->gU;
-        a.psi = W.wsT;
-        if (Lv >= 2) {
-            a.Fs = p->gF;
-            a.Fp = W.S + (size_t)LL.off * ncols * n3;
-        }
-        dev::launch_near_grad(a, h.kernel.id, (int)LL.nb, st);
+        gradients(plan, sigma_dev, nullptr, psi_dev, ncols, nullptr, grad_dev, precision, (hipStream_t)stream);
+    });
+}
+
+PBB_API pbb_status pbb_plan_gradients(pbb_plan *plan, const double *sigma_dev, const double *kept_dev,
+                                      const double *psi_dev, int32_t ncols, double *wgrad_dev, double *grad_dev,
+                                      int32_t precision, void *stream)
+{
+    return guarded([&] {
+        if (!plan || !sigma_dev || !psi_dev || !grad_dev) fail(PBB_ERR_INVALID_ARG, "NULL argument");
+        gradients(plan, sigma_dev, kept_dev, psi_dev, ncols, wgrad_dev, grad_dev, precision, (hipStream_t)stream);
     });
 }
 
