@@ -2132,7 +2132,7 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
     const int cc_m2m = std::max(1, std::min(ncols, 2048 / n3));
     if (Lv >= 2 && direct) {
         dev::UpArgs a{};
-        a.n = n; a.ncols = ncols;
+        a.n = n; a.ncols = ncols; a.all = W.all;
         fill_levels(p, a.lt);
         a.items = p->up_items;
         a.Tkz = o->d_Tkz; a.x = p->x; a.y = p->y; a.z = p->z; a.wsT = W.wsT; a.S = W.S;
@@ -2144,6 +2144,9 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
         const int i0 = hyb ? (Le >= 2 ? p->lv[Le].up_item0 : i1) : 0;
         const int r0 = hyb ? (Le >= 2 ? p->lv[Le].up_red0 : r1) : 0;
         a.items = p->up_items + i0;
+        // the levels of more than 32 points a box, the coarse ones
+        for (int l = hyb ? Le : 2; l < Lp && l <= Lv && p->N > 32 * p->lv[l].nb; l++)
+            a.nbig = (l + 1 < Lp && l < Lv ? p->lv[l + 1].up_item0 : i1) - i0;
         dev::UpReduce r{};
         r.ncols = ncols; r.n3 = n3; r.reds = p->up_reds + r0; r.nred = r1 - r0;
         r.scratch = W.up; r.S = W.S; r.s32 = s32;

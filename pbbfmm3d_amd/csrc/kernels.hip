@@ -991,118 +991,157 @@ __global__ __launch_bounds__(256, 5) void l2p_f32(DownArgs a)
 // 234-333, :956-1034) equals P2M at every level straight from the points:
 // the child-to-parent transfer interpolates the parent's Chebyshev
 // polynomials S_m, which have degree n-1, at the child's nodes, which is
-// exact.  One workgroup per work item (a box of levels 2..L, or a segment of
-// P2M_SEG points of a larger box); thread pencils (column c, l1, l2) hold
-// the n values of l3 in registers.
-template <int N, typename TS>
-__global__ __launch_bounds__(256) void p2m_levels(UpArgs a)
+// exact.  A work item is a box of levels 2..L, or a segment of P2M_SEG points
+// of a larger box.
+// A box's expansion is the matrix product
+//   S[(l2, l3), (c, l1)] = sum_p [Sy_l2(p) Sz_l3(p)] [w_pc Sx_l1(p)],
+// n^2 rows and ncols n columns, column-major as S is stored, over its points:
+// on the FP64 matrix cores, 16 points to a table of S_m in LDS and 4 to a
+// step.  A wave holds all row blocks x CB column blocks (9 tiles at most),
+// further columns are other waves.  Columns for three waves and more: a
+// workgroup takes an item, its waves a column range each.  Fewer: the first
+// nbig items (those of the levels of many points a box) take a workgroup each,
+// the points dealt to its 4 waves and their sums added up in LDS; the others
+// go by fours, a wave to each, or one after another in the first way where one
+// of them is large.
+// Bound by the writes of S (one column: by the few waves of the coarse
+// levels).  Threads that held (column, l1, l2) pencils, barriers per box, and
+// now: 5k points, 1 column, order 4 21.6 -> 5.7 us; 78k points, 3 columns of
+// weights on 30k, order 5 568 -> 36 us; 1M points, 8 columns, order 5 3.04 ->
+// 1.26 ms; 1M clustered, 32 columns, order 6 6.40 -> 5.76 ms (FP32 expansions,
+// one level 1.38 -> 0.82 ms).
+template <int N, int CB, typename TS>
+__global__ __launch_bounds__(256, (N * N + 15) / 16 * CB > 6 ? 2 : 3) void p2m_levels(UpArgs a)
 {
-    constexpr int N2 = N * N, N3 = N2 * N, PTS = 64, PP = PTS + 1;
-    constexpr int CC = N <= 6 ? 32 : 16;        // columns per pass
-    constexpr int PR = (CC * N2 + 255) / 256;   // pencils per thread
-    // LDS: the point tables of a pass, then (FP32 expansions) the pass's
-    // expansion, staged so that it is stored with whole 16-byte writes
-    constexpr int U_SS = 3 * N * PP, U_SW = PTS * (CC + 1), U_SF = (CC * N3 + 1) / 2;
-    constexpr int U_ALL = U_SS + U_SW > U_SF ? U_SS + U_SW : U_SF;
-    __shared__ double smem[U_ALL];
-    double(*sS)[N][PP] = reinterpret_cast<double(*)[N][PP]>(smem);
-    double(*sw)[CC + 1] = reinterpret_cast<double(*)[CC + 1]>(smem + U_SS);
-    float *sF = reinterpret_cast<float *>(smem);
-    const int tid = threadIdx.x;
-    const int4 it = a.items[blockIdx.x];
-    const int li = it.x, b = it.y, p0 = it.z;
-    const int p1 = min(p0 + P2M_SEG, a.lt.pstart[li][b + 1]);
-    const uint32_t cc = (uint32_t)a.lt.coord[li][b];
-    const double *ctab = a.lt.ctab[li];
-    const double cen[3] = {ctab[cc & 1023], ctab[(cc >> 10) & 1023], ctab[(cc >> 20) & 1023]};
-    const double ihalfL = 2.0 / a.lt.len[li];
-    // split boxes write FP64 partial sums to scratch slots, others S directly
-    double *Sp = it.w >= 0 ? a.scratch + (size_t)it.w * a.ncols * N3 : nullptr;
-    TS *Sb = it.w >= 0 ? nullptr : (TS *)a.S + (size_t)(a.lt.off[li] + b) * a.ncols * N3;
-    for (int c0 = 0; c0 < a.ncols; c0 += CC) {
-        const int cn = min(CC, a.ncols - c0);
-        double acc[PR][N];
+    constexpr int N2 = N * N, N3 = N2 * N, RB = (N2 + 15) / 16, TP = (3 * N) | 1;
+    constexpr int SMALL = 32;  // points up to which an item is one wave's
+    constexpr int U_T = 4 * 16 * TP, U_ALL = U_T > 2048 ? U_T : 2048;
+    __shared__ double smem[U_ALL];  // the waves' point tables, then the sums of two tiles
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, fk = lane >> 4;
+    const int ncols = a.ncols, J = ncols * N;
+    const int j0 = (a.by_columns ? (int)blockIdx.y * 4 + wave : (int)blockIdx.y) * (16 * CB);
+    double *T = smem + wave * 16 * TP;
+    int r2[RB], r3[RB], cl[CB], ch[CB];  // rows' l2 and l3, columns' l1 and c
 #pragma unroll
-        for (int r = 0; r < PR; r++)
+    for (int r = 0; r < RB; r++) {
+        const int row = min(r * 16 + fr, N2 - 1);
+        r2[r] = N + row / N;
+        r3[r] = 2 * N + row % N;
+    }
 #pragma unroll
-            for (int m = 0; m < N; m++) acc[r][m] = 0.0;
-        for (int j0 = p0; j0 < p1; j0 += PTS) {
-            const int jn = min(PTS, p1 - j0);
-            __syncthreads();  // the previous chunk is consumed
-            if (tid < 3 * PTS) {
-                const int pp = tid % PTS, ax = tid / PTS;
+    for (int cb = 0; cb < CB; cb++) {
+        const int j = min(j0 + cb * 16 + fr, J - 1);
+        ch[cb] = j / N;
+        cl[cb] = j - ch[cb] * N;
+    }
+    dbl4 acc[RB][CB];
+    // acc += the product over points p0 + 16 (first + k step) ..., below p1
+    auto sum = [&](const int4 &it, int p1, int first, int step) __attribute__((always_inline)) {
+        const int li = it.x;
+        const uint32_t cc = (uint32_t)a.lt.coord[li][it.y];
+        const double *ctab = a.lt.ctab[li];
+        const int ax = min(lane >> 4, 2);
+        const double cen = ctab[(cc >> (10 * ax)) & 1023], ihalfL = 2.0 / a.lt.len[li];
+        const double *xa = ax == 0 ? a.x : ax == 1 ? a.y : a.z;
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++) acc[r][cb] = dbl4{0, 0, 0, 0};
+        for (int q0 = it.z + 16 * first; q0 < p1; q0 += 16 * step) {
+            const int jn = min(16, p1 - q0);
+            double wv[4][CB];
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++)
+                    wv[s][cb] = 4 * s + fk < jn ? a.wsT[(int64_t)(q0 + 4 * s + fk) * ncols + ch[cb]] : 0.0;
+            if (lane < 48) {
                 double S[N];
-                if (pp < jn) {
-                    const double *xa = ax == 0 ? a.x : ax == 1 ? a.y : a.z;
-                    sn_eval_n<N>(a.Tkz, ihalfL * (xa[j0 + pp] - cen[ax]), S);
-                } else {
 #pragma unroll
-                    for (int m = 0; m < N; m++) S[m] = 0.0;
+                for (int m = 0; m < N; m++) S[m] = 0.0;
+                if (fr < jn) sn_eval_n<N>(a.Tkz, ihalfL * (xa[q0 + fr] - cen), S);
+#pragma unroll
+                for (int m = 0; m < N; m++) T[fr * TP + ax * N + m] = S[m];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                if (4 * s >= jn) break;
+                const double *t = T + (4 * s + fk) * TP;
+                double av[RB], bv[CB];
+#pragma unroll
+                for (int r = 0; r < RB; r++) av[r] = t[r2[r]] * t[r3[r]];
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++) bv[cb] = wv[s][cb] * t[cl[cb]];
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++) {
+                    if (cb > 0 && j0 + cb * 16 >= J) break;
+#pragma unroll
+                    for (int r = 0; r < RB; r++)
+                        acc[r][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r], bv[cb], acc[r][cb], 0, 0, 0);
                 }
+                __builtin_amdgcn_sched_barrier(0);  // (read ahead, the tables of all steps would spill)
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    // element (row, column) of the item's expansion: split boxes write FP64
+    // partial sums to scratch slots, others S directly
+    auto store = [&](const int4 &it, int row, int j, double v) __attribute__((always_inline)) {
+        if (row >= N2 || j >= J) return;
+        const size_t at = (size_t)j * N2 + row;
+        if (it.w >= 0) a.scratch[(size_t)it.w * ncols * N3 + at] = v;
+        else ((TS *)a.S)[(size_t)(a.lt.off[it.x] + it.y) * ncols * N3 + at] = (TS)v;
+    };
+    auto end = [&](const int4 &it) { return min(it.z + P2M_SEG, a.lt.pstart[it.x][it.y + 1]); };
+
+    auto store_all = [&](const int4 &it) __attribute__((always_inline)) {
 #pragma unroll
-                for (int m = 0; m < N; m++) sS[ax][m][pp] = S[m];
-            }
-            for (int q = tid; q < PTS * CC; q += 256) {
-                const int pp = q / CC, c = q - pp * CC;
-                sw[pp][c] = (pp < jn && c < cn) ? a.wsT[(int64_t)(j0 + pp) * a.ncols + c0 + c] : 0.0;
-            }
+        for (int r = 0; r < RB; r++)
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) store(it, r * 16 + fk + 4 * v, j0 + cb * 16 + fr, acc[r][cb][v]);
+    };
+    const bool big = (int)blockIdx.x < a.nbig;
+    const int k0 = big ? (int)blockIdx.x : a.nbig + 4 * ((int)blockIdx.x - a.nbig);
+    const int k1 = big ? k0 + 1 : min(k0 + 4, a.nitems);
+    bool together = big;
+    for (int k = k0; k < k1 && !big; k++) together |= end(a.items[k]) - a.items[k].z > SMALL;
+    if (a.by_columns || !together) {
+        const int k = a.by_columns ? k0 : k0 + wave;
+        if (k >= k1 || j0 >= J) return;
+        const int4 it = a.items[k];
+        sum(it, end(it), 0, 1);
+        store_all(it);
+        return;
+    }
+    for (int k = k0; k < k1; k++) {
+        const int4 it = a.items[k];
+        sum(it, end(it), wave, 4);
+        // two tiles at a time: [tile][wave][v][lane]
+#pragma unroll
+        for (int t0 = 0; t0 < RB * CB; t0 += 2) {
             __syncthreads();
-            for (int pp = 0; pp < jn; pp++) {
-                double sz[N];
 #pragma unroll
-                for (int m = 0; m < N; m++) sz[m] = sS[2][m][pp];
+            for (int u = 0; u < 2; u++)
+                if (t0 + u < RB * CB)
 #pragma unroll
-                for (int r = 0; r < PR; r++) {
-                    const int q = tid + 256 * r;
-                    if (q < CC * N2) {
-                        const int c = q / N2, l12 = q - c * N2, l1 = l12 / N, l2 = l12 - l1 * N;
-                        const double t = sw[pp][c] * sS[0][l1][pp] * sS[1][l2][pp];
+                    for (int v = 0; v < 4; v++)
+                        smem[(u * 4 + wave) * 256 + v * 64 + lane] = acc[(t0 + u) / CB][(t0 + u) % CB][v];
+            __syncthreads();
 #pragma unroll
-                        for (int m = 0; m < N; m++) acc[r][m] += t * sz[m];
-                    }
+            for (int u = 0; u < 2; u++)
+                if (t0 + u < RB * CB) {
+                    const double *p = smem + u * 1024 + tid;  // (tid: v = wave, and the lane)
+                    store(it, (t0 + u) / CB * 16 + fk + 4 * wave, j0 + (t0 + u) % CB * 16 + fr,
+                          (p[0] + p[256]) + (p[512] + p[768]));
                 }
-            }
         }
-        if constexpr (sizeof(TS) == 4) {
-            if (!Sp) {  // FP32 S: through LDS, then contiguous (16-byte where aligned) stores
-                __syncthreads();  // the pass's point tables are consumed
-#pragma unroll
-                for (int r = 0; r < PR; r++) {
-                    const int q = tid + 256 * r;
-                    if (q < CC * N2) {
-                        const int c = q / N2, l12 = q - c * N2;
-#pragma unroll
-                        for (int m = 0; m < N; m++) sF[c * N3 + l12 * N + m] = (float)acc[r][m];
-                    }
-                }
-                __syncthreads();
-                float *dst = (float *)Sb + (size_t)c0 * N3;
-                const int n = cn * N3;
-                if ((n & 3) == 0 && ((uintptr_t)dst & 15) == 0) {
-                    for (int q = tid; q < n / 4; q += 256) ((float4 *)dst)[q] = ((const float4 *)sF)[q];
-                } else {
-                    for (int q = tid; q < n; q += 256) dst[q] = sF[q];
-                }
-                continue;
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < PR; r++) {
-            const int q = tid + 256 * r;
-            if (q < CC * N2) {
-                const int c = q / N2, l12 = q - c * N2;
-                if (c < cn) {
-                    const size_t at = (size_t)(c0 + c) * N3 + l12 * N;
-                    if (Sp) {
-#pragma unroll
-                        for (int m = 0; m < N; m++) Sp[at + m] = acc[r][m];
-                    } else {
-#pragma unroll
-                        for (int m = 0; m < N; m++) Sb[at + m] = (TS)acc[r][m];
-                    }
-                }
-            }
-        }
+        __syncthreads();
     }
 }
 
@@ -2044,19 +2083,42 @@ bool launch_near_split(const NearArgs &args, int kid, int nleaf, hipStream_t st)
     return true;
 }
 
-bool launch_p2m_levels(const UpArgs &a, int nitems, const UpReduce &r, hipStream_t st)
+bool launch_p2m_levels(const UpArgs &args, int nitems, const UpReduce &r, hipStream_t st)
 {
+    UpArgs a = args;
+    a.nitems = nitems;
+    a.nbig = std::min(a.nbig, nitems);
     if (a.n < 4 || a.n > 8) return false;
     if (nitems <= 0) return true;
-#define PBB_P2M_N(TS)                                                      \
-    switch (a.n) {                                                         \
-    case 4: p2m_levels<4, TS><<<nitems, 256, 0, st>>>(a); break;           \
-    case 5: p2m_levels<5, TS><<<nitems, 256, 0, st>>>(a); break;           \
-    case 6: p2m_levels<6, TS><<<nitems, 256, 0, st>>>(a); break;           \
-    case 7: p2m_levels<7, TS><<<nitems, 256, 0, st>>>(a); break;           \
-    default: p2m_levels<8, TS><<<nitems, 256, 0, st>>>(a); break;          \
+    // column blocks of a wave: those of the call, or what 9 tiles hold
+    const int blocks = (a.ncols * a.n + 15) / 16;
+    // (the whole call's columns choose how the points are summed, so that a
+    // chunk of them gives the same bits)
+    const int whole = (a.all * a.n + 15) / 16, most = a.n == 4 ? 4 : a.n <= 6 ? 3 : 2;
+    a.by_columns = whole > 2 * most;
+    if (a.by_columns) a.nbig = nitems;
+    auto grid = [&](int cb) {
+        const int ways = (blocks + cb - 1) / cb;
+        return dim3((unsigned)(a.nbig + (nitems - a.nbig + 3) / 4), (unsigned)(a.by_columns ? (ways + 3) / 4 : ways));
+    };
+#define PBB_P2M_CB(N, CB, TS)                                                                             \
+    do {                                                                                                  \
+        const dim3 g = grid(CB);                                                                          \
+        p2m_levels<N, CB, TS><<<g, 256, 0, st>>>(a);                                                      \
+    } while (0)
+#define PBB_P2M_N(N, CB, TS)                                                                              \
+    case N:                                                                                               \
+        if (blocks <= 1) PBB_P2M_CB(N, 1, TS);                                                            \
+        else if (blocks <= 2) PBB_P2M_CB(N, 2, TS);                                                       \
+        else PBB_P2M_CB(N, CB, TS);                                                                       \
+        break;
+#define PBB_P2M(TS)                                                                                       \
+    switch (a.n) {                                                                                        \
+        PBB_P2M_N(4, 4, TS) PBB_P2M_N(5, 3, TS) PBB_P2M_N(6, 3, TS) PBB_P2M_N(7, 2, TS) PBB_P2M_N(8, 2, TS) \
     }
-    if (a.s32) PBB_P2M_N(float) else PBB_P2M_N(double)
+    if (a.s32) { PBB_P2M(float) } else { PBB_P2M(double) }
+#undef PBB_P2M
+#undef PBB_P2M_CB
 #undef PBB_P2M_N
     check(hipGetLastError(), "p2m_levels");
     if (r.nred > 0) {

@@ -66,6 +66,7 @@ constexpr int P2M_SEG = 2048;  // points per workgroup of the direct upward pass
 
 struct UpArgs {
     int n, ncols;
+    int all;                   // columns of the whole call (>= ncols)
     LevelTab lt;
     // work items (level index, box, first point, scratch slot or -1), coarse
     // levels first; boxes of more than P2M_SEG points are split into items
@@ -75,6 +76,8 @@ struct UpArgs {
     void *S;                   // expansions: FP64, or FP32 with s32
     double *scratch;           // partial expansions of split boxes (FP64)
     int s32;
+    int nitems, nbig;          // the first nbig items take a workgroup each (p2m_levels)
+    int by_columns;            // ... and its waves divide the columns
 };
 
 struct UpReduce {
