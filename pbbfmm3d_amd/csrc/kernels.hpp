@@ -155,7 +155,8 @@ struct M2LArgs {
 constexpr int SYM_TB = 64;    // boxes of a tile
 constexpr int SYM_CONFS = 9;  // row configurations
 constexpr int SYM_NG2 = 32;   // row groups up to which a wave holds 32 columns (else 16)
-constexpr int SYM_NB = 2;     // orbits to a barrier
+constexpr int SYM_NG3 = 20;   // row groups up to which three workgroups fit a CU's registers
+constexpr int SYM_NB = 8;     // orbits to a barrier, at most
 
 // Row layout of a set: the configuration's groups of 4 rows (ng in each of
 // nrow slices, where a class has more than the configuration holds)
@@ -165,6 +166,7 @@ struct SymShape {
 
 struct SymArgs {
     int ncols, TB, cpt, side;
+    int NB;                    // orbits to a barrier
     int ldp, ldf;              // P and Pf strides per (box, column)
     int nrow;                  // row slices (SymShape)
     int npz, noz;              // sum parts: classes p = zp mod npz, orbits = zo mod noz

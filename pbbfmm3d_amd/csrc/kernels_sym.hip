@@ -15,8 +15,10 @@
 // Bound: the FP64 matrix cores (the Walsh-Hadamard sums share their issue
 // slots), then the latency of the gathered sources.  M2L of one matvec, with
 // the set's own factors and here: 1M uniform points, 1/r, order 5, 8 columns
-// 281 -> 66 ms (at the deepest level 57 ms; its products alone take 26 ms at
-// 77 TFLOP/s); 1M clustered points, Gaussian, 32 columns 1410 -> 115 ms.
+// 281 -> 62 ms (at the deepest level 54 ms; its products alone take 26 ms at
+// 77 TFLOP/s); 1M clustered points, Gaussian, 32 columns 1410 -> 95 ms.
+// Loading a step's sources under the products of the step before (16 columns a
+// wave, two register sets) was slower: 75 -> 89 ms for the first of these calls.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -189,7 +191,7 @@ __device__ __forceinline__ void sym_step(const uint32_t *const (&tab)[C::CB], co
 // registers.  Steps: class p and 8 k of it (two per lane, 64 bytes of a
 // proxy), outermost, so that the workgroups of an XCD read the same slice of
 // every proxy and operator at about the same time; then the orbits with a
-// source, SYM_NB to a barrier.  A batch's operator chunks are copied to a
+// source, NB to a barrier.  A batch's operator chunks are copied to a
 // double-buffered LDS tile without passing through registers.  Proxies are
 // gathered straight from memory as pairs of k, [box][k / 2][column][2], so
 // that neighbouring lanes read neighbouring columns; between two barriers one
@@ -198,16 +200,17 @@ __device__ __forceinline__ void sym_step(const uint32_t *const (&tab)[C::CB], co
 // offsets (one 64-bit add each; a box that is not there is the level's box of
 // zeros).
 template <class C>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m2l_sym_f64(SymArgs a)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(C::NG <= SYM_NG3 ? 3 : 2))) void m2l_sym_f64(SymArgs a)
 {
-    constexpr int NT = 256, NG = C::NG, NB = SYM_NB, ECH = 2 * NG * 16;  // doubles of an operator chunk
-    __shared__ double sE[2][NB][ECH];
+    constexpr int NT = 256, NG = C::NG, ECH = 2 * NG * 16;  // doubles of an operator chunk
+    const int NB = a.NB;
     __shared__ unsigned long long s_mask[56];
     __shared__ int4 s_list[56];  // the orbits of this sum part that have a source: kind, block, table offset, boxes
     __shared__ int s_n;
     __shared__ int s_tgt[SYM_TB];
     __shared__ int s_xyz[SYM_TB];
-    extern __shared__ uint32_t s_off[];  // [TB][189]: source offsets in units of 16 bytes
+    extern __shared__ double sE[];                      // [2][NB][ECH]
+    uint32_t *s_off = (uint32_t *)(sE + 2 * NB * ECH);  // [TB][189]: source offsets in units of 16 bytes
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int TB = a.TB;
@@ -309,16 +312,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     auto copy = [&](int p, int j0, int oi, int buf) {
         const double *src = a.Ef + ((size_t)rowp * a.nj + a.kb[p] + j0) * (size_t)(NG * 16);
         constexpr int UNITS = (ECH * 8 + 1023) / 1024;  // wave copies of 1 KB (the last one may overlap the one before)
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-            if (oi + b >= n) break;
+        for (int b = 0; b < NB && oi + b < n; b++) {
             const double *e = src + (size_t)(__builtin_amdgcn_readfirstlane(s_list[oi + b].x) >> 8) * blk;
 #pragma unroll
             for (int u = 0; u < UNITS; u += 4) {
                 if (u + wave < UNITS) {
                     const int at = min((u + wave) * 128, ECH - 128);
                     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(e + at + lane * 2),
-                                                     (__attribute__((address_space(3))) void *)&sE[buf][b][at], 16, 0,
+                                                     (__attribute__((address_space(3))) void *)(sE + (buf * NB + b) * ECH + at), 16, 0,
                                                      0);
                 }
             }
@@ -371,7 +372,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             const uint32_t *tab[C::CB];
 #pragma unroll
             for (int cb = 0; cb < C::CB; cb++) tab[cb] = tab0[cb] + le.y;
-            const double *e4 = &sE[buf][b][ai4], *e16 = &sE[buf][b][ai16];
+            const double *eb = sE + (buf * NB + b) * ECH, *e4 = eb + ai4, *e16 = eb + ai16;
 #define PBB_SYM_K(X, Y, Z)                                                                                   \
     case X * 16 + Y * 4 + Z:                                                                                 \
         if constexpr (X < 2 || Y < 2 || Z < 2) {                                                             \
@@ -495,6 +496,8 @@ constexpr SymConf CONF[SYM_CONFS] = {
     {{2, 2, 1, 1}}, {{2, 2, 2, 2}}, {{3, 3, 2, 2}}, {{5, 4, 3, 2}}, {{6, 4, 3, 2}},
     {{6, 5, 3, 2}}, {{6, 5, 4, 3}}, {{6, 5, 5, 4}}, {{7, 6, 6, 5}},
 };
+constexpr size_t SYM_LDS = 160 * 1024;      // of a CU
+constexpr size_t SYM_LDS_FIXED = 3328;      // the kernel's other arrays, and the allocation's granularity
 int blocks_for(int64_t total) { return (int)std::min<int64_t>((total + 255) / 256, 16384); }
 }  // namespace
 
@@ -537,8 +540,9 @@ void upload_sym_orbits()
     check(hipMemcpyToSymbol(HIP_SYMBOL(c_orb), &o, sizeof(o)), "hipMemcpyToSymbol(c_orb)");
 }
 
-void launch_m2l_sym(const SymArgs &a, const SymShape &s, int ncolchunks, hipStream_t st)
+void launch_m2l_sym(const SymArgs &args, const SymShape &s, int ncolchunks, hipStream_t st)
 {
+    SymArgs a = args;
     if (a.class_start[8] <= 0) return;
     if (a.TB < 1 || a.TB > SYM_TB || a.TB * a.cpt > sym_width(s) || (a.npz & (a.npz - 1)) != 0)
         fail(PBB_ERR_INTERNAL, "M2L tile does not fit its workgroup");
@@ -546,7 +550,16 @@ void launch_m2l_sym(const SymArgs &a, const SymShape &s, int ncolchunks, hipStre
         fail(PBB_ERR_INTERNAL, "M2L level of more than 64 GB of proxies");
     const int most = *std::max_element(a.class_tiles, a.class_tiles + 8);
     dim3 grid((unsigned)most * 8, (unsigned)ncolchunks, (unsigned)(a.nrow * a.npz * a.noz));
-    const size_t lds = sizeof(uint32_t) * 189 * a.TB;
+    // orbits to a barrier: what LDS holds beside the table at the workgroups
+    // per CU that the registers allow (a barrier waits for the slowest wave's
+    // gathers).  Two for all and now, one matvec: 1M points, 8 columns (4
+    // orbits) 75.4 -> 72.0 ms; 1M clustered, 32 columns (4, with the third
+    // workgroup of small configurations) 147 -> 129 ms.  Four at the price of a
+    // workgroup (500k points, 4 columns) was slower by a third.
+    const size_t table = sizeof(uint32_t) * 189 * a.TB, chunk = 2 * sizeof(double) * 2 * s.ng * 16;
+    const size_t room = SYM_LDS / (s.ng <= SYM_NG3 || s.conf == 6 ? 3 : 2) - SYM_LDS_FIXED;
+    a.NB = (int)std::max<size_t>(2, std::min<size_t>(SYM_NB, room > table ? (room - table) / chunk : 0));
+    const size_t lds = chunk * a.NB + table;
     switch (s.conf) {
     case 0: m2l_sym_f64<Cfg<2, 2, 1, 1>><<<grid, 256, lds, st>>>(a); break;
     case 1: m2l_sym_f64<Cfg<2, 2, 2, 2>><<<grid, 256, lds, st>>>(a); break;
