@@ -195,6 +195,11 @@ __global__ __launch_bounds__(TPB) void fill_i32(int32_t *__restrict__ p, int64_t
     for (int64_t q = blockIdx.x * (int64_t)TPB + threadIdx.x; q < n; q += (int64_t)gridDim.x * TPB) p[q] = v;
 }
 
+__global__ __launch_bounds__(TPB) void iota_i32(int32_t *__restrict__ p, int64_t n)
+{
+    for (int64_t q = blockIdx.x * (int64_t)TPB + threadIdx.x; q < n; q += (int64_t)gridDim.x * TPB) p[q] = (int32_t)q;
+}
+
 // child[p * 8 + octant] of every parent p, from each child's parent index
 __global__ __launch_bounds__(TPB) void child_table(const uint32_t *__restrict__ ck, const int32_t *__restrict__ parent,
                                                    int64_t nb, int32_t *__restrict__ child)
@@ -210,29 +215,41 @@ __global__ __launch_bounds__(TPB) void box_ranges(const int32_t *__restrict__ fi
                                                   int32_t *__restrict__ pstart, uint32_t *__restrict__ cls,
                                                   int32_t *__restrict__ ids, unsigned long long *__restrict__ hist)
 {
+    __shared__ unsigned sh[8];
+    if (threadIdx.x < 8) sh[threadIdx.x] = 0;
+    __syncthreads();
     for (int64_t b = blockIdx.x * (int64_t)TPB + threadIdx.x; b < nb; b += (int64_t)gridDim.x * TPB) {
         pstart[b] = leaf_start[first[b]];
         cls[b] = key[b] & 7u;
         ids[b] = (int32_t)b;
-        atomicAdd(&hist[key[b] & 7u], 1ull);
+        atomicAdd(&sh[key[b] & 7u], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < 8 && sh[threadIdx.x]) atomicAdd(&hist[threadIdx.x], (unsigned long long)sh[threadIdx.x]);
+}
+
+// per box: L2P segments, upward work items, scratch slots, reductions (element
+// nb is zero: its exclusive sum is the total)
+__global__ __launch_bounds__(TPB) void box_counts(const int32_t *__restrict__ pstart, int64_t nb, int4 *__restrict__ cnt)
+{
+    for (int64_t b = blockIdx.x * (int64_t)TPB + threadIdx.x; b <= nb; b += (int64_t)gridDim.x * TPB) {
+        int4 c{0, 0, 0, 0};
+        if (b < nb) {
+            const int np = pstart[b + 1] - pstart[b];
+            const int m = (np + P2M_SEG - 1) / P2M_SEG;
+            const bool split = np > P2M_SEG;
+            c = int4{(np + L2P_SEG - 1) / L2P_SEG, split ? m : 1, split ? m : 0, split ? 1 : 0};
+        }
+        cnt[b] = c;
     }
 }
 
-// per box: L2P segments, upward work items, scratch slots, reductions
-__global__ __launch_bounds__(TPB) void box_counts(const int32_t *__restrict__ pstart, int64_t nb, int *__restrict__ nseg,
-                                                  int *__restrict__ nitem, int *__restrict__ nslot,
-                                                  int *__restrict__ nred)
-{
-    for (int64_t b = blockIdx.x * (int64_t)TPB + threadIdx.x; b < nb; b += (int64_t)gridDim.x * TPB) {
-        const int np = pstart[b + 1] - pstart[b];
-        nseg[b] = (np + L2P_SEG - 1) / L2P_SEG;
-        const int m = (np + P2M_SEG - 1) / P2M_SEG;
-        const bool split = np > P2M_SEG;
-        nitem[b] = split ? m : 1;
-        nslot[b] = split ? m : 0;
-        nred[b] = split ? 1 : 0;
+struct Sum4 {
+    __host__ __device__ int4 operator()(const int4 &a, const int4 &b) const
+    {
+        return int4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w};
     }
-}
+};
 
 struct LevelBase {
     int li;           // level index l - 2
@@ -241,27 +258,27 @@ struct LevelBase {
 };
 
 __global__ __launch_bounds__(TPB) void box_emit(const int32_t *__restrict__ pstart, int64_t nb,
-                                                const int *__restrict__ sseg, const int *__restrict__ sitem,
-                                                const int *__restrict__ sslot, const int *__restrict__ sred,
-                                                LevelBase lb, int32_t *__restrict__ seg_box, int32_t *__restrict__ seg_p0,
+                                                const int4 *__restrict__ first_of, LevelBase lb,
+                                                int32_t *__restrict__ seg_box, int32_t *__restrict__ seg_p0,
                                                 int4 *__restrict__ items, int4 *__restrict__ reds)
 {
     for (int64_t b = blockIdx.x * (int64_t)TPB + threadIdx.x; b < nb; b += (int64_t)gridDim.x * TPB) {
         const int p0 = pstart[b], p1 = pstart[b + 1], np = p1 - p0;
-        int s = sseg[b];
+        const int4 f = first_of[b];
+        int s = f.x;
         for (int q = p0; q < p1; q += L2P_SEG, s++) {
             seg_box[s] = (int32_t)b;
             seg_p0[s] = q;
         }
-        const int it = lb.item0 + sitem[b];
+        const int it = lb.item0 + f.y;
         if (np <= P2M_SEG) {
             items[it] = int4{lb.li, (int)b, p0, -1};
             continue;
         }
-        const int first = lb.slot0 + sslot[b];
+        const int first = lb.slot0 + f.z;
         int k = 0;
         for (int q = p0; q < p1; q += P2M_SEG, k++) items[it + k] = int4{lb.li, (int)b, q, first + k};
-        reds[lb.red0 + sred[b]] = int4{(int)(lb.off + b), first, k, 0};
+        reds[lb.red0 + f.w] = int4{(int)(lb.off + b), first, k, 0};
     }
 }
 
@@ -274,6 +291,9 @@ __global__ __launch_bounds__(TPB) void leaf_stats(const int32_t *__restrict__ le
                                                   unsigned long long *__restrict__ hist, int *__restrict__ max_leaf,
                                                   unsigned long long *__restrict__ near_pairs)
 {
+    __shared__ unsigned sh[8];
+    if (threadIdx.x < 8) sh[threadIdx.x] = 0;
+    __syncthreads();
     const int64_t S = 1LL << levels;
     unsigned long long q = 0;
     int mx = 0;
@@ -283,7 +303,7 @@ __global__ __launch_bounds__(TPB) void leaf_stats(const int32_t *__restrict__ le
         while (c < NEAR_CLASSES - 1 && nt > (2 << c)) c++;
         cls[b] = (uint32_t)c;
         ids[b] = (int32_t)b;
-        atomicAdd(&hist[c], 1ull);
+        atomicAdd(&sh[c], 1u);
         mx = max(mx, nt);
         const int32_t cc = coord[b];
         const int64_t ix = cc & 1023, iy = (cc >> 10) & 1023, iz = (cc >> 20) & 1023;
@@ -304,28 +324,60 @@ __global__ __launch_bounds__(TPB) void leaf_stats(const int32_t *__restrict__ le
         if (q) atomicAdd(near_pairs, q);
         atomicMax(max_leaf, mx);
     }
+    __syncthreads();
+    if (threadIdx.x < 8 && sh[threadIdx.x]) atomicAdd(&hist[threadIdx.x], (unsigned long long)sh[threadIdx.x]);
 }
 
 // far-field (target, source) box pairs of one level: the 189 offsets of
-// each box's octant class that land on a non-empty box
+// each box's octant class that land on a non-empty box, a wave to a box and
+// an offset to a lane (a thread per box made them a serial chain, 83 us a level
+// of 4096 boxes)
 __global__ __launch_bounds__(TPB) void m2l_pair_count(const int32_t *__restrict__ coord, const int32_t *__restrict__ map,
                                                       int64_t nb, int l, const int *__restrict__ dirs,
                                                       unsigned long long *__restrict__ pairs)
 {
-    const int64_t S = 1LL << l;
+    __shared__ unsigned long long sq[TPB / 64];
+    const int S = 1 << l, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     unsigned long long q = 0;
-    for (int64_t b = blockIdx.x * (int64_t)TPB + threadIdx.x; b < nb; b += (int64_t)gridDim.x * TPB) {
+    for (int64_t b = blockIdx.x * (int64_t)(TPB / 64) + wave; b < nb; b += (int64_t)gridDim.x * (TPB / 64)) {
         const int32_t c = coord[b];
-        const int64_t ix = c & 1023, iy = (c >> 10) & 1023, iz = (c >> 20) & 1023;
-        const int *d = dirs + (((ix & 1) << 2) | ((iy & 1) << 1) | (iz & 1)) * 189 * 4;
-        for (int k = 0; k < 189; k++) {
-            const int64_t sx = ix + d[4 * k], sy = iy + d[4 * k + 1], sz = iz + d[4 * k + 2];
+        const int ix = c & 1023, iy = (c >> 10) & 1023, iz = (c >> 20) & 1023;
+        const int4 *d = (const int4 *)dirs + (((ix & 1) << 2) | ((iy & 1) << 1) | (iz & 1)) * 189;
+        for (int k = lane; k < 189; k += 64) {
+            const int4 v = d[k];
+            const int sx = ix + v.x, sy = iy + v.y, sz = iz + v.z;
             if (sx < 0 || sy < 0 || sz < 0 || sx >= S || sy >= S || sz >= S) continue;
-            if (map[(sx * S + sy) * S + sz] >= 0) q++;
+            if (map[((int64_t)sx * S + sy) * S + sz] >= 0) q++;
         }
     }
     for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o);
-    if ((threadIdx.x & 63) == 0 && q) atomicAdd(pairs, q);
+    if (lane == 0) sq[wave] = q;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < TPB / 64; w++) q += sq[w];
+        if (q) atomicAdd(pairs, q);
+    }
+}
+
+// Boxes of every level from the sorted leaf keys: a leaf starts a new box at
+// the levels from the first one at which its key differs from the leaf's
+// before it; counts[l] boxes start at l and not above it.
+__global__ __launch_bounds__(TPB) void level_starts(const uint32_t *__restrict__ key, int64_t nleaf, int levels,
+                                                    int *__restrict__ counts)
+{
+    __shared__ int sc[16];
+    if (threadIdx.x < 16) sc[threadIdx.x] = 0;
+    __syncthreads();
+    for (int64_t b = blockIdx.x * (int64_t)TPB + threadIdx.x; b < nleaf; b += (int64_t)gridDim.x * TPB) {
+        int l = 0;
+        if (b > 0) {  // (the keys differ: 3 bits a level, the leaf's lowest)
+            const uint32_t x = key[b] ^ key[b - 1];
+            l = levels - (31 - __clz(x)) / 3;
+        }
+        atomicAdd(&sc[l], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < 16 && sc[threadIdx.x]) atomicAdd(&counts[threadIdx.x], sc[threadIdx.x]);
 }
 
 // device allocations of one build: freed unless handed over; a buffer is
@@ -333,6 +385,22 @@ __global__ __launch_bounds__(TPB) void m2l_pair_count(const int32_t *__restrict_
 struct Pool {
     hipStream_t st;
     std::vector<void *> owned;
+    char *slab = nullptr;  // small arrays of the build, carved from blocks of 1 MB and more
+    size_t slab_left = 0;
+    template <typename T>
+    T *carve(size_t n, const char *what)
+    {
+        const size_t bytes = (std::max<size_t>(1, n) * sizeof(T) + 255) & ~(size_t)255;
+        if (bytes > slab_left) {
+            const size_t block = std::max<size_t>(bytes, 1 << 20);
+            slab = get<char>(block, what);
+            slab_left = block;
+        }
+        T *p = (T *)slab;
+        slab += bytes;
+        slab_left -= bytes;
+        return p;
+    }
     template <typename T>
     T *get(size_t n, const char *what)
     {
@@ -404,12 +472,10 @@ int exclusive_count(Temp &tmp, const int *in, int *out, int64_t n, hipStream_t s
 void sort_by_class(Temp &tmp, Pool &pool, const uint32_t *cls, const int32_t *ids, int32_t *out, int64_t n, int bits,
                    hipStream_t st)
 {
-    uint32_t *cls_out = pool.get<uint32_t>(n, "class sort keys");
+    uint32_t *cls_out = pool.carve<uint32_t>(n, "class sort keys");
     size_t b = 0;
     check(hipcub::DeviceRadixSort::SortPairs(nullptr, b, cls, cls_out, ids, out, (int)n, 0, bits, st), "sort size");
     check(hipcub::DeviceRadixSort::SortPairs(tmp.need(b), b, cls, cls_out, ids, out, (int)n, 0, bits, st), "sort");
-    check(hipStreamSynchronize(st), "hipStreamSynchronize");
-    pool.drop(cls_out);
 }
 
 }  // namespace
@@ -493,30 +559,34 @@ void build_tree_gpu(GpuTree &T, const double *xyz_host, int64_t N, int64_t nbox,
     // levels L-1 .. 0: parents are the runs of equal key >> 3
     T.lv.assign(levels + 1, GpuLevel());
     T.lv[levels].nb = nleaf;
-    lfirst[levels] = pool.get<int32_t>(nleaf, "first leaves");
-    {
-        std::vector<int32_t> iota(nleaf);
-        for (int b = 0; b < nleaf; b++) iota[b] = b;
-        check(hipMemcpyAsync(lfirst[levels], iota.data(), sizeof(int32_t) * nleaf, hipMemcpyHostToDevice, st),
-              "upload leaf ids");
-        check(hipStreamSynchronize(st), "hipStreamSynchronize");
-    }
+    lfirst[levels] = pool.carve<int32_t>(nleaf, "first leaves");
+    iota_i32<<<nblocks(nleaf), TPB, 0, st>>>(lfirst[levels], nleaf);
+    check(hipGetLastError(), "iota_i32");
+    // every level's box count in one read: the levels' arrays follow without
+    // another wait
+    int *starts = pool.carve<int>(16, "level counts");
+    fill_i32<<<1, TPB, 0, st>>>(starts, 16, 0);
+    level_starts<<<nblocks(nleaf, 256), TPB, 0, st>>>(lkeys[levels], nleaf, levels, starts);
+    check(hipGetLastError(), "level_starts");
+    int hs[16];
+    check(hipMemcpyAsync(hs, starts, sizeof(hs), hipMemcpyDeviceToHost, st), "copy level counts");
+    check(hipStreamSynchronize(st), "hipStreamSynchronize");
+    for (int l = 0, run = 0; l < levels; l++) T.lv[l].nb = run += hs[l];
     std::vector<int32_t *> parent(levels + 1, nullptr);
     for (int l = levels - 1; l >= 0; l--) {
-        const int64_t nbc = T.lv[l + 1].nb;
-        int *h = pool.get<int>(nbc, "heads"), *p = pool.get<int>(nbc, "positions");
+        const int64_t nbc = T.lv[l + 1].nb, nbp = T.lv[l].nb;
+        int *h = pool.carve<int>(nbc, "heads"), *p = pool.carve<int>(nbc, "positions");
         parent_heads<<<nblocks(nbc), TPB, 0, st>>>(lkeys[l + 1], nbc, h);
         check(hipGetLastError(), "parent_heads");
-        const int nbp = exclusive_count(tmp, h, p, nbc, st);
-        T.lv[l].nb = nbp;
-        lkeys[l] = pool.get<uint32_t>(nbp, "box keys");
-        lfirst[l] = pool.get<int32_t>(nbp, "first leaves");
-        parent[l + 1] = pool.get<int32_t>(nbc, "parent ids");
+        size_t b = 0;
+        check(hipcub::DeviceScan::ExclusiveSum(nullptr, b, h, p, (int)nbc, st), "scan size");
+        check(hipcub::DeviceScan::ExclusiveSum(tmp.need(b), b, h, p, (int)nbc, st), "scan");
+        lkeys[l] = pool.carve<uint32_t>(nbp, "box keys");
+        lfirst[l] = pool.carve<int32_t>(nbp, "first leaves");
+        parent[l + 1] = pool.carve<int32_t>(nbc, "parent ids");
         parent_boxes<<<nblocks(nbc), TPB, 0, st>>>(lkeys[l + 1], lfirst[l + 1], h, p, nbc, lkeys[l], lfirst[l],
                                                     parent[l + 1]);
         check(hipGetLastError(), "parent_boxes");
-        pool.drop(h);
-        pool.drop(p);
     }
     for (int l = 0; l <= levels; l++) {
         GpuLevel &V = T.lv[l];
@@ -534,55 +604,58 @@ void build_tree_gpu(GpuTree &T, const double *xyz_host, int64_t N, int64_t nbox,
         }
     }
 
-    // levels >= 2: point ranges, octant-class order, L2P segments, upward items
-    struct Counts {
-        int *seg, *item, *slot, *red, *sseg, *sitem, *sslot, *sred;
-        int nseg, nitem, nslot, nred;
-    };
-    std::vector<Counts> cnts(levels + 1);
-    int items_total = 0, slots_total = 0, reds_total = 0;
-    std::vector<LevelBase> base(levels + 1);
+    // levels >= 2: point ranges, octant-class order, L2P segments, upward
+    // items; one wait for all levels' counts
+    // (a wait and two small copies for each of four counts a level, and one
+    // for every parent level, were half of a 20k-point host call: 2.38 -> 1.39 ms
+    // with them gathered, the statistics kernels included)
+    std::vector<int4 *> scans(levels + 1, nullptr);
+    std::vector<int4> totals(levels + 1);
+    int4 *dtot = pool.carve<int4>(levels + 1, "totals");  // (levels 0 and 1 are not used)
+    unsigned long long *hist = pool.carve<unsigned long long>(8 * (levels + 1), "class counts");
+    check(hipMemsetAsync(hist, 0, 8 * (levels + 1) * sizeof(unsigned long long), st), "clear histogram");
+    std::vector<unsigned long long> hh(8 * (levels + 1));
     int64_t off = 0;
     for (int l = 2; l <= levels; l++) {
         GpuLevel &V = T.lv[l];
         V.off = off;
         off += V.nb;
         V.pstart = pool.get<int32_t>((size_t)V.nb + 1, "box point ranges");
-        uint32_t *cls = pool.get<uint32_t>(V.nb, "classes");
-        int32_t *ids = pool.get<int32_t>(V.nb, "ids");
-        unsigned long long *hist = cnt + 8;
-        check(hipMemsetAsync(hist, 0, 8 * sizeof(unsigned long long), st), "clear histogram");
-        box_ranges<<<nblocks(V.nb), TPB, 0, st>>>(lfirst[l], T.leaf_start, lkeys[l], V.nb, V.pstart, cls, ids, hist);
+        uint32_t *cls = pool.carve<uint32_t>(V.nb, "classes");
+        int32_t *ids = pool.carve<int32_t>(V.nb, "ids");
+        box_ranges<<<nblocks(V.nb), TPB, 0, st>>>(lfirst[l], T.leaf_start, lkeys[l], V.nb, V.pstart, cls, ids,
+                                                   hist + 8 * l);
         check(hipGetLastError(), "box_ranges");
         set_i32<<<1, 1, 0, st>>>(V.pstart + V.nb, (int32_t)N);
-        unsigned long long hh[8];
-        check(hipMemcpyAsync(hh, hist, sizeof(hh), hipMemcpyDeviceToHost, st), "copy histogram");
         V.order = pool.get<int32_t>(V.nb, "class order");
         sort_by_class(tmp, pool, cls, ids, V.order, V.nb, 3, st);
-        for (int c = 0; c < 8; c++) V.class_count[c] = (int64_t)hh[c];
-        pool.drop(cls);
-        pool.drop(ids);
-        Counts &C = cnts[l];
-        C.seg = pool.get<int>(V.nb, "counts");
-        C.item = pool.get<int>(V.nb, "counts");
-        C.slot = pool.get<int>(V.nb, "counts");
-        C.red = pool.get<int>(V.nb, "counts");
-        C.sseg = pool.get<int>(V.nb, "scans");
-        C.sitem = pool.get<int>(V.nb, "scans");
-        C.sslot = pool.get<int>(V.nb, "scans");
-        C.sred = pool.get<int>(V.nb, "scans");
-        box_counts<<<nblocks(V.nb), TPB, 0, st>>>(V.pstart, V.nb, C.seg, C.item, C.slot, C.red);
+        int4 *counts = pool.carve<int4>(V.nb + 1, "counts");
+        scans[l] = pool.carve<int4>(V.nb + 1, "scans");
+        box_counts<<<nblocks(V.nb + 1), TPB, 0, st>>>(V.pstart, V.nb, counts);
         check(hipGetLastError(), "box_counts");
-        C.nseg = exclusive_count(tmp, C.seg, C.sseg, V.nb, st);
-        C.nitem = exclusive_count(tmp, C.item, C.sitem, V.nb, st);
-        C.nslot = exclusive_count(tmp, C.slot, C.sslot, V.nb, st);
-        C.nred = exclusive_count(tmp, C.red, C.sred, V.nb, st);
+        size_t b = 0;
+        const int4 zero{0, 0, 0, 0};
+        check(hipcub::DeviceScan::ExclusiveScan(nullptr, b, counts, scans[l], Sum4(), zero, (int)(V.nb + 1), st),
+              "scan size");
+        check(hipcub::DeviceScan::ExclusiveScan(tmp.need(b), b, counts, scans[l], Sum4(), zero, (int)(V.nb + 1), st),
+              "scan");
+        check(hipMemcpyAsync(dtot + l, scans[l] + V.nb, sizeof(int4), hipMemcpyDeviceToDevice, st), "copy totals");
+    }
+    check(hipMemcpyAsync(totals.data(), dtot, totals.size() * sizeof(int4), hipMemcpyDeviceToHost, st),
+          "copy totals");
+    check(hipMemcpyAsync(hh.data(), hist, hh.size() * sizeof(hh[0]), hipMemcpyDeviceToHost, st), "copy histogram");
+    check(hipStreamSynchronize(st), "hipStreamSynchronize");
+    int items_total = 0, slots_total = 0, reds_total = 0;
+    std::vector<LevelBase> base(levels + 1);
+    for (int l = 2; l <= levels; l++) {
+        GpuLevel &V = T.lv[l];
+        for (int c = 0; c < 8; c++) V.class_count[c] = (int64_t)hh[8 * l + c];
         base[l] = LevelBase{l - 2, V.off, items_total, slots_total, reds_total};
         V.up_item0 = items_total;
         V.up_red0 = reds_total;
-        items_total += C.nitem;
-        slots_total += C.nslot;
-        reds_total += C.nred;
+        items_total += totals[l].y;
+        slots_total += totals[l].z;
+        reds_total += totals[l].w;
     }
     T.Btot = off;
     if (off >= (1LL << 31)) fail(PBB_ERR_UNSUPPORTED, "too many boxes");
@@ -593,21 +666,20 @@ void build_tree_gpu(GpuTree &T, const double *xyz_host, int64_t N, int64_t nbox,
     T.n_up_slots = slots_total;
     for (int l = 2; l <= levels; l++) {
         GpuLevel &V = T.lv[l];
-        Counts &C = cnts[l];
-        V.nseg = C.nseg;
-        V.seg_box = pool.get<int32_t>(C.nseg, "L2P segments");
-        V.seg_p0 = pool.get<int32_t>(C.nseg, "L2P segments");
-        box_emit<<<nblocks(V.nb), TPB, 0, st>>>(V.pstart, V.nb, C.sseg, C.sitem, C.sslot, C.sred, base[l], V.seg_box,
-                                                 V.seg_p0, T.up_items, T.up_reds);
+        V.nseg = totals[l].x;
+        V.seg_box = pool.get<int32_t>(V.nseg, "L2P segments");
+        V.seg_p0 = pool.get<int32_t>(V.nseg, "L2P segments");
+        box_emit<<<nblocks(V.nb), TPB, 0, st>>>(V.pstart, V.nb, scans[l], base[l], V.seg_box, V.seg_p0, T.up_items,
+                                                 T.up_reds);
         check(hipGetLastError(), "box_emit");
     }
 
     // near-field leaf classes, largest leaf, pair counts
     {
         const GpuLevel &V = T.lv[levels];
-        uint32_t *cls = pool.get<uint32_t>(V.nb, "leaf classes");
-        int32_t *ids = pool.get<int32_t>(V.nb, "ids");
-        int *mxl = pool.get<int>(1, "max leaf");
+        uint32_t *cls = pool.carve<uint32_t>(V.nb, "leaf classes");
+        int32_t *ids = pool.carve<int32_t>(V.nb, "ids");
+        int *mxl = pool.carve<int>(1, "max leaf");
         check(hipMemsetAsync(mxl, 0, sizeof(int), st), "clear");
         check(hipMemsetAsync(cnt + 8, 0, 8 * sizeof(unsigned long long), st), "clear histogram");
         leaf_stats<<<nblocks(V.nb), TPB, 0, st>>>(T.leaf_start, V.coord, V.map, V.nb, levels, cls, ids, cnt + 8, mxl,
@@ -624,8 +696,6 @@ void build_tree_gpu(GpuTree &T, const double *xyz_host, int64_t N, int64_t nbox,
             run += (int)hh[c];
         }
         T.leaf_class_off[NEAR_CLASSES] = run;
-        pool.drop(cls);
-        pool.drop(ids);
     }
     int *ddirs = pool.get<int>(8 * 189 * 4, "directions");
     check(hipMemcpyAsync(ddirs, dirs, sizeof(int) * 8 * 189 * 4, hipMemcpyHostToDevice, st), "upload directions");
@@ -634,7 +704,7 @@ void build_tree_gpu(GpuTree &T, const double *xyz_host, int64_t N, int64_t nbox,
     unsigned long long *lpairs = pool.get<unsigned long long>(16, "pair counters");
     check(hipMemsetAsync(lpairs, 0, 16 * sizeof(unsigned long long), st), "clear pair counters");
     for (int l = 2; l <= levels; l++) {
-        m2l_pair_count<<<nblocks(T.lv[l].nb, 4096), TPB, 0, st>>>(T.lv[l].coord, T.lv[l].map, T.lv[l].nb, l, ddirs,
+        m2l_pair_count<<<nblocks(64 * T.lv[l].nb, 4096), TPB, 0, st>>>(T.lv[l].coord, T.lv[l].map, T.lv[l].nb, l, ddirs,
                                                                   lpairs + l);
         check(hipGetLastError(), "m2l_pair_count");
     }
