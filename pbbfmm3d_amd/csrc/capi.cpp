@@ -2611,7 +2611,9 @@ static int64_t kept_doubles(pbb_plan *p, int ncols, int prec)
     check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
     const size_t margin = std::max((size_t)(1ull << 30), total_b / 16);
     const size_t grow = need > p->ws_bytes ? need - p->ws_bytes : 0;
-    return grow + (size_t)n * sizeof(double) + margin <= free_b ? n : 0;
+    // twice the expansions: the caller's allocator may hold a freed buffer of the
+    // last step where this step's gradient has to make its own
+    return grow + 2 * (size_t)n * sizeof(double) + margin <= free_b ? n : 0;
 }
 
 PBB_API pbb_status pbb_plan_kept_size(pbb_plan *plan, int32_t ncols, int32_t precision, int64_t *count)
