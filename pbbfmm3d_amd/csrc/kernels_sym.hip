@@ -15,7 +15,7 @@
 // Bound: the FP64 matrix cores (the Walsh-Hadamard sums share their issue
 // slots), then the latency of the gathered sources.  M2L of one matvec, with
 // the set's own factors and here: 1M uniform points, 1/r, order 5, 8 columns
-// 281 -> 62 ms (at the deepest level 54 ms; its products alone take 26 ms at
+// 281 -> 64 ms (at the deepest level 56 ms; its products alone take 26 ms at
 // 77 TFLOP/s); 1M clustered points, Gaussian, 32 columns 1410 -> 95 ms.
 // Loading a step's sources under the products of the step before (16 columns a
 // wave, two register sets) was slower: 75 -> 89 ms for the first of these calls.
@@ -209,8 +209,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(C::NG <= SY
     __shared__ int s_n;
     __shared__ int s_tgt[SYM_TB];
     __shared__ int s_xyz[SYM_TB];
-    extern __shared__ double sE[];                      // [2][NB][ECH]
-    uint32_t *s_off = (uint32_t *)(sE + 2 * NB * ECH);  // [TB][189]: source offsets in units of 16 bytes
+    extern __shared__ __attribute__((aligned(16))) double sE[];  // [2][NB][ECH], written 16 bytes a lane
+    uint32_t *s_off = (uint32_t *)(sE + 2 * NB * ECH);           // [TB][189]: source offsets in units of 16 bytes
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int TB = a.TB;
