@@ -700,6 +700,8 @@ struct pbb_plan {
     int n_up_items = 0, n_up_reds = 0, n_up_slots = 0;
     bool expansion_route = false;               // PBB_PLAN_EXPANSION_ROUTE: no proxy passes
     int leaf_class_off[dev::NEAR_CLASSES + 1] = {0};
+    int2 *near_passes = nullptr;                // (leaf, pass) of the last class (nullptr: one pass a leaf)
+    int n_near_passes = 0;
     std::vector<DevLevel> lv;
     int64_t Btot = 0;
     Workspace W;                  // the plan's own matvec buffers (one block)
@@ -734,7 +736,7 @@ struct pbb_plan {
         (void)hipGetDevice(&prev);
         (void)hipSetDevice(device);
         if (stream) (void)hipStreamSynchronize(stream);
-        dfree(x); dfree(y); dfree(z); dfree(perm); dfree(leaf_start); dfree(leaf_class);
+        dfree(x); dfree(y); dfree(z); dfree(perm); dfree(leaf_start); dfree(leaf_class); dfree(near_passes);
         dfree(up_items); dfree(up_reds); dfree(pt_leaf);
         for (auto &L : lv) {
             dfree(L.coord); dfree(L.map); dfree(L.child); dfree(L.order); dfree(L.ctab);
@@ -1386,6 +1388,12 @@ static void plan_create_host(pbb_ops *ops, const double *xyz, int64_t npoints, i
             }
             plan->leaf_class_off[dev::NEAR_CLASSES] = (int)all.size();
             plan->leaf_class = dupload(all, "leaf classes");
+            std::vector<int2> passes;
+            for (int32_t b : cls[dev::NEAR_CLASSES - 1])
+                for (int k = 0; 64 * k < T.leaf_start[b + 1] - T.leaf_start[b]; k++) passes.push_back(int2{b, k});
+            plan->n_near_passes = (int)passes.size();
+            if (passes.size() > cls[dev::NEAR_CLASSES - 1].size())
+                plan->near_passes = dupload(passes, "near-field passes");
         }
         plan->lv.resize(T.Lv + 1);
         int64_t off = 0;
@@ -1540,6 +1548,8 @@ static void plan_create_gpu(pbb_ops *ops, const double *xyz, int64_t npoints, in
     }
     for (int l = 0; l <= Lv; l++) plan->lv[l].ctab = dupload(ctab[l], "ctab");
     std::copy(std::begin(T.leaf_class_off), std::end(T.leaf_class_off), plan->leaf_class_off);
+    plan->near_passes = T.near_passes;
+    plan->n_near_passes = T.n_near_passes;
     plan->n_up_items = T.n_up_items;
     plan->n_up_reds = T.n_up_reds;
     plan->n_up_slots = T.n_up_slots;
@@ -2488,7 +2498,8 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
         a.leaf_class = p->leaf_class;
         std::copy(std::begin(p->leaf_class_off), std::end(p->leaf_class_off), a.leaf_class_off);
         a.kf32 = mixed ? 1 : 0;
-        a.max_leaf = (int)p->info.max_leaf_points;
+        a.passes = p->near_passes;
+        a.npass = p->n_near_passes;
         a.all = W.all;
         if (!(direct && dev::launch_near_split(a, h.kernel.id, (int)LL.nb, st)))
             dev::launch_near(a, h.kernel.id, (int)LL.nb, st);
@@ -2703,7 +2714,8 @@ static void gradients(pbb_plan *p, const double *sigma_dev, const double *kept_d
     a.ctab = LL.ctab; a.Tkz = p->ops->d_Tkz; a.x = p->x; a.y = p->y; a.z = p->z;
     a.leaf_class = p->leaf_class;
     std::copy(std::begin(p->leaf_class_off), std::end(p->leaf_class_off), a.leaf_class_off);
-    a.max_leaf = (int)p->info.max_leaf_points;
+    a.passes = p->near_passes;
+    a.npass = p->n_near_passes;
     a.grad = grad_dev;
     a.sig = p->gU;
     a.psi = W.wsT;

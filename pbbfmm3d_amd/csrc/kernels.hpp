@@ -256,7 +256,10 @@ struct NearArgs {
     int leaf_class_off[NEAR_CLASSES + 1];
     int kf32;                   // dense leaves: kernel values in FP32 (mixed modes)
     int all;                    // columns of the whole call (of which ncols run now)
-    int max_leaf, passes;       // points of the largest leaf; passes over the last class (the launcher's)
+    // passes over 64 targets each of the last class: (leaf, pass) in passes, or
+    // nullptr where none of its leaves holds more (npass: its leaves)
+    const int2 *passes;
+    int npass;
 };
 
 struct DirectArgs {
@@ -299,7 +302,8 @@ struct NearGradArgs {
     const double *Fs, *Fp;      // leaf expansions [leaf][col][n3] of sig (forward) and psi (transposed), or nullptr
     const int32_t *leaf_class;  // as in NearArgs
     int leaf_class_off[NEAR_CLASSES + 1];
-    int max_leaf, passes;
+    const int2 *passes;
+    int npass;
     double *grad;               // AoS N x 3, caller's order, accumulated
 };
 

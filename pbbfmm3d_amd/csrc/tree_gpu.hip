@@ -283,19 +283,20 @@ __global__ __launch_bounds__(TPB) void box_emit(const int32_t *__restrict__ psta
 }
 
 // near-field class of every leaf (class c: at most 2 << c points; the last
-// class takes the rest), its histogram, the largest leaf and the ordered
-// near-field point pairs
+// class takes the rest), its histogram, the largest leaf, the ordered
+// near-field point pairs (count[0]) and the last class's passes of 64 targets
+// (count[1])
 __global__ __launch_bounds__(TPB) void leaf_stats(const int32_t *__restrict__ leaf_start, const int32_t *__restrict__ coord,
                                                   const int32_t *__restrict__ map, int64_t nb, int levels,
                                                   uint32_t *__restrict__ cls, int32_t *__restrict__ ids,
                                                   unsigned long long *__restrict__ hist, int *__restrict__ max_leaf,
-                                                  unsigned long long *__restrict__ near_pairs)
+                                                  unsigned long long *__restrict__ count)
 {
     __shared__ unsigned sh[8];
     if (threadIdx.x < 8) sh[threadIdx.x] = 0;
     __syncthreads();
     const int64_t S = 1LL << levels;
-    unsigned long long q = 0;
+    unsigned long long q = 0, np = 0;
     int mx = 0;
     for (int64_t b = blockIdx.x * (int64_t)TPB + threadIdx.x; b < nb; b += (int64_t)gridDim.x * TPB) {
         const int nt = leaf_start[b + 1] - leaf_start[b];
@@ -305,6 +306,7 @@ __global__ __launch_bounds__(TPB) void leaf_stats(const int32_t *__restrict__ le
         ids[b] = (int32_t)b;
         atomicAdd(&sh[c], 1u);
         mx = max(mx, nt);
+        if (c == NEAR_CLASSES - 1) np += (nt + 63) / 64;
         const int32_t cc = coord[b];
         const int64_t ix = cc & 1023, iy = (cc >> 10) & 1023, iz = (cc >> 20) & 1023;
         for (int dx = -1; dx <= 1; dx++)
@@ -318,14 +320,32 @@ __global__ __launch_bounds__(TPB) void leaf_stats(const int32_t *__restrict__ le
     }
     for (int o = 32; o > 0; o >>= 1) {
         q += __shfl_xor(q, o);
+        np += __shfl_xor(np, o);
         mx = max(mx, __shfl_xor(mx, o));
     }
     if ((threadIdx.x & 63) == 0) {
-        if (q) atomicAdd(near_pairs, q);
+        if (q) atomicAdd(&count[0], q);
+        if (np) atomicAdd(&count[1], np);
         atomicMax(max_leaf, mx);
     }
     __syncthreads();
     if (threadIdx.x < 8 && sh[threadIdx.x]) atomicAdd(&hist[threadIdx.x], (unsigned long long)sh[threadIdx.x]);
+}
+
+// passes of 64 targets of the last class's leaves (element n is zero), and
+// the list of them from their exclusive sums
+__global__ __launch_bounds__(TPB) void pass_counts(const int32_t *__restrict__ leaf, int64_t n,
+                                                   const int32_t *__restrict__ leaf_start, int *__restrict__ cnt)
+{
+    for (int64_t q = blockIdx.x * (int64_t)TPB + threadIdx.x; q <= n; q += (int64_t)gridDim.x * TPB)
+        cnt[q] = q < n ? (leaf_start[leaf[q] + 1] - leaf_start[leaf[q]] + 63) / 64 : 0;
+}
+
+__global__ __launch_bounds__(TPB) void pass_emit(const int32_t *__restrict__ leaf, int64_t n,
+                                                 const int *__restrict__ first, int2 *__restrict__ list)
+{
+    for (int64_t q = blockIdx.x * (int64_t)TPB + threadIdx.x; q < n; q += (int64_t)gridDim.x * TPB)
+        for (int k = first[q]; k < first[q + 1]; k++) list[k] = int2{leaf[q], k - first[q]};
 }
 
 // far-field (target, source) box pairs of one level: the 189 offsets of
@@ -708,12 +728,27 @@ void build_tree_gpu(GpuTree &T, const double *xyz_host, int64_t N, int64_t nbox,
                                                                   lpairs + l);
         check(hipGetLastError(), "m2l_pair_count");
     }
-    unsigned long long hc[2], hl[16];
+    unsigned long long hc[3], hl[16];
     check(hipMemcpyAsync(hc, cnt, sizeof(hc), hipMemcpyDeviceToHost, st), "copy counters");
     check(hipMemcpyAsync(hl, lpairs, sizeof(hl), hipMemcpyDeviceToHost, st), "copy pair counters");
     check(hipStreamSynchronize(st), "hipStreamSynchronize");
     T.outside = (int64_t)hc[0];
     T.near_pairs = (int64_t)hc[1];
+    const int big0 = T.leaf_class_off[NEAR_CLASSES - 1], big = T.leaf_class_off[NEAR_CLASSES] - big0;
+    if (hc[2] > INT32_MAX) fail(PBB_ERR_UNSUPPORTED, "too many near-field passes");
+    T.n_near_passes = (int)hc[2];
+    if (T.n_near_passes > big) {
+        const int32_t *leaf = T.leaf_class + big0;
+        int *counts = pool.carve<int>((size_t)big + 1, "pass counts"), *first = pool.carve<int>((size_t)big + 1, "passes");
+        pass_counts<<<nblocks(big + 1), TPB, 0, st>>>(leaf, big, T.leaf_start, counts);
+        check(hipGetLastError(), "pass_counts");
+        size_t b = 0;
+        check(hipcub::DeviceScan::ExclusiveSum(nullptr, b, counts, first, big + 1, st), "scan size");
+        check(hipcub::DeviceScan::ExclusiveSum(tmp.need(b), b, counts, first, big + 1, st), "scan");
+        T.near_passes = pool.get<int2>(T.n_near_passes, "near-field passes");
+        pass_emit<<<nblocks(big), TPB, 0, st>>>(leaf, big, first, T.near_passes);
+        check(hipGetLastError(), "pass_emit");
+    }
     T.m2l_pairs = 0;
     for (int l = 2; l <= levels; l++) {
         T.m2l_pairs_level[l] = (int64_t)hl[l];
@@ -722,8 +757,8 @@ void build_tree_gpu(GpuTree &T, const double *xyz_host, int64_t N, int64_t nbox,
 
     // hand the tree's arrays over; everything else is freed with the pool
     for (void *p : {(void *)T.x, (void *)T.y, (void *)T.z, (void *)T.perm, (void *)T.pt_leaf, (void *)T.leaf_start,
-                    (void *)T.leaf_class, (void *)T.up_items, (void *)T.up_reds})
-        pool.keep(p);
+                    (void *)T.leaf_class, (void *)T.near_passes, (void *)T.up_items, (void *)T.up_reds})
+        if (p) pool.keep(p);
     for (auto &V : T.lv)
         for (void *p : {(void *)V.coord, (void *)V.map, (void *)V.child, (void *)V.order, (void *)V.pstart,
                         (void *)V.seg_box, (void *)V.seg_p0})

@@ -32,6 +32,8 @@ struct GpuTree {
     int32_t *leaf_start = nullptr;                    // leaves + 1
     int32_t *leaf_class = nullptr;                    // leaves grouped by near-field class
     int leaf_class_off[NEAR_CLASSES + 1] = {0};
+    int2 *near_passes = nullptr;                      // (leaf, pass) of the last class (nullptr: one pass a leaf)
+    int n_near_passes = 0;
     int4 *up_items = nullptr, *up_reds = nullptr;
     int n_up_items = 0, n_up_reds = 0, n_up_slots = 0;
     std::vector<GpuLevel> lv;                         // 0..Lv
