@@ -2960,8 +2960,9 @@ PBB_API pbb_status pbb_direct_sum(const pbb_kernel_desc *kernel, const double *t
         hipStream_t st = (hipStream_t)stream;
         dev::DirectArgs a{};
         a.T = ntargets; a.Ns = nsources; a.ncols = ncols;
-        // workgroups of 64 targets and one slice of the sources: 4096 and more
-        // keep the last round of the 256 CUs (two workgroups each) short;
+        // workgroups of 64 targets and one slice of the sources: about 4096
+        // (and one slice from there on) keep the last round of the 256 CUs, two
+        // workgroups each, short;
         // slices of fewer than 512 sources leave a wave less than its reduction
         const int64_t tblocks = (ntargets + 63) / 64;
         a.nsplit = (int)std::min<int64_t>(256, std::max<int64_t>(1, 4096 / std::max<int64_t>(1, tblocks)));

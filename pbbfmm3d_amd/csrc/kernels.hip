@@ -1856,7 +1856,7 @@ __global__ __launch_bounds__(64 * DS_WAVES) void direct_partial(DirectArgs a, in
 {
     __shared__ double sh[DS_WAVES][DS_TGT];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t i = (int64_t)blockIdx.x * DS_TGT + lane;
+    const int64_t i = a.t0 + (int64_t)blockIdx.x * DS_TGT + lane;
     const int split = blockIdx.y;
     const int64_t per = (a.Ns + a.nsplit - 1) / a.nsplit;
     const int64_t s0 = split * per, s1 = min(a.Ns, s0 + per);
@@ -2169,12 +2169,17 @@ bool launch_l2p_level(const DownArgs &a, int nseg, hipStream_t st)
     return true;
 }
 
-void launch_direct(const DirectArgs &a, int kid, hipStream_t st)
+void launch_direct(const DirectArgs &args, int kid, hipStream_t st)
 {
+    DirectArgs a = args;
     if (a.T <= 0) return;
-    dim3 grid((unsigned)((a.T + DS_TGT - 1) / DS_TGT), (unsigned)a.nsplit);
-    for (int c0 = 0; c0 < a.ncols; c0 += 16) {
-        const int cn = a.ncols - c0;
+    // ranges of targets: a launch holds fewer than 2^32 threads, 16 a target
+    constexpr int64_t RANGE = (int64_t)DS_TGT << 21;
+    const int ncg = (a.ncols + 15) / 16;
+    for (int64_t k = 0, n = (a.T + RANGE - 1) / RANGE * ncg; k < n; k++) {
+        const int c0 = (int)(k % ncg) * 16, cn = a.ncols - c0;
+        a.t0 = k / ncg * RANGE;
+        dim3 grid((unsigned)((std::min(RANGE, a.T - a.t0) + DS_TGT - 1) / DS_TGT), (unsigned)a.nsplit);
 #define PBB_DIRECT_CASE(K)                                                                   \
     case K:                                                                                  \
         if (cn <= 1) direct_partial<K, 1><<<grid, 64 * DS_WAVES, 0, st>>>(a, c0);            \

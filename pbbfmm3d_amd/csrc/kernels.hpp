@@ -264,6 +264,7 @@ struct NearArgs {
 
 struct DirectArgs {
     int64_t T, Ns;
+    int64_t t0;                    // first target of the launch (the launcher's)
     int ncols, nsplit;
     KParams kp;
     const double *tgt, *src, *w;   // AoS targets / sources, column-major weights

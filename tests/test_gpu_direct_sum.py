@@ -54,3 +54,28 @@ def test_range_of_the_inverse_root(gpu, name, r):
         want = f(np.float64(r) ** 2)
     want = 0.0 if np.isinf(want) else want
     assert np.isnan(got) if np.isnan(want) else abs(got - want) <= 4 * 2.0**-52 * abs(want)
+
+
+def test_more_targets_than_one_launch_holds(gpu):
+    """2^28 + 65 targets at 16 threads each: more than the 2^32 - 1 threads of
+    a launch, and the remainders of a workgroup and of a range of targets."""
+    import ctypes as C
+
+    import torch
+    from pbbfmm3d_amd import _capi as capi
+    nt = 2**28 + 65
+    print(f"case nt={nt}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    t = torch.rand(nt, 3, dtype=torch.float64, device="cuda", generator=g)
+    s = torch.tensor([[0.25, 0.5, 0.75], [0.5, -1.0, 2.0]], dtype=torch.float64, device="cuda")
+    w = torch.tensor([[1.0, -3.0]], dtype=torch.float64, device="cuda")
+    out = torch.full((nt,), -1.0, dtype=torch.float64, device="cuda")
+    d = pbb.quadric().desc()
+    capi.check(capi.lib().pbb_direct_sum(C.byref(d), t.data_ptr(), nt, s.data_ptr(), 2, w.data_ptr(), 1,
+                                         out.data_ptr(), None))
+    torch.cuda.synchronize()
+    for i in range(0, nt, 2**25):
+        x = t[i:i + 2**25]
+        k = [1 + ((x - s[j]) ** 2).sum(1) for j in (0, 1)]
+        bound = 2 * (2 + 32) * 2.0**-53 * (k[0] + 3 * k[1])
+        assert bool(((out[i:i + 2**25] - (k[0] - 3 * k[1])).abs() <= bound).all())
