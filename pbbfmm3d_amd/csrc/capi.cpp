@@ -425,7 +425,8 @@ struct pbb_ops {
 
     // Set s: bases C_f, C_s of the columns of U and V, A = C_f^T U and
     // B = C_s^T V; the orbits' blocks from A E_d B^T, averaged over the
-    // reflections; kept when A^T K_d B gives every E_d back to rounding.
+    // reflections; kept when X^T K_d Y (their pseudo-inverses) gives every E_d
+    // back to rounding.
     bool make_sym_set(int s, double tau, hipStream_t st)
     {
         const int n3 = h.n3, rf = h.rf, rs = h.rs;
@@ -494,7 +495,7 @@ struct pbb_ops {
         double *dK = tmp.take(K.size()), *part = tmp.take(2 * 1024);
         const int *dcf = tmp.put(F.cls.data(), tf), *dcs = tmp.put(S.cls.data(), ts);
         const int *ddir = tmp.put(dir, 56 * 8), *dof = tmp.put(of, 316), *dre = tmp.put(refl, 316);
-        const std::vector<double> At = transposed(F.A, tf, rf), Bt = transposed(S.A, ts, rs);
+        const std::vector<double> At = transposed(F.X, tf, rf), Bt = transposed(S.X, ts, rs);
         const double *dA = tmp.put(F.A.data(), F.A.size()), *dB = tmp.put(S.A.data(), S.A.size());
         const double *dAt = tmp.put(At.data(), At.size()), *dBt = tmp.put(Bt.data(), Bt.size());
         const double *dE = d_E + (size_t)s * 316 * rf * rs;
@@ -512,9 +513,9 @@ struct pbb_ops {
         sym_complete(F, S, rf, rs, K.data(), 56);
         check(hipMemcpyAsync(dK, K.data(), K.size() * sizeof(double), hipMemcpyHostToDevice, st), "copy blocks");
         dev::launch_sym_expand(dK, dcf, dcs, tf, ts, dof, dre, X, st);
-        gemm(dAt, rf, tf, X, (int64_t)316 * ts, Y);           // A^T K_d
+        gemm(dAt, rf, tf, X, (int64_t)316 * ts, Y);           // X^T K_d
         dev::launch_transpose_blocks(Y, rf, ts, 316, X, st);
-        gemm(dBt, rs, ts, X, (int64_t)316 * rf, Y);           // (A^T K_d B)^T
+        gemm(dBt, rs, ts, X, (int64_t)316 * rf, Y);           // (X^T K_d Y)^T
         dev::launch_transpose_blocks(Y, rs, rf, 316, X, st);
         // the operators themselves hold the symmetry to a few 1e-14 of their norm
         const double err = device_rel_diff(X, dE, (int64_t)316 * rf * rs, part, st);
@@ -539,12 +540,12 @@ struct pbb_ops {
             for (int p = 0; p < 8; p++) {
                 for (int i = 0; i < S.cnt[p]; i++) {
                     double v = 0;
-                    for (int b = 0; b < rs; b++) v += S.A[cbase[p] + i + (size_t)b * ts] * VT[b + (size_t)x * rs];
+                    for (int b = 0; b < rs; b++) v += S.X[cbase[p] + i + (size_t)b * ts] * VT[b + (size_t)x * rs];
                     VTs[4 * q.kb[p] + i + (size_t)x * q.nk] = v * h.w.Kw[x];
                 }
                 for (int i = 0; i < F.cnt[p]; i++) {
                     double v = 0;
-                    for (int a = 0; a < rf; a++) v += F.A[rbase[p] + i + (size_t)a * tf] * U[x + (size_t)a * n3];
+                    for (int a = 0; a < rf; a++) v += F.X[rbase[p] + i + (size_t)a * tf] * U[x + (size_t)a * n3];
                     Us[x + (size_t)dev::sym_row(q.shape, p, i) * n3] = v * h.w.Kw[x];
                 }
             }

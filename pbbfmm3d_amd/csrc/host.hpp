@@ -106,12 +106,13 @@ void reduce_set(const HostOps &ops, int set, const double *VTw, const double *Uw
 
 // ---- reflection symmetry of an operator set (symm.cpp) ----------------------
 // One side's basis of pure parity: rt columns ordered by class (bits x 4, y 2,
-// z 1; set = odd), cnt of each class, A = C^T U (rt x r, column-major).
+// z 1; set = odd), cnt of each class, A = C^T U (rt x r, column-major) and X,
+// A's pseudo-inverse transposed: U ~ C A and U X^T ~ C.
 struct SymSide {
     int rt = 0;
     int cnt[8] = {0};
     std::vector<int> cls;   // class of every column
-    std::vector<double> A;
+    std::vector<double> A, X;
 };
 // Finds the basis of the columns of U (n3 x r), each weighted with w, to
 // within tau of the weighted Frobenius norm; false when more than max_rt

@@ -8,6 +8,12 @@
 // columns C (n3 x rt, orthonormal, each of one parity class) and A = C^T U,
 // with U ~ C A.  A cluster cut by the rank gives a few more columns than the
 // rank, directions of singular values at the rounding level give fewer.
+//
+// The way back is A's pseudo-inverse, not A^T: the singular vectors of the
+// precompute are orthonormal to 1e-14 at order 4 and 2e-13 at order 6 only, and
+// the operators rebuilt with A^T carry that error (order 4 1.3e-14 of their
+// norm, order 6 8.7e-14; with the pseudo-inverse 1.1e-15 and 7.0e-15, the
+// rounding of the operators themselves).
 #include <algorithm>
 #include <cmath>
 
@@ -100,6 +106,27 @@ bool sym_side(int n, int r, const double *U, const double *w, double tau, int ma
             out.cls.push_back(p);
             at++;
         }
+    // X = (2 - A A^T) A: the singular values of A are 1 to the rounding of U,
+    // or 0 (directions of U that no column holds): s (2 - s^2) is 1 / s there
+    const int rt = out.rt;
+    std::vector<double> G((size_t)rt * rt);
+    out.X.assign((size_t)rt * r, 0.0);
+    const double *A = out.A.data();
+    parallel_for(rt, [&](int64_t j) {
+        double *g = &G[(size_t)j * rt];
+        for (int c = 0; c < r; c++) {
+            const double *a = A + (size_t)c * rt;
+            for (int i = 0; i < rt; i++) g[i] -= a[i] * a[j];
+        }
+        g[j] += 2.0;
+    });
+    parallel_for(r, [&](int64_t c) {
+        double *x = &out.X[(size_t)c * rt];
+        for (int j = 0; j < rt; j++) {
+            const double a = A[j + (size_t)c * rt], *g = &G[(size_t)j * rt];
+            for (int i = 0; i < rt; i++) x[i] += g[i] * a;
+        }
+    });
     return true;
 }
 
@@ -147,7 +174,7 @@ static void solve_full_pivot(std::vector<double> &T, std::vector<double> &b, int
 
 void sym_complete(const SymSide &f, const SymSide &s, int rf, int rs, double *M, int nblocks)
 {
-    // P = A A^T of each side: the identity but on the columns a cut cluster
+    // P = A X^T of each side: the identity but on the columns a cut cluster
     // added, of which the operators hold a projection only.  M holds
     // avg_R (D_R P D_R) K (D_R P' D_R); those rows and columns are undone.
     constexpr int DEF_MAX = 10;
@@ -155,7 +182,7 @@ void sym_complete(const SymSide &f, const SymSide &s, int rf, int rs, double *M,
         P.assign((size_t)q.rt * q.rt, 0.0);
         for (int c = 0; c < r; c++)
             for (int j = 0; j < q.rt; j++) {
-                const double v = q.A[j + (size_t)c * q.rt];
+                const double v = q.X[j + (size_t)c * q.rt];
                 for (int i = 0; i < q.rt; i++) P[i + (size_t)j * q.rt] += q.A[i + (size_t)c * q.rt] * v;
             }
         for (int i = 0; i < q.rt; i++) {
