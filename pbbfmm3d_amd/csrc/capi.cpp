@@ -769,15 +769,16 @@ struct pbb_plan {
 };
 
 // ---- the FP64 M2L in the reflection-adapted bases ---------------------------
-// The set of level l's M2L, or nullptr where the level keeps the set's own
-// factors (no bases of pure parity within the bounds of make_sym_set).  Where
+// The set of level l's M2L in a pass of ncols columns, or nullptr where the
+// level keeps the set's own factors: no bases of pure parity within the bounds
+// of make_sym_set, or more proxies than its offsets reach.  Where
 // they exist they were faster down to the smallest plan measured (1M points,
 // 8 columns 293 -> 78 ms; 5k points, 1 column 1.77 -> 0.42 ms per matvec).
-static const SymSet *sym_level(const pbb_plan &p, const pbb_ops *o, int l)
+static const SymSet *sym_level(const pbb_plan &p, const pbb_ops *o, int l, int ncols)
 {
     if (!o->sym_ready.load(std::memory_order_acquire) || o->fp64_reduced) return nullptr;
     const SymSet &q = o->sym[o->h.ops_set(l)];
-    return q.ok ? &q : nullptr;
+    return q.ok && sym_level_fits(p.lv[l].nb, ncols, q.nk) ? &q : nullptr;
 }
 
 // Tile and sum parts of a level's M2L for ncols of the call's `all` columns.
@@ -836,7 +837,7 @@ static FarDims far_dims(const pbb_plan &p, const pbb_ops *o, int ncols, int all,
     const int rmax = std::max(o->h.rf, o->h.rs);
     d.ldp = d.ldf = rmax;
     for (int l = 2; sym && l <= p.Lv; l++) {
-        const SymSet *q = sym_level(p, o, l);
+        const SymSet *q = sym_level(p, o, l, ncols);
         if (!q) continue;
         d.sym = true;
         d.ldp = std::max(d.ldp, q->nk);
@@ -1810,7 +1811,8 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
 // One matvec of the plan's operator set o in its own workspace.
 // Columns are independent: when the workspace of all ncols columns does not
 // fit beside what the device already holds, the matvec runs over chunks of
-// columns, each a complete FMM pass (the same sums, so the same results).
+// columns, each a complete FMM pass (the same sums, so the same results); so it
+// does when a level's proxies are more than its M2L addresses.
 // A pass that keeps its expansions for the caller (keep: the complete leaf
 // expansions in W.S; out may be nullptr) is not split.
 static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, double *out, hipStream_t st, int prec,
@@ -1832,6 +1834,8 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
         }
     }
     if (!keep) {
+        for (int l = 2; sym && l <= p->Lv; l++)
+            if (const SymSet *q = sym_level(*p, o, l, 1)) chunk = sym_columns(p->lv[l].nb, chunk, q->nk);
         Workspace tmp;
         size_t need = layout_workspace(*p, chunk, mixed, far_dims(*p, o, chunk, ncols, sym), nullptr, tmp);
         if (need > p->ws_bytes || (p->ws_limit && need > p->ws_limit)) {
@@ -2094,7 +2098,7 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
     const bool split_acc = split_acc_on(p, prec);
     const pbb_plan::M2LTile &tmx = p->m2l_tile[1];
     const int ldP = mixed ? W.kpad : h.rs;
-    auto sym_of = [&](int l) -> const SymSet * { return !mixed && W.sym ? sym_level(*p, o, l) : nullptr; };
+    auto sym_of = [&](int l) -> const SymSet * { return !mixed && W.sym ? sym_level(*p, o, l, ncols) : nullptr; };
     if (mixed && h.rs > W.kpad) fail(PBB_ERR_INTERNAL, "proxy padding too small");
     mark(0);
     // orders 4..8 run the direct passes: P2M at every level instead of

@@ -123,6 +123,17 @@ bool sym_side(int n, int r, const double *U, const double *w, double tau, int ma
 // the rank added to the bases.
 void sym_complete(const SymSide &f, const SymSide &s, int rf, int rs, double *M, int nblocks);
 
+// The M2L of an adapted set holds source offsets in 32 bits, in units of 16
+// bytes: a level's boxes (and the box of zeros) x columns x nk proxies stay
+// below 64 GB.  sym_columns: the columns of a pass, ncols halved until they do
+// (1 where not even one column does: such a level keeps its own factors).
+constexpr bool sym_level_fits(int64_t nb, int64_t ncols, int64_t nk) { return (nb + 1) * ncols * nk / 2 <= UINT32_MAX; }
+constexpr int sym_columns(int64_t nb, int ncols, int64_t nk)
+{
+    while (ncols > 1 && !sym_level_fits(nb, ncols, nk)) ncols = (ncols + 1) / 2;
+    return ncols;
+}
+
 // Orbits of the 316 far directions under the axis reflections.  pm, zm: the
 // axes whose component is 1 or 2 (both signs occur), and 0; slot: the first
 // of the orbit's directions among the 189 of a class.

@@ -546,8 +546,7 @@ void launch_m2l_sym(const SymArgs &args, const SymShape &s, int ncolchunks, hipS
     if (a.class_start[8] <= 0) return;
     if (a.TB < 1 || a.TB > SYM_TB || a.TB * a.cpt > sym_width(s) || (a.npz & (a.npz - 1)) != 0)
         fail(PBB_ERR_INTERNAL, "M2L tile does not fit its workgroup");
-    if ((a.class_start[8] + 1) * a.ncols * a.ldp / 2 > UINT32_MAX)
-        fail(PBB_ERR_INTERNAL, "M2L level of more than 64 GB of proxies");
+    if (!sym_level_fits(a.class_start[8], a.ncols, a.ldp)) fail(PBB_ERR_INTERNAL, "M2L level of more than 64 GB of proxies");
     const int most = *std::max_element(a.class_tiles, a.class_tiles + 8);
     dim3 grid((unsigned)most * 8, (unsigned)ncolchunks, (unsigned)(a.nrow * a.npz * a.noz));
     // orbits to a barrier: what LDS holds beside the table at the workgroups
