@@ -1808,13 +1808,26 @@ static PointIo point_io(const pbb_plan *p, const pbb_ops *o)
 static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double *w, int ncols, double *out,
                        hipStream_t st, int prec, bool build, bool keep = false);
 
+// Device memory that workspaces of `held` bytes may grow to.  They stay after
+// the call, so the caller is left a sixteenth of the device (at least 1 GiB)
+// for its own allocations.
+static size_t device_room(size_t held, size_t *free_bytes = nullptr)
+{
+    size_t free_b = 0, total_b = 0;
+    check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    if (free_bytes) *free_bytes = free_b;
+    return held + free_b - std::min(free_b, std::max((size_t)(1ull << 30), total_b / 16));
+}
+
 // One matvec of the plan's operator set o in its own workspace.
 // Columns are independent: when the workspace of all ncols columns does not
 // fit beside what the device already holds, the matvec runs over chunks of
 // columns, each a complete FMM pass (the same sums, so the same results); so it
 // does when a level's proxies are more than its M2L addresses.
 // A pass that keeps its expansions for the caller (keep: the complete leaf
-// expansions in W.S; out may be nullptr) is not split.
+// expansions in W.S; out may be nullptr) is not split; like a single column, it
+// takes the sets' own factors, whose rows are not padded, where the adapted
+// sets' workspace does not fit.
 static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, double *out, hipStream_t st, int prec,
                        bool keep = false)
 {
@@ -1833,24 +1846,23 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
             }
         }
     }
-    if (!keep) {
+    Workspace tmp;
+    auto bytes = [&] { return layout_workspace(*p, chunk, mixed, far_dims(*p, o, chunk, ncols, sym), nullptr, tmp); };
+    if (keep) {
+        const size_t need = sym ? bytes() : 0;
+        if (need > p->ws_bytes && need > device_room(p->ws_bytes)) sym = false;
+    } else {
         for (int l = 2; sym && l <= p->Lv; l++)
             if (const SymSet *q = sym_level(*p, o, l, 1)) chunk = sym_columns(p->lv[l].nb, chunk, q->nk);
-        Workspace tmp;
-        size_t need = layout_workspace(*p, chunk, mixed, far_dims(*p, o, chunk, ncols, sym), nullptr, tmp);
+        size_t need = bytes();
         if (need > p->ws_bytes || (p->ws_limit && need > p->ws_limit)) {
-            size_t free_b = 0, total_b = 0;
-            check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-            // The workspace stays with the plan after the call, so leave the
-            // caller a sixteenth of the device (at least 1 GiB) for its own
-            // allocations.
-            const size_t margin = std::max((size_t)(1ull << 30), total_b / 16);
-            size_t room = p->ws_bytes + free_b - std::min(free_b, margin);
+            size_t free_b = 0, room = device_room(p->ws_bytes, &free_b);
             if (p->ws_limit) room = std::min(room, p->ws_limit);
             while (chunk > 1 && need > room) {
                 chunk = (chunk + 1) / 2;
-                need = layout_workspace(*p, chunk, mixed, far_dims(*p, o, chunk, ncols, sym), nullptr, tmp);
+                need = bytes();
             }
+            if (need > p->ws_bytes + free_b) sym = false;
         }
     }
     for (int c0 = 0; c0 < ncols; c0 += chunk) {
@@ -2623,13 +2635,9 @@ static int64_t kept_doubles(pbb_plan *p, int ncols, int prec)
     if (sym) p->ops->ensure_sym((hipStream_t)0);
     Workspace tmp;
     const size_t need = layout_workspace(*p, ncols, false, far_dims(*p, p->ops, ncols, ncols, sym), nullptr, tmp);
-    size_t free_b = 0, total_b = 0;
-    check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-    const size_t margin = std::max((size_t)(1ull << 30), total_b / 16);
-    const size_t grow = need > p->ws_bytes ? need - p->ws_bytes : 0;
     // twice the expansions: the caller's allocator may hold a freed buffer of the
     // last step where this step's gradient has to make its own
-    return grow + 2 * (size_t)n * sizeof(double) + margin <= free_b ? n : 0;
+    return std::max(need, p->ws_bytes) + 2 * (size_t)n * sizeof(double) <= device_room(p->ws_bytes) ? n : 0;
 }
 
 PBB_API pbb_status pbb_plan_kept_size(pbb_plan *plan, int32_t ncols, int32_t precision, int64_t *count)
@@ -2835,22 +2843,29 @@ static void batch_create(const pbb_batch_entry *E, int nplans, int ncols, int pr
                 break;
             }
     }
+    auto first_of = [&](int i) { return (int)(std::find(plans.begin(), plans.end(), plans[i]) - plans.begin()); };
+    auto bytes = [&](int i) {
+        Workspace tmp;
+        return layout_workspace(*plans[i], ncols, mixed, dims[i], nullptr, tmp);
+    };
+    size_t total = 0;
+    bool any_sym = false;
+    for (int i = 0; i < nplans; i++)
+        if (first_of(i) == i) {
+            total += bytes(i);
+            any_sym |= dims[i].sym;
+        }
+    // workspaces that fit only without the adapted sets' padded rows: the own
+    // factors for all
+    if (any_sym && total > device_room(0))
+        for (int i = 0; i < nplans; i++) dims[i] = far_dims(*plans[i], ops[i], ncols, ncols, false);
     for (int i = 0; i < nplans; i++) {
-        pbb_plan *p = plans[i];
-        int first = i;
-        for (int k = 0; k < i; k++)
-            if (plans[k] == p) {
-                first = k;
-                break;
-            }
-        if (first < i) {
-            wsp[i] = wsp[first];
+        if (first_of(i) < i) {
+            wsp[i] = wsp[first_of(i)];
             continue;
         }
-        Workspace tmp;
-        const size_t need = layout_workspace(*p, ncols, mixed, dims[i], nullptr, tmp);
-        b->blocks.push_back(dalloc<char>(need, "batch workspace"));
-        layout_workspace(*p, ncols, mixed, dims[i], b->blocks.back(), wsp[i]);
+        b->blocks.push_back(dalloc<char>(bytes(i), "batch workspace"));
+        layout_workspace(*plans[i], ncols, mixed, dims[i], b->blocks.back(), wsp[i]);
     }
     check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
     // independent entries run as concurrent graph branches.  Entries
