@@ -156,10 +156,12 @@ static double device_rel_diff(const double *a, const double *b, int64_t n, doubl
 struct pbb_ops {
     HostOps h;
     std::mutex mu;
-    // the FP64 mode's reflection-adapted sets, made by its first matvec
-    // (sym_ready: done; a set without the symmetry keeps ok = false)
+    // the FP64 mode's reflection-adapted sets, made by its first matvec with
+    // the memory for it (sym_ready: done; a set without the symmetry keeps
+    // ok = false)
     std::vector<SymSet> sym;
     std::atomic<bool> sym_ready{false};
+    int sym_failed = 0;  // attempts that ran out of memory all the same
     int device = -1;
     std::unique_ptr<pbb_ops> adj;  // transposed operator set, built on demand
     double *d_Tkz = nullptr, *d_Cw = nullptr, *d_VTw = nullptr, *d_Uw = nullptr, *d_E = nullptr;
@@ -395,12 +397,21 @@ struct pbb_ops {
         d_E = dupload(h.E, "E");
         device = dev;
     }
-    // Makes the reflection-adapted sets (allocates and waits for st).
+    // Makes the reflection-adapted sets (allocates and waits for st).  Without
+    // the memory for it the call runs the sets' own factors and a later one
+    // tries again: the 1 GiB left free is more than the attempt's estimate can
+    // be short by, so a third failure means that other work takes the memory as
+    // the sets are made, and ends it.
     void ensure_sym(hipStream_t st)
     {
         if (sym_ready.load(std::memory_order_acquire)) return;
         std::lock_guard<std::mutex> lk(mu);
         if (sym_ready.load(std::memory_order_relaxed)) return;
+        // the operators of one set twice at the padded ranks, and its blocks
+        const size_t tm = std::max(h.rf, h.rs) + 8, temps = (2 * 316 + 56) * tm * tm * sizeof(double);
+        size_t free_b = 0, total_b = 0;
+        check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        if (free_b < temps + (1ull << 30)) return;
         sym.assign(h.nsets, SymSet{});
         try {
             dev::upload_sym_orbits();
@@ -417,8 +428,8 @@ struct pbb_ops {
                 dfree(q.Ef);
                 q = SymSet{};
             }
-            // no room beside what the device holds: the sets' own factors serve
             if (e.status != PBB_ERR_OUT_OF_MEMORY) throw;
+            if (++sym_failed < 3) return;
         }
         sym_ready.store(true, std::memory_order_release);
     }
@@ -1842,7 +1853,7 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
             check(hipStreamIsCapturing(st, &cs), "hipStreamIsCapturing");
             if (cs == hipStreamCaptureStatusNone) {
                 o->ensure_sym(st);
-                sym = true;
+                sym = o->sym_ready.load(std::memory_order_acquire);
             }
         }
     }
@@ -2828,6 +2839,7 @@ static void batch_create(const pbb_batch_entry *E, int nplans, int ncols, int pr
     std::vector<pbb_ops *> ops(nplans);
     std::vector<Workspace> wsp(nplans);
     std::vector<FarDims> dims(nplans);  // of a plan's first entry: what all its entries need
+    std::vector<char> adapted(nplans);  // whether the entry runs adapted sets in it
     for (int i = 0; i < nplans; i++) {
         pbb_plan *p = plans[i];
         ops[i] = (E[i].flags & PBB_BATCH_TRANSPOSE) ? p->ops->adjoint() : p->ops;
@@ -2837,6 +2849,7 @@ static void batch_create(const pbb_batch_entry *E, int nplans, int ncols, int pr
         split_ops(p, ops[i], precision, true, b->stream, se, sa);
         if (!mixed && p->Lv >= 2 && !ops[i]->fp64_reduced) ops[i]->ensure_sym(b->stream);
         dims[i] = far_dims(*p, ops[i], ncols, ncols, !mixed);
+        adapted[i] = dims[i].sym;
         for (int k = 0; k < i; k++)
             if (plans[k] == p) {
                 dims[k] = merge(dims[k], dims[i]);
@@ -2858,14 +2871,19 @@ static void batch_create(const pbb_batch_entry *E, int nplans, int ncols, int pr
     // workspaces that fit only without the adapted sets' padded rows: the own
     // factors for all
     if (any_sym && total > device_room(0))
-        for (int i = 0; i < nplans; i++) dims[i] = far_dims(*plans[i], ops[i], ncols, ncols, false);
+        for (int i = 0; i < nplans; i++) {
+            dims[i] = far_dims(*plans[i], ops[i], ncols, ncols, false);
+            adapted[i] = 0;
+        }
     for (int i = 0; i < nplans; i++) {
         if (first_of(i) < i) {
             wsp[i] = wsp[first_of(i)];
-            continue;
+        } else {
+            b->blocks.push_back(dalloc<char>(bytes(i), "batch workspace"));
+            layout_workspace(*plans[i], ncols, mixed, dims[i], b->blocks.back(), wsp[i]);
         }
-        b->blocks.push_back(dalloc<char>(bytes(i), "batch workspace"));
-        layout_workspace(*plans[i], ncols, mixed, dims[i], b->blocks.back(), wsp[i]);
+        // (sets made since the layout stay out of it)
+        wsp[i].sym = adapted[i] != 0;
     }
     check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
     // independent entries run as concurrent graph branches.  Entries

@@ -1,5 +1,7 @@
 """Calls on a device with no room for the padded rows of the reflection-adapted
-sets: passes that cannot run in column chunks take the sets' own factors."""
+sets: passes that cannot run in column chunks take the sets' own factors.  And
+without the memory to make the sets, a matvec runs the own factors until a later
+one has it."""
 import contextlib
 import ctypes as C
 
@@ -13,16 +15,17 @@ pytestmark = pytest.mark.gpu
 
 
 @contextlib.contextmanager
-def _filled():
-    """64 MB less free than what workspaces leave to the caller (a sixteenth
-    of the device, so that every allocation of the tests still succeeds)."""
+def _filled(left=None):
+    """64 MB less free than `left` bytes, by default what workspaces leave to
+    the caller, a sixteenth of the device (every allocation of the tests still
+    succeeds)."""
     import torch
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     held = []
     for _ in range(4):  # (the free memory reported after an allocation of this size is not exact)
         free, total = torch.cuda.mem_get_info()
-        more = free - max(1 << 30, total // 16) + (64 << 20)
+        more = free - (left or max(1 << 30, total // 16)) + (64 << 20)
         if more > 0:
             held.append(torch.empty(max(more, 32 << 20), dtype=torch.uint8, device="cuda"))
     try:
@@ -76,3 +79,21 @@ def test_batch_takes_the_own_factors(gpu):
     pbb.Batch([plan], [w], [out], nc).launch()  # and with the memory free again
     torch.cuda.synchronize()
     assert torch.equal(out, adapted)
+
+
+def test_sets_are_made_when_there_is_memory(gpu):
+    import torch
+    n, nc = 2500, 3
+    ops = pbb.Operators(pbb.laplacian(), 1.0, 3, 5, 1e-7)
+    plan = pbb.Plan(ops, uniform_points(n, seed=620))
+    g = torch.Generator(device="cuda").manual_seed(621)
+    w = torch.randn(nc, n, dtype=torch.float64, device="cuda", generator=g)
+    own = torch.zeros_like(w)
+    capi.check(capi.lib().pbb_plan_matvec_noalloc(plan._h, C.c_void_p(w.data_ptr()), nc, C.c_void_p(own.data_ptr()),
+                                                  capi.PREC_FP64, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    with _filled(1 << 30):
+        for _ in range(4):  # (as often as a call likes)
+            assert torch.equal(plan.matvec(w), own)
+    got = plan.matvec(w)
+    assert not torch.equal(got, own)
+    assert float((got - own).norm() / own.norm()) <= 1e-11
