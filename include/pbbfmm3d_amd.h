@@ -404,8 +404,12 @@ PBB_API pbb_status pbb_plan_set_timing(pbb_plan *plan, int32_t enable);
  * PBB_M2L_DIR_GROUPS(g) (mixed modes, g <= 64) to split the 316 M2L
  * operators into g groups of consecutive index, one launch per group on the
  * large levels, so that a launch's operators stay in L2.  width 0 restores
- * the built-in choice.  No reference counterpart: tuning of this build's
- * M2L.                                                                    */
+ * the built-in choice.  FP64 levels whose operator set has a
+ * reflection-adapted basis (every kernel of pbb_kernel_id, as a rule) do not
+ * use tiles; the FP64 tiles serve the sets' own factors: re-compressed sets
+ * (pbb_ops_set_fp64_recompressed), sets without that symmetry and calls
+ * without the memory for the adapted sets.  No reference counterpart: tuning
+ * of this build's M2L.                                                    */
 #define PBB_M2L_CHUNK_MAJOR 1
 #define PBB_M2L_ROW_SPLIT 2
 #define PBB_M2L_WAVE_ROWS 4
@@ -430,8 +434,10 @@ PBB_API pbb_status pbb_plan_get_m2l_tile(const pbb_plan *plan, int32_t precision
  * the plan and returns it in best[3] = {width, cols_per_box, flags} (may be
  * NULL).  From the same runs it also picks the fastest tile of each tree
  * level and keeps those per-level tiles when the combination is faster
- * (pbb_plan_get_m2l_tile reads them).  Runs on `stream`, waits for it, and
- * uses a scratch output of its own.  No reference counterpart.           */
+ * (pbb_plan_get_m2l_tile reads them).  In FP64 the timed matvecs run the
+ * operator sets' own factors (see pbb_plan_set_m2l_tile).  Runs on `stream`,
+ * waits for it, and uses a scratch output of its own.  No reference
+ * counterpart.                                                            */
 PBB_API pbb_status pbb_plan_tune_m2l(pbb_plan *plan, const double *w_dev, int32_t ncols,
                                      int32_t precision, void *stream, int32_t *best);
 

@@ -1838,15 +1838,15 @@ static size_t device_room(size_t held, size_t *free_bytes = nullptr)
 // A pass that keeps its expansions for the caller (keep: the complete leaf
 // expansions in W.S; out may be nullptr) is not split; like a single column, it
 // takes the sets' own factors, whose rows are not padded, where the adapted
-// sets' workspace does not fit.
+// sets' workspace does not fit.  own: the own factors everywhere.
 static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, double *out, hipStream_t st, int prec,
-                       bool keep = false)
+                       bool keep = false, bool own = false)
 {
     const bool mixed = prec != PBB_PREC_FP64;
     const PointIo io = point_io(p, o);
     int chunk = ncols;
     bool sym = false;
-    if (!mixed && p->Lv >= 2 && !o->fp64_reduced) {
+    if (!mixed && p->Lv >= 2 && !o->fp64_reduced && !own) {
         sym = o->sym_ready.load(std::memory_order_acquire);
         if (!sym) {  // nothing is prepared inside a caller's stream capture
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1901,7 +1901,9 @@ static double device_rel_diff(const double *a, const double *b, int64_t n, doubl
     return b2 > 0 ? std::sqrt(d2 / b2) : (d2 > 0 ? INFINITY : 0.0);
 }
 
-// The M2L tile autotuner.  max_rel_diff > 0 (mixed modes): a candidate is
+// The M2L tile autotuner.  FP64 candidates run on the sets' own factors, which
+// the tiles are for (timed on adapted sets, which have none, the pick would be
+// noise).  max_rel_diff > 0 (mixed modes): a candidate is
 // kept only if its matvec differs from the FP64 matvec on the same weights
 // by at most max_rel_diff (relative 2-norm); when none does, the most
 // accurate one is kept.  achieved: that candidate's difference (0 without
@@ -1952,11 +1954,11 @@ static void tune_m2l(pbb_plan *plan, const double *w_dev, int ncols, int precisi
             matvec_own(plan, plan->ops, w_dev, ncols, ref, st, PBB_PREC_FP64);
         }
         // one untimed matvec builds the operator splits and workspaces
-        matvec_own(plan, plan->ops, w_dev, ncols, scratch, st, precision);
+        matvec_own(plan, plan->ops, w_dev, ncols, scratch, st, precision, false, true);
         for (int c = 0; c < ncand; c++) {
             plan->m2l_tile[mixed ? 1 : 0] = {cands[c][0], std::min(cands[c][1], ncols), cands[c][2]};
             if (bounded) dev::launch_fill_zero(scratch, nout, st);
-            matvec_own(plan, plan->ops, w_dev, ncols, scratch, st, precision);
+            matvec_own(plan, plan->ops, w_dev, ncols, scratch, st, precision, false, true);
             check(hipStreamSynchronize(st), "hipStreamSynchronize");
             float t = 0;
             check(hipEventElapsedTime(&t, plan->ev[3], plan->ev[4]), "hipEventElapsedTime");
@@ -2001,7 +2003,7 @@ static void tune_m2l(pbb_plan *plan, const double *w_dev, int ncols, int precisi
         if (differs) {
             std::copy(std::begin(lev), std::end(lev), plan->m2l_level[cls]);
             if (bounded) dev::launch_fill_zero(scratch, nout, st);
-            matvec_own(plan, plan->ops, w_dev, ncols, scratch, st, precision);
+            matvec_own(plan, plan->ops, w_dev, ncols, scratch, st, precision, false, true);
             check(hipStreamSynchronize(st), "hipStreamSynchronize");
             float t = 0;
             check(hipEventElapsedTime(&t, plan->ev[3], plan->ev[4]), "hipEventElapsedTime");

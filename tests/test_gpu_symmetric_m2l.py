@@ -110,3 +110,18 @@ def test_operators_without_the_symmetry_keep_their_factors(gpu):
     w = torch.randn(2, 1500, dtype=torch.float64, device="cuda", generator=g)
     own = _noalloc(torch, plan, w)
     assert torch.equal(plan.matvec(w), own)
+
+
+def test_tuner_times_the_own_factors(gpu):
+    # FP64 tiles serve the sets' own factors, so the tuner runs these: it
+    # leaves the adapted sets unmade, and the allocation-free matvec the same
+    import torch
+    kernel, order, eps = KERNELS["lap5"]
+    plan = pbb.Plan(pbb.Operators(kernel, 1.0, 3, order, eps), uniform_points(3000, seed=330))
+    g = torch.Generator(device="cuda").manual_seed(331)
+    w = torch.randn(4, 3000, dtype=torch.float64, device="cuda", generator=g)
+    own = _noalloc(torch, plan, w)
+    plan.tune_m2l(w)
+    plan.set_m2l_tile(0)
+    assert torch.equal(_noalloc(torch, plan, w), own)
+    assert not torch.equal(plan.matvec(w), own)
