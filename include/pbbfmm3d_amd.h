@@ -407,9 +407,9 @@ PBB_API pbb_status pbb_plan_set_timing(pbb_plan *plan, int32_t enable);
  * the built-in choice.  FP64 levels whose operator set has a
  * reflection-adapted basis (every kernel of pbb_kernel_id, as a rule) do not
  * use tiles; the FP64 tiles serve the sets' own factors: re-compressed sets
- * (pbb_ops_set_fp64_recompressed), sets without that symmetry and calls
- * without the memory for the adapted sets.  No reference counterpart: tuning
- * of this build's M2L.                                                    */
+ * (pbb_ops_set_fp64_recompressed), sets without that symmetry, calls of many
+ * columns on sets of ranks below 16 and calls without the memory for the
+ * adapted sets.  No reference counterpart: tuning of this build's M2L.    */
 #define PBB_M2L_CHUNK_MAJOR 1
 #define PBB_M2L_ROW_SPLIT 2
 #define PBB_M2L_WAVE_ROWS 4

@@ -780,16 +780,26 @@ struct pbb_plan {
 };
 
 // ---- the FP64 M2L in the reflection-adapted bases ---------------------------
-// The set of level l's M2L in a pass of ncols columns, or nullptr where the
-// level keeps the set's own factors: no bases of pure parity within the bounds
-// of make_sym_set, or more proxies than its offsets reach.  Where
-// they exist they were faster down to the smallest plan measured (1M points,
-// 8 columns 293 -> 78 ms; 5k points, 1 column 1.77 -> 0.42 ms per matvec).
-static const SymSet *sym_level(const pbb_plan &p, const pbb_ops *o, int l, int ncols)
+// The set of level l's M2L in a pass of ncols of the call's `all` columns, or
+// nullptr where the level keeps the set's own factors: no bases of pure parity
+// within the bounds of make_sym_set, more proxies than its offsets reach, or a
+// small rank.  Else they were faster down to the smallest plan measured (1M
+// points, 8 columns 293 -> 78 ms; 5k points, 1 column 1.77 -> 0.42 ms per
+// matvec).  Ranks below 16 are one step of one block a direction in the own
+// factors (189 steps), while the 56 orbits take a step for each of 7 or 8
+// classes of a few columns: at 31k boxes, rank 7, VT' to U' of 24 / 64 / 128
+// columns 4.7 / 10.9 / 21.0 ms against 5.0 / 12.5 / 25.1 ms, rank 15 5.5 / 12.6
+// / 24.5 against 5.6 / 14.0 / 28.4 (rank 16 24.2 against 14.0 at 64, four classes
+// at rank 4 11.6 against 8.3).  Launches that leave the GPU idle gain from the
+// sum parts, which only the adapted sets have: the M2L of 4096 boxes, 48 / 64
+// columns 1.5 / 1.6 ms against 1.2 / 1.5 ms, 100 columns 2.6 against 2.9 ms.
+static const SymSet *sym_level(const pbb_plan &p, const pbb_ops *o, int l, int ncols, int all)
 {
     if (!o->sym_ready.load(std::memory_order_acquire) || o->fp64_reduced) return nullptr;
     const SymSet &q = o->sym[o->h.ops_set(l)];
-    return q.ok && sym_level_fits(p.lv[l].nb, ncols, q.nk) ? &q : nullptr;
+    if (!q.ok || !sym_level_fits(p.lv[l].nb, ncols, q.nk)) return nullptr;
+    const bool small = o->h.rf < 16 && o->h.rs < 16 && q.nj >= 7;
+    return small && (all > 64 || p.lv[l].nb * all > 600000) ? nullptr : &q;
 }
 
 // Tile and sum parts of a level's M2L for ncols of the call's `all` columns.
@@ -848,7 +858,7 @@ static FarDims far_dims(const pbb_plan &p, const pbb_ops *o, int ncols, int all,
     const int rmax = std::max(o->h.rf, o->h.rs);
     d.ldp = d.ldf = rmax;
     for (int l = 2; sym && l <= p.Lv; l++) {
-        const SymSet *q = sym_level(p, o, l, ncols);
+        const SymSet *q = sym_level(p, o, l, ncols, all);
         if (!q) continue;
         d.sym = true;
         d.ldp = std::max(d.ldp, q->nk);
@@ -1864,7 +1874,7 @@ static void matvec_own(pbb_plan *p, pbb_ops *o, const double *w, int ncols, doub
         if (need > p->ws_bytes && need > device_room(p->ws_bytes)) sym = false;
     } else {
         for (int l = 2; sym && l <= p->Lv; l++)
-            if (const SymSet *q = sym_level(*p, o, l, 1)) chunk = sym_columns(p->lv[l].nb, chunk, q->nk);
+            if (const SymSet *q = sym_level(*p, o, l, 1, ncols)) chunk = sym_columns(p->lv[l].nb, chunk, q->nk);
         size_t need = bytes();
         if (need > p->ws_bytes || (p->ws_limit && need > p->ws_limit)) {
             size_t free_b = 0, room = device_room(p->ws_bytes, &free_b);
@@ -2123,7 +2133,7 @@ static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double
     const bool split_acc = split_acc_on(p, prec);
     const pbb_plan::M2LTile &tmx = p->m2l_tile[1];
     const int ldP = mixed ? W.kpad : h.rs;
-    auto sym_of = [&](int l) -> const SymSet * { return !mixed && W.sym ? sym_level(*p, o, l, ncols) : nullptr; };
+    auto sym_of = [&](int l) -> const SymSet * { return !mixed && W.sym ? sym_level(*p, o, l, ncols, W.all) : nullptr; };
     if (mixed && h.rs > W.kpad) fail(PBB_ERR_INTERNAL, "proxy padding too small");
     mark(0);
     // orders 4..8 run the direct passes: P2M at every level instead of

@@ -125,3 +125,22 @@ def test_tuner_times_the_own_factors(gpu):
     plan.set_m2l_tile(0)
     assert torch.equal(_noalloc(torch, plan, w), own)
     assert not torch.equal(plan.matvec(w), own)
+
+
+def test_small_ranks_of_many_columns_run_the_own_factors(gpu):
+    # ranks below 16 in 7 parity classes: the own factors above 64 columns, the
+    # whole call's (column chunks give the same bits)
+    import torch
+    ops = pbb.Operators(pbb.laplacian(), 1.0, 3, 4, 1e-2)
+    assert ops.rank_f == ops.rank_s == 7
+    plan = pbb.Plan(ops, uniform_points(1500, seed=340))
+    g = torch.Generator(device="cuda").manual_seed(341)
+    w = torch.randn(65, 1500, dtype=torch.float64, device="cuda", generator=g)
+    own = _noalloc(torch, plan, w)
+    adapted = plan.matvec(w[:64].contiguous())
+    assert not torch.equal(adapted, own[:64])
+    assert float((adapted - own[:64]).norm() / own.norm()) <= 1e-11
+    assert torch.equal(plan.matvec(w), own)
+    assert torch.equal(_noalloc(torch, plan, w), own)
+    plan.set_workspace_limit(1)
+    assert torch.equal(plan.matvec(w), own)
