@@ -155,7 +155,10 @@ struct M2LArgs {
 constexpr int SYM_TB = 64;    // boxes of a tile
 constexpr int SYM_CONFS = 9;  // row configurations
 constexpr int SYM_NG2 = 32;   // row groups up to which a wave holds 32 columns (else 16)
-constexpr int SYM_NG3 = 20;   // row groups up to which three workgroups fit a CU's registers
+// Workgroups of ng row groups that a CU's registers hold (a workgroup is a
+// wave on each SIMD): three up to 168 registers a lane.  32 columns a wave
+// need 168 at 20 groups and 212 at 28, 16 columns 154 at 36 and 170 at 40.
+constexpr int sym_workgroups(int ng) { return ng <= 20 || (ng > SYM_NG2 && ng <= 36) ? 3 : 2; }
 constexpr int SYM_NB = 8;     // orbits to a barrier, at most
 
 // Row layout of a set: the configuration's groups of 4 rows (ng in each of

@@ -200,7 +200,7 @@ __device__ __forceinline__ void sym_step(const uint32_t *const (&tab)[C::CB], co
 // offsets (one 64-bit add each; a box that is not there is the level's box of
 // zeros).
 template <class C>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(C::NG <= SYM_NG3 ? 3 : 2))) void m2l_sym_f64(SymArgs a)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sym_workgroups(C::NG)))) void m2l_sym_f64(SymArgs a)
 {
     constexpr int NT = 256, NG = C::NG, ECH = 2 * NG * 16;  // doubles of an operator chunk
     const int NB = a.NB;
@@ -556,7 +556,7 @@ void launch_m2l_sym(const SymArgs &args, const SymShape &s, int ncolchunks, hipS
     // workgroup of small configurations) 147 -> 129 ms.  Four at the price of a
     // workgroup (500k points, 4 columns) was slower by a third.
     const size_t table = sizeof(uint32_t) * 189 * a.TB, chunk = 2 * sizeof(double) * 2 * s.ng * 16;
-    const size_t room = SYM_LDS / (s.ng <= SYM_NG3 || s.conf == 6 ? 3 : 2) - SYM_LDS_FIXED;
+    const size_t room = SYM_LDS / sym_workgroups(s.ng) - SYM_LDS_FIXED;
     a.NB = (int)std::max<size_t>(2, std::min<size_t>(SYM_NB, room > table ? (room - table) / chunk : 0));
     const size_t lds = chunk * a.NB + table;
     switch (s.conf) {
