@@ -304,7 +304,11 @@ PBB_API pbb_status pbb_plan_update_points(pbb_plan *plan, const double *xyz, int
  * all work is enqueued.  Every call on one plan (matvec, transpose,
  * gradients, tuning) uses the plan's one device workspace: issue them on
  * one stream, or order the streams yourself; calls on different plans are
- * independent and may run on any streams and host threads.              */
+ * independent and may run on any streams and host threads.  The first FP64
+ * matvec of an operator object, and the first transposed one, also makes the
+ * reflection-adapted form of its sets and waits for the stream (3 ms at order
+ * 4, 7 at order 5, 18 to 27 a set at order 6, 57 at order 8); not within a
+ * stream capture, which runs the sets' own factors if it comes first.    */
 PBB_API pbb_status pbb_plan_matvec(pbb_plan *plan, const double *w_dev,
                                    int32_t ncols, double *out_dev,
                                    int32_t precision, void *stream);
@@ -359,7 +363,9 @@ PBB_API pbb_status pbb_plan_grad_positions(pbb_plan *plan, const double *sigma_d
  * again).  pbb_plan_matvec_keep is pbb_plan_matvec that also writes the leaf
  * expansions, pbb_plan_kept_size doubles; that size is 0 where a forward had
  * better not keep them (fewer than two levels, the mixed modes, plans without
- * position gradients or with a workspace cap, not enough free device memory).
+ * position gradients or with a workspace cap, not enough free device memory:
+ * it is looked up at every call, so that equal calls can take either forward,
+ * whose sums differ in their order).
  * No reference counterpart; used by the autograd function.                 */
 PBB_API pbb_status pbb_plan_kept_size(pbb_plan *plan, int32_t ncols, int32_t precision,
                                       int64_t *count);
@@ -375,7 +381,10 @@ PBB_API pbb_status pbb_plan_gradients(pbb_plan *plan, const double *sigma_dev,
 /* Caps the plan's matvec workspace at `bytes` (0: what the device holds).
  * A matvec whose workspace for all its columns does not fit runs as
  * chunks of columns, each a complete FMM pass with the same sums (phase
- * times then cover the last chunk).  No reference counterpart.           */
+ * times then cover the last chunk).  Gradients and batches are not split:
+ * where the FP64 workspace of the reflection-adapted operator sets does not
+ * fit the device they run the sets' own factors, which need less of it and
+ * more time.  No reference counterpart.                                   */
 PBB_API pbb_status pbb_plan_set_workspace_limit(pbb_plan *plan, int64_t bytes);
 
 /* Phase times of the last pbb_plan_matvec on this plan, in ms

@@ -7,8 +7,11 @@
               interpolants and of the P2P kernel; box membership and the
               bbox centre are held fixed, as they are piecewise constant).
 Both together take one transposed pass; a forward in FP64 whose points need
-a gradient saves its leaf expansions for it (otherwise the backward runs the
-forward's far field again).
+a gradient saves its leaf expansions for it where the device has the memory
+beside them (otherwise the backward runs the forward's far field again).  The
+two forwards sum in different orders: on a device that is nearly full, equal
+calls can differ in their last bits, and a checkpointed step (which compares
+what its two forwards saved) can find different ones.
 The tree is built from xyz at every forward call, unless a plan is given:
 then its points are moved to xyz (pbb_plan_update_points, which fails if a
 point leaves its leaf box) and its tree is reused.  Weights of any floating

@@ -528,7 +528,9 @@ struct pbb_ops {
         dev::launch_transpose_blocks(Y, rf, ts, 316, X, st);
         gemm(dBt, rs, ts, X, (int64_t)316 * rf, Y);           // (X^T K_d Y)^T
         dev::launch_transpose_blocks(Y, rs, rf, 316, X, st);
-        // the operators themselves hold the symmetry to a few 1e-14 of their norm
+        // good sets come out at 1e-15 to 7e-15 of the norm of all blocks.  The
+        // bound is the same for every eps of the compression: it keeps out sets
+        // without the symmetry, not a larger share of a smaller eps
         const double err = device_rel_diff(X, dE, (int64_t)316 * rf * rs, part, st);
         if (!(err <= 1e-13)) return false;
 
@@ -2056,8 +2058,6 @@ PBB_API pbb_status pbb_plan_tune_m2l_within(pbb_plan *plan, const double *w_dev,
         [&] { tune_m2l(plan, w_dev, ncols, precision, (hipStream_t)stream, max_rel_diff, best, achieved); });
 }
 
-// One FMM application.  out == nullptr stops after the downward pass, leaving
-// the leaf local expansions in W.S and the sorted weights in W.ws.
 static void fill_levels(const pbb_plan *p, dev::LevelTab &t)
 {
     t.nlev = p->Lv - 1;
@@ -2117,6 +2117,9 @@ static void split_ops(const pbb_plan *p, pbb_ops *o, int prec, bool build, hipSt
     if (want3) SA = &o->vt3;
 }
 
+// One FMM application.  out == nullptr stops after the downward pass, leaving
+// the leaf local expansions in W.S and the sorted weights in W.wsT (orders 4..8,
+// point-major; W.ws then holds the caller's order) or in W.ws.
 static void matvec_run(pbb_plan *p, pbb_ops *o, const Workspace &W, const double *w, int ncols, double *out,
                        hipStream_t st, int prec, bool build, bool keep)
 {

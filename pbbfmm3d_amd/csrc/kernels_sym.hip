@@ -12,11 +12,15 @@
 // 189 directions shrink to 39.5 in an open cloud.  Of these 81% fill at rank
 // 101 (classes padded to 4 rows and 4 k), 89% at rank 181.
 //
-// Bound: the FP64 matrix cores (the Walsh-Hadamard sums share their issue
-// slots), then the latency of the gathered sources.  M2L of one matvec, with
-// the set's own factors and here: 1M uniform points, 1/r, order 5, 8 columns
-// 281 -> 64 ms (at the deepest level 56 ms; its products alone take 26 ms at
-// 77 TFLOP/s); 1M clustered points, Gaussian, 32 columns 1410 -> 95 ms.
+// Bound: the latency of the gathered sources and the barriers, beside the FP64
+// matrix cores (the Walsh-Hadamard sums share their issue slots).  M2L of one
+// matvec, with the set's own factors and here: 1M uniform points, 1/r, order 5,
+// 8 columns 281 -> 64 ms, from the orbits (at the deepest level 56 ms, of which
+// the matrix cores are busy 48%; its products at 78.6 TFLOP/s 21 ms); 1M
+// clustered points, Gaussian, order 6, 32 columns 1410 -> 95 ms, from the orbits
+// and, more, from the columns at the rounding level that the bases leave out
+// (rank 181: 181, 181, 135, 81 and 53 at levels 2 to 6, at level 6 an eleventh
+// of a block; there 59 ms, matrix cores 39% busy, 46% L2 hits, products 13 ms).
 // Loading a step's sources under the products of the step before (16 columns a
 // wave, two register sets) was slower: 75 -> 89 ms for the first of these calls.
 #include <hip/hip_runtime.h>
@@ -488,7 +492,11 @@ __global__ __launch_bounds__(256) void sym_expand(const double *__restrict__ K, 
 
 namespace {
 // row-group capacities by the number of odd axes, in the order of their
-// cost; the operators are padded to a configuration's groups
+// cost; the operators are padded to a configuration's groups.  The list is
+// made for order 4, order 5 at eps 1e-7 and order 6 at eps 1e-7 and 1e-8; other
+// class counts take the next that holds them, some with much padding (order 5
+// at eps 1e-9, 26 or 27 columns in the even class: 48 groups where 33 would do;
+// 1/r, order 5, eps 1e-5: 28 where 17 would).
 struct SymConf {
     int cap[4];
 };
